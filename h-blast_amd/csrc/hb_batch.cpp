@@ -38,7 +38,7 @@ struct hb_batch {
     int32_t group_res = 0;
     float build_ms = 0;
     // launch geometry: 0 = the configuration's own choice
-    int32_t g_waves = 0, g_ring = 0, g_items = 64;
+    int32_t g_waves = 0, g_ring = 0, g_items = 0;
     int32_t tune_candidates = 0;
     // groups
     hb_group_set gs;
@@ -47,7 +47,7 @@ struct hb_batch {
     // run state
     hb_hsp *d_out = nullptr;
     uint32_t cap = 0;
-    uint32_t *d_misc = nullptr;                // [0] HSP count, [1 + c] work counter of class c
+    uint32_t *d_misc = nullptr;                // HSP count in its own line, then each group's tile queues
     unsigned long long *d_totals = nullptr;    // 3 per group
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -66,11 +66,16 @@ static void free_graph(hb_batch *b)
     b->graph = nullptr;
 }
 
+static size_t misc_words(const hb_batch *b)
+{
+    return HB_QUEUE_STRIDE + b->gs.desc.size() * (size_t)HB_QUEUE_WORDS;
+}
+
 static void free_groups(hb_batch *b)
 {
     free_graph(b);
     hb_group_set_free(&b->gs);
-    hb_pool_put(b->ctx, b->d_misc, (1 + b->classes.size()) * sizeof(uint32_t));
+    hb_pool_put(b->ctx, b->d_misc, misc_words(b) * sizeof(uint32_t));
     hb_pool_put(b->ctx, b->d_totals, 3 * b->gs.desc.size() * sizeof(unsigned long long));
     for (Class &c : b->classes)
         if (c.d_gstate) hb_pool_put(b->ctx, c.d_gstate, c.gstate_bytes);
@@ -155,13 +160,15 @@ static void make_groups(hb_batch *b, int32_t target, std::vector<hb_concat> *gro
     }
 }
 
+static int32_t items_per_workgroup(const hb_batch *b) { return b->g_items > 0 ? b->g_items : 64; }
+
 // Sizes work items for a pass over n_tiles tiles: about 64 items per
 // workgroup for balance, few enough for the queue atomic.
 static void size_items(hb_batch *b, uint32_t n_tiles)
 {
     for (Class &c : b->classes) {
         const uint32_t n_groups = (uint32_t)(c.g_end - c.g_begin);
-        const uint64_t want = (uint64_t)c.cfg.blocks * (uint64_t)std::max(b->g_items, 1);
+        const uint64_t want = (uint64_t)c.cfg.blocks * (uint64_t)items_per_workgroup(b);
         const uint64_t per_group = std::max<uint64_t>(1, want / std::max<uint32_t>(n_groups, 1));
         c.tiles_per_item = (uint32_t)std::max<uint64_t>(1, (n_tiles + per_group - 1) / per_group);
     }
@@ -242,7 +249,7 @@ static int build(hb_batch *b, int32_t target)
         }
     }
     size_items(b, b->db->n_tiles);
-    b->d_misc = static_cast<uint32_t *>(hb_pool_get(b->ctx, (1 + b->classes.size()) * sizeof(uint32_t)));
+    b->d_misc = static_cast<uint32_t *>(hb_pool_get(b->ctx, misc_words(b) * sizeof(uint32_t)));
     b->d_totals = static_cast<unsigned long long *>(
         hb_pool_get(b->ctx, 3 * (size_t)ng * sizeof(unsigned long long)));
     if (!b->d_misc || !b->d_totals) return HB_ERR_NOMEM;
@@ -258,7 +265,10 @@ static int enqueue(hb_batch *b, uint32_t t_begin, uint32_t t_end)
 {
     hb_db *db = b->db;
     const uint32_t nc = (uint32_t)b->classes.size();
-    HB_CHECK(hb_launch_fill_u32(b->d_misc, 0u, 1 + nc, b->st));
+    HB_CHECK(hb_launch_fill_u32(b->d_misc, 0u, (uint32_t)misc_words(b), b->st));
+    // a full pass takes the plain scan's shrinking tiles one by one unless
+    // the items per workgroup were asked for or tuned
+    const bool whole = t_begin == 0 && t_end == db->n_tiles && b->g_items == 0;
     HB_CHECK(hb_launch_fill_u32(reinterpret_cast<uint32_t *>(b->d_totals), 0u,
                                 (uint32_t)(6 * b->gs.desc.size()), b->st));
     for (uint32_t ci = 0; ci < nc; ++ci) {
@@ -272,6 +282,11 @@ static int enqueue(hb_batch *b, uint32_t t_begin, uint32_t t_end)
         a.tile_begin = t_begin;
         a.tile_end = t_end;
         a.tiles_per_item = C.tiles_per_item;
+        if (whole) {
+            a.tiles = db->d_tiles + db->n_tiles + 1;
+            a.tile_end = db->n_qtiles;
+            a.tiles_per_item = 1;
+        }
         a.groups = b->gs.d_desc + C.g_begin;
         a.n_groups = (uint32_t)(C.g_end - C.g_begin);
         a.qlen_pad_max = C.qlen_pad_max;
@@ -284,7 +299,9 @@ static int enqueue(hb_batch *b, uint32_t t_begin, uint32_t t_end)
         a.state_limit = hb_state_limit(C.place, db->max_len);
         a.mat32 = b->gs.d_mat;
         a.window = b->p.window;
-        a.work_counter = b->d_misc + 1 + ci;
+        a.work_counter = b->d_misc + HB_QUEUE_STRIDE + (size_t)C.g_begin * HB_QUEUE_WORDS;
+        a.n_streams = std::min({a.n_groups, 8u, (uint32_t)C.cfg.blocks});
+        a.n_queues = std::min((uint32_t)HB_QUEUES, (uint32_t)C.cfg.blocks / a.n_streams);
         a.out = b->d_out;
         a.out_cap = b->cap;
         a.out_count = b->d_misc;
@@ -522,7 +539,7 @@ int hb_batch_create_on(hb_ctx *ctx, hb_db *db, const hb_params *params, const hb
     }
     b->g_waves = o.waves_per_workgroup;
     b->g_ring = o.ring_bytes;
-    b->g_items = o.items_per_workgroup > 0 ? o.items_per_workgroup : 64;
+    b->g_items = o.items_per_workgroup;
     int rc = hb_resolve_params(params, &b->p);
     if (rc) {
         delete b;
@@ -713,7 +730,7 @@ int hb_batch_info_get(hb_batch *b, hb_batch_info *info)
             info->waves_per_workgroup = c.cfg.waves;
             info->ring_bytes = c.cfg.ring;
         }
-    info->items_per_workgroup = b->g_items;
+    info->items_per_workgroup = items_per_workgroup(b);
     info->tune_candidates = b->tune_candidates;
     return HB_OK;
 }

@@ -17,6 +17,9 @@
 #ifndef HB_RING_MAX
 #define HB_RING_MAX 4096    // largest staging ring per wave (subjects up to the ring are staged)
 #endif
+#define HB_QUEUES 16        // tile queues of a query group
+#define HB_QUEUE_STRIDE 32  // words between two queues' counters (a 128-byte line each)
+#define HB_QUEUE_WORDS (HB_QUEUES * HB_QUEUE_STRIDE)
 #define HB_BLOCK 256        // at most 4 wavefronts per workgroup
 // Diagonal state kept in LDS: one 32-bit word per diagonal, 23-bit positions
 // between resets (hb_scan_args::state_limit), so the longest subject and
@@ -57,7 +60,9 @@ struct hb_scan_args {
     const uint32_t *tiles;       // tile boundaries into subj
     uint32_t tile_begin;         // tiles [tile_begin, tile_end) are scanned
     uint32_t tile_end;
-    uint32_t tiles_per_item;     // batched: tiles per (group, tile chunk) work item
+    uint32_t tiles_per_item;     // batched: tiles per pop of a group's queue
+    uint32_t n_streams;          // batched: 1 .. min(groups, workgroups)
+    uint32_t n_queues;           // batched: 1 .. min(HB_QUEUES, workgroups / n_streams)
     // query groups
     const hb_group_desc *groups;
     uint32_t n_groups;
@@ -71,7 +76,7 @@ struct hb_scan_args {
     const int8_t *mat32;         // 32x32 scores, -128 padded
     int32_t window;
     // work queue and output
-    uint32_t *work_counter;
+    uint32_t *work_counter;      // HB_QUEUE_WORDS words per group, zero at launch
     hb_hsp *out;
     uint32_t out_cap;
     uint32_t *out_count;

@@ -1089,10 +1089,24 @@ __device__ __forceinline__ void bind_group(WaveScan<GS> &w, const hb_group_desc 
     w.dmul = (uint32_t)(0xffffffffu / (uint32_t)G.diag_len) + 1u;
 }
 
+// Scans the subjects of one tile (at most 64): lane j holds the record of
+// subject j, so that the records cost one load per tile.
+template <bool GS>
+__device__ __forceinline__ void scan_tile(WaveScan<GS> &w, const hb_scan_args &a, uint32_t t)
+{
+    const uint32_t s0 = a.tiles[t], ns = a.tiles[t + 1] - s0;
+    uint4 rec = make_uint4(0, 0, 0, 0);
+    if ((uint32_t)w.lane < ns) rec = a.subj[s0 + (uint32_t)w.lane];
+    for (uint32_t j = 0; j < ns; ++j)
+        w.scan_subject(make_uint4((uint32_t)__builtin_amdgcn_readlane((int)rec.x, (int)j),
+                                  (uint32_t)__builtin_amdgcn_readlane((int)rec.y, (int)j),
+                                  (uint32_t)__builtin_amdgcn_readlane((int)rec.z, (int)j),
+                                  (uint32_t)__builtin_amdgcn_readlane((int)rec.w, (int)j)));
+}
+
 // MULTI = false: one group; each wavefront pops subject tiles on its own.
-// MULTI = true: many groups; the workgroup pops (group, tile) items and its
-// wavefronts share the tile's subjects, so all of them use one group's LDS
-// tables at a time.
+// MULTI = true: many groups; a workgroup binds one group at a time, so that
+// its wavefronts use one set of LDS tables.
 // GSTATE: the diagonal words live in global memory (a.gstate, diag_len_max
 // per wavefront of the grid) instead of LDS, for queries (groups) whose
 // state does not fit LDS or would leave it too few wavefronts, and for
@@ -1119,7 +1133,7 @@ template <bool MULTI, bool GSTATE>
 __device__ __forceinline__ void scan_body(const hb_scan_args &a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ uint32_t s_item, s_next;
+    __shared__ uint32_t s_group;
     const int lane = threadIdx.x & (HB_WAVE - 1);
     const int wid = threadIdx.x / HB_WAVE;
     int8_t *sm_mat = reinterpret_cast<int8_t *>(lds);
@@ -1172,61 +1186,80 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
         bind_group(w, G);
         w.clear_words();
         __syncthreads();
-        for (;;) {
-            uint32_t t = 0;
-            if (lane == 0) t = atomicAdd(a.work_counter, 1u);
-            t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
-            if (t >= n_tiles) break;
-            t += a.tile_begin;
-            const uint32_t i_end = a.tiles[t + 1];
-            for (uint32_t it = a.tiles[t]; it < i_end; ++it) w.scan_subject(a.subj[it]);
+        // The tiles are dealt to up to HB_QUEUES queues (tile i to queue i mod
+        // n_q) and the workgroups likewise; a wavefront starts on a tile of
+        // its own and then pops its queue.
+        const uint32_t n_q = min((uint32_t)gridDim.x, (uint32_t)HB_QUEUES);
+        const uint32_t k = blockIdx.x % n_q;
+        const uint32_t wpb = blockDim.x / HB_WAVE;
+        const uint32_t len = n_tiles > k ? (n_tiles - k + n_q - 1) / n_q : 0u;
+        const uint32_t first = (gridDim.x - k + n_q - 1) / n_q * wpb;   // the queue's wavefronts
+        uint32_t i = (blockIdx.x / n_q) * wpb + (uint32_t)wid;
+        while (i < len) {
+            uint32_t nx = 0;   // popped ahead: the atomic overlaps the tile's work
+            if (lane == 0) nx = atomicAdd(a.work_counter + HB_QUEUE_STRIDE * k, 1u);
+            scan_tile(w, a, a.tile_begin + k + i * n_q);
+            i = first + (uint32_t)__builtin_amdgcn_readfirstlane((int)nx);
         }
         w.template finish<true>(w.ring);
         w.flush_totals(0);
     } else {
-        uint32_t cur = 0xffffffffu;
-        const uint32_t tpi = a.tiles_per_item;
-        const uint32_t n_chunks = (n_tiles + tpi - 1) / tpi;
-        const uint32_t n_items = n_chunks * a.n_groups;
+        // The groups are dealt to n_streams streams (8: workgroup b runs on
+        // XCD b mod 8, so an XCD's L2 holds one or two groups' tables at a
+        // time).  A workgroup takes the groups of its stream in order, then
+        // any group with items left, and binds one group at a time; its
+        // wavefronts pop the group's items (tiles_per_item tiles) on their
+        // own and meet only where the group changes.
+        const uint32_t n_s = a.n_streams, n_q = a.n_queues, tpi = a.tiles_per_item;
+        const uint32_t stream = blockIdx.x % n_s, k = (blockIdx.x / n_s) % n_q;
+        const uint32_t n_items = (n_tiles + tpi - 1) / tpi;
+        const uint32_t len = n_items > k ? (n_items - k + n_q - 1) / n_q : 0u;
+        const uint32_t n_own = (a.n_groups - stream + n_s - 1) / n_s;
+        uint32_t pos = 0;   // candidates already passed over (wavefront 0)
         for (;;) {
-            if (threadIdx.x == 0) s_item = atomicAdd(a.work_counter, 1u);
-            __syncthreads();
-            const uint32_t item = s_item;
-            if (item >= n_items) break;
-            const uint32_t g = item / n_chunks;
-            const uint32_t t0 = a.tile_begin + (item % n_chunks) * tpi;
-            const uint32_t t1 = min(t0 + tpi, a.tile_end);
-            if (g != cur) {
-                if (cur != 0xffffffffu) {
-                    w.template finish<true>(w.ring);   // still with the old group's tables
-                    w.flush_totals(cur);
+            if (wid == 0) {
+                uint32_t g = 0xffffffffu;
+                for (; pos < n_own + a.n_groups; pos += HB_WAVE) {
+                    const uint32_t p = pos + (uint32_t)lane;
+                    const uint32_t gp = p < n_own ? stream + p * n_s : p - n_own;
+                    bool left = false;
+                    if (p < n_own + a.n_groups)
+                        left = __hip_atomic_load(
+                                   &a.work_counter[(size_t)gp * HB_QUEUE_WORDS + HB_QUEUE_STRIDE * k],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < len;
+                    const uint64_t m = ballot(left);
+                    if (m) {
+                        const int f = (int)__builtin_ctzll(m);
+                        g = (uint32_t)__builtin_amdgcn_readlane((int)gp, f);
+                        pos += (uint32_t)f + 1;
+                        break;
+                    }
                 }
-                __syncthreads();
-                const hb_group_desc G = a.groups[g];
-                load_group(a, G, sm_ctx, sm_q);
-                bind_group(w, G);
-                w.clear_words();
-                cur = g;
-                __syncthreads();
-            }
-            // the chunk's subjects are taken one at a time by whichever
-            // wavefront is free (LDS counter), so the workgroup's wavefronts
-            // reach the next barrier at most one subject apart
-            if (threadIdx.x == 0) s_next = a.tiles[t0];
-            __syncthreads();
-            const uint32_t i_end = a.tiles[t1];
-            for (;;) {
-                uint32_t it = 0;
-                if (lane == 0) it = atomicAdd(&s_next, 1u);
-                it = (uint32_t)__builtin_amdgcn_readfirstlane((int)it);
-                if (it >= i_end) break;
-                w.scan_subject(a.subj[it]);
+                if (lane == 0) s_group = g;
             }
             __syncthreads();
-        }
-        if (cur != 0xffffffffu) {
+            const uint32_t g = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_group);
+            if (g == 0xffffffffu) break;
+            const hb_group_desc G = a.groups[g];
+            load_group(a, G, sm_ctx, sm_q);
+            bind_group(w, G);
+            w.clear_words();
+            __syncthreads();
+            uint32_t *ctr = a.work_counter + (size_t)g * HB_QUEUE_WORDS + HB_QUEUE_STRIDE * k;
+            uint32_t i = 0;
+            if (lane == 0) i = atomicAdd(ctr, 1u);
+            i = (uint32_t)__builtin_amdgcn_readfirstlane((int)i);
+            while (i < len) {
+                uint32_t nx = 0;
+                if (lane == 0) nx = atomicAdd(ctr, 1u);
+                const uint32_t t0 = a.tile_begin + (k + i * n_q) * tpi;
+                const uint32_t t1 = min(t0 + tpi, a.tile_end);
+                for (uint32_t t = t0; t < t1; ++t) scan_tile(w, a, t);
+                i = (uint32_t)__builtin_amdgcn_readfirstlane((int)nx);
+            }
             w.template finish<true>(w.ring);
-            w.flush_totals(cur);
+            w.flush_totals(g);
+            __syncthreads();
         }
     }
 }

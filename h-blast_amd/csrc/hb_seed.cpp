@@ -344,7 +344,7 @@ int hb_scan_config(hb_ctx *c, bool multi, int32_t qlen_pad_max, int32_t ctx_pad_
         const size_t per_block = HB_GSTATE_WORD * (size_t)diag_len_max * (size_t)cfg->waves;
         blocks = std::min(blocks, (int)std::max<size_t>(1, HB_GSTATE_MAX_BYTES / per_block));
     }
-    const uint32_t per_block = multi ? 1u : (uint32_t)cfg->waves;
+    const uint32_t per_block = (uint32_t)cfg->waves;
     const int need = (int)((work_items + per_block - 1) / per_block);
     if (need < blocks) blocks = std::max(need, 1);
     cfg->blocks = blocks;
@@ -403,7 +403,7 @@ struct hb_scan {
     hb_query *q = nullptr;
     hb_hsp *d_out = nullptr;
     uint32_t cap = 0;
-    uint32_t *d_misc = nullptr;   // [0] HSP count, [1] tile counter
+    uint32_t *d_misc = nullptr;   // HSP count in its own line, then the tile queues
     uint32_t *d_stats = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool waited = false;
@@ -417,11 +417,12 @@ struct hb_scan {
 
 // ------------------------------------------------------------------ no-alloc scan
 // Scratch of hb_scan_noalloc, one copy per GPU, held until the process ends:
-// the scan's HSP cursor and tile counter (the first 256 bytes), then the
+// the scan's HSP cursor and tile queues (HB_NOALLOC_HEAD bytes), then the
 // diagonal words of a query whose state lives in global memory.  Host code
 // uses the device address hipGetSymbolAddress returns (hb_ctx::scratch_dev),
 // never the array's name.
-#define HB_NOALLOC_HEAD 256
+#define HB_SCAN_MISC_WORDS (HB_QUEUE_STRIDE + HB_QUEUE_WORDS)
+#define HB_NOALLOC_HEAD (HB_SCAN_MISC_WORDS * 4)
 static __device__ __align__(256) unsigned char scratch[HB_NOALLOC_HEAD + HB_NOALLOC_STATE_BYTES];
 static std::mutex g_scratch_mu;
 static unsigned char *g_scratch_dev[256];   // per device
@@ -573,15 +574,29 @@ int hb_db_free(hb_db *db)
     return HB_OK;
 }
 
+// Tiles: runs of subjects in processing order that are handed out together,
+// at most 64 subjects and about kTileMax residues.
+// A batched launch's workgroups take tiles of one size, at least two for
+// every wavefront of a full grid where the database has the subjects for it
+// (four subjects or more: a workgroup's wavefronts share them).
+// A plain scan's wavefronts pop tiles that shrink with what is left to do, a
+// quarter of a wavefront's share of it, down to a sixteenth of its share of
+// the whole database: with tiles of 16K residues throughout, 1,000 subjects
+// kept 22 wavefronts of 4,096 busy (scan of a 60-residue query 334 us, 40 us
+// now), 20,000 subjects 500 (350 residues: 526 us, 230 us now) and 200,000
+// subjects ran 1.2 rounds of tiles (960 us, 700 us now).  Tiles of 64
+// residues gained nothing over 256 on 200,000 subjects and more, and a
+// single queue took 10 ns for each pop of every wavefront of the chip, which
+// at one subject a tile made 200,000 subjects slower than 16K tiles did.
+static constexpr uint64_t kTileMax = 16384, kQueueTileMin = 256;
+
 // Processing order and tiles of a database whose host offsets are set, and
 // the device copies of offsets, per-subject records in processing order and
 // tiles.
 static int db_meta(hb_db *db)
 {
     const uint32_t n = db->n;
-    // Length-descending processing order, then tiles of <= 64 subjects and
-    // ~16K residues: one queue pop per tile keeps atomics off the hot path
-    // and the longest subjects start first.
+    // Length-descending processing order: the longest subjects start first.
     // (stable LSD radix sort on the length, 11 bits a pass: a comparison
     // sort reading scattered offsets took ~0.2 s for 2M subjects)
     std::vector<uint32_t> order(n), tmp(n), key(n), key2(n);
@@ -611,24 +626,39 @@ static int db_meta(hb_db *db)
     // the residues, laid out in the same order, so consecutive subjects share
     // no cache line with subjects read at other times
     std::vector<uint4> subj(n);
-    std::vector<uint32_t> tiles;
-    tiles.push_back(0);
-    uint64_t acc = 0, dst = 0;
-    uint32_t cnt = 0;
+    std::vector<uint32_t> tiles(1, 0), qtiles(1, 0);
+    uint64_t acc = 0, qacc = 0, dst = 0, left = db->total;
+    uint32_t cnt = 0, qcnt = 0;
+    const uint64_t waves = db->ctx->n_cu * 16ull;
+    const uint64_t want = std::min(kTileMax, db->total / (4 * waves));
+    const uint64_t qmin = std::min(kQueueTileMin, db->total / (16 * waves));
+    uint64_t qwant = want;
     for (uint32_t i = 0; i < n; ++i) {
         const uint64_t len = db->h_offs[order[i] + 1] - db->h_offs[order[i]];
         subj[i] = make_uint4(order[i], (uint32_t)len, (uint32_t)dst, (uint32_t)(dst >> 32));
         dst += (len + 15) & ~15ull;   // the scan stages subjects with 16-byte loads
         acc += len;
+        qacc += len;
+        left -= len;
         ++cnt;
-        if (cnt >= 64 || acc >= 16384) {
+        ++qcnt;
+        if (cnt >= 64 || acc >= want) {
             tiles.push_back(i + 1);
             acc = 0;
             cnt = 0;
         }
+        if (qcnt >= 64 || qacc >= qwant) {
+            qtiles.push_back(i + 1);
+            qacc = 0;
+            qcnt = 0;
+            qwant = std::min(kTileMax, std::max(qmin, left / (4 * waves)));
+        }
     }
     if (tiles.back() != n) tiles.push_back(n);
+    if (qtiles.back() != n) qtiles.push_back(n);
     db->n_tiles = (uint32_t)tiles.size() - 1;
+    db->n_qtiles = (uint32_t)qtiles.size() - 1;
+    tiles.insert(tiles.end(), qtiles.begin(), qtiles.end());
     db->scan_bytes = dst;
     if (hipMalloc(&db->d_offs, ((size_t)n + 1) * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc(&db->d_subj, (size_t)std::max<uint32_t>(n, 1) * sizeof(uint4)) != hipSuccess ||
@@ -1015,9 +1045,9 @@ static int plain_scan_args(const hb_db *db, const hb_query *q, int place,
     a->res = db->d_scan_res;   // subjects in processing order (a->subj's offsets)
     a->offs = db->d_offs;
     a->subj = db->d_subj;
-    a->tiles = db->d_tiles;
+    a->tiles = db->d_tiles + db->n_tiles + 1;   // the plain scan's tiles
     a->tile_begin = 0;
-    a->tile_end = db->n_tiles;
+    a->tile_end = db->n_qtiles;
     a->groups = q->gs.d_desc;
     a->n_groups = 1;
     a->qlen_pad_max = q->gs.qlen_pad_max;
@@ -1047,7 +1077,7 @@ static int launch_scan(hb_scan *s)
     if (place < 0) return HB_ERR_UNSUPPORTED;   // LDS state asked for, subjects too long
     s->place = place;
     int rc = hb_scan_config(c, false, q->gs.qlen_pad_max, q->gs.ctx_pad_max, q->gs.diag_len_max,
-                            db->n_tiles, &cfg, place);
+                            db->n_qtiles, &cfg, place);
     if (rc) return rc;
     if (place == HB_PLACE_GLOBAL && !s->d_gstate) {
         s->gstate_bytes =
@@ -1059,15 +1089,15 @@ static int launch_scan(hb_scan *s)
     rc = plain_scan_args(db, q, place, cfg, &a);
     if (rc) return rc;
     a.gstate = place == HB_PLACE_GLOBAL ? s->d_gstate : nullptr;   // cleared by each wavefront
-    a.work_counter = s->d_misc + 1;
+    a.work_counter = s->d_misc + HB_QUEUE_STRIDE;
     a.out = s->d_out;
     a.out_cap = s->cap;
     a.out_count = s->d_misc;
     a.stats = s->d_stats;
     a.group_totals = nullptr;
-    HB_CHECK(hipMemsetAsync(s->d_misc, 0, 2 * sizeof(uint32_t), c->stream));
+    HB_CHECK(hb_launch_fill_u32(s->d_misc, 0u, HB_SCAN_MISC_WORDS, c->stream));
     HB_CHECK(hipEventRecord(s->ev0, c->stream));
-    if (db->n_tiles) HB_CHECK(hb_launch_scan(a, false, cfg.blocks, cfg.waves * HB_WAVE, cfg.lds, c->stream));
+    if (db->n_qtiles) HB_CHECK(hb_launch_scan(a, false, cfg.blocks, cfg.waves * HB_WAVE, cfg.lds, c->stream));
     HB_CHECK(hipEventRecord(s->ev1, c->stream));
     return HB_OK;
 }
@@ -1088,7 +1118,7 @@ static uint64_t scan_need_bytes(const hb_ctx *c, const hb_query *q, uint64_t fil
                                 uint64_t residues, uint32_t n, uint64_t max_len)
 {
     const uint64_t R = residues ? residues : file_bytes;
-    const uint64_t meta = 8ull * (n + 1) + 16ull * n + 4ull * (n / 64 + 2);
+    const uint64_t meta = 8ull * (n + 1) + 16ull * n + 4ull * (n / 16 + std::min(n, 1u << 17) + 4);
     const uint64_t upload = file_bytes + (R + 64) + 4ull * n + meta;
     const uint64_t resident = (R + 64) + (R + 16ull * n + 64) + meta;
     const uint64_t cap = std::max<uint64_t>(1u << 18, n / 4);
@@ -1238,7 +1268,7 @@ int hb_scan_noalloc(hb_ctx *c, hb_db *db, hb_query *q, hb_hsp *d_hsps, uint32_t 
     if (place < 0) return HB_ERR_UNSUPPORTED;
     hb_launch_cfg cfg;
     int rc = hb_scan_config(c, false, q->gs.qlen_pad_max, q->gs.ctx_pad_max, q->gs.diag_len_max,
-                            db->n_tiles, &cfg, place);
+                            db->n_qtiles, &cfg, place);
     if (rc) return rc;
     hb_scan_args a;
     rc = plain_scan_args(db, q, place, cfg, &a);
@@ -1254,14 +1284,14 @@ int hb_scan_noalloc(hb_ctx *c, hb_db *db, hb_query *q, hb_hsp *d_hsps, uint32_t 
     }
     uint32_t *ctr = reinterpret_cast<uint32_t *>(c->scratch_dev);
     a.out_count = ctr;
-    a.work_counter = ctr + 1;
+    a.work_counter = ctr + HB_QUEUE_STRIDE;
     a.out = d_hsps;
     a.out_cap = hsp_cap;
     a.stats = d_counts;
     a.group_totals = nullptr;
     // the previous call's counters stay in the scratch: cleared by a kernel
-    HB_CHECK(hb_launch_fill_u32(ctr, 0u, 2, st));
-    if (db->n_tiles)
+    HB_CHECK(hb_launch_fill_u32(ctr, 0u, HB_SCAN_MISC_WORDS, st));
+    if (db->n_qtiles)
         HB_CHECK(hb_launch_scan(a, false, blocks, cfg.waves * HB_WAVE, cfg.lds, st));
     HB_CHECK(hipMemcpyAsync(d_n_hsp, ctr, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
     return HB_OK;
@@ -1273,7 +1303,7 @@ int hb_scan_free(hb_scan *s)
     hipSetDevice(s->ctx->device);
     if (!s->waited) hipStreamSynchronize(s->ctx->stream);
     hb_pool_put(s->ctx, s->d_out, (size_t)s->cap * sizeof(hb_hsp));
-    hb_pool_put(s->ctx, s->d_misc, 2 * sizeof(uint32_t));
+    hb_pool_put(s->ctx, s->d_misc, HB_SCAN_MISC_WORDS * sizeof(uint32_t));
     hb_pool_put(s->ctx, s->d_stats, (size_t)std::max<uint32_t>(s->db->n, 1) * 3 * sizeof(uint32_t));
     if (s->d_gstate) hb_pool_put(s->ctx, s->d_gstate, s->gstate_bytes);
     if (s->ev0) hipEventDestroy(s->ev0);
@@ -1301,7 +1331,7 @@ int hb_scan_start(hb_ctx *c, hb_db *db, hb_query *q, hb_scan **out)
     s->q = q;
     s->cap = std::max<uint32_t>(1u << 18, db->n / 4);
     s->d_out = (hb_hsp *)hb_pool_get(c, (size_t)s->cap * sizeof(hb_hsp));
-    s->d_misc = (uint32_t *)hb_pool_get(c, 2 * sizeof(uint32_t));
+    s->d_misc = (uint32_t *)hb_pool_get(c, HB_SCAN_MISC_WORDS * sizeof(uint32_t));
     s->d_stats = (uint32_t *)hb_pool_get(c, (size_t)std::max<uint32_t>(db->n, 1) * 3 * sizeof(uint32_t));
     if (!s->d_out || !s->d_misc || !s->d_stats) {
         hb_scan_free(s);
