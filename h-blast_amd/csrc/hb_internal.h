@@ -9,6 +9,7 @@
 #define HB_ALPHA 28
 #define HB_NCELLS 32768     // 3 letters x 5 bits
 #define HB_PV_WORDS 1024    // HB_NCELLS / 32
+#define HB_NPAIRS 1024      // letter pairs (a, b) of the cells, 32 cells each
 #define HB_WAVE 64
 #define HB_JOBCAP 128       // queued two-hit extensions per wave (a ring)
 #define HB_BLKCAP 128       // hits waiting on a pending diagonal per wave
@@ -42,9 +43,8 @@ struct hb_group_desc {
     int32_t qlen_pad;            // multiple of 16
     int32_t n_ctx;
     int32_t diag_len;            // >= qlen + window, multiple of 64
-    uint32_t n_entries;
     int32_t ctx_base;            // added to context indices in HSP records
-    int32_t pad[2];
+    int32_t pad[3];
 };
 
 // Kernel arguments of the scan.
@@ -123,21 +123,23 @@ hipError_t hb_launch_gather_subjects(const uint8_t *res, const uint64_t *offs, c
                                      hipStream_t st);
 hipError_t hb_launch_check_residues(const uint8_t *res, uint64_t n, uint32_t *flag,
                                     hipStream_t st);
-// Lookup tables of n groups (grid.y = group).  qflag[q] = residue | 0x80 when
-// the 3-mer at q lies inside one context.
+// Lookup tables of n groups (grid.y = group).
 struct hb_lut_job {
-    const uint8_t *qflag;
-    int32_t qlen;
-    int32_t pad;
-    uint32_t *count_start;       // HB_NCELLS + 1: counts, then exclusive starts
+    // per query offset q: letters q | q+1 << 5 | q+2 << 10, and 0x8000 when
+    // the word seeds (inside one context, unmasked); n_words is qlen rounded
+    // up to a multiple of 256, the words past qlen are 0
+    const uint16_t *words;
+    uint32_t n_words;
+    uint32_t cap;                // room in entries[]: none is written past it
     uint32_t *entries;
     uint2 *cells;
     uint32_t *pv;
-    uint32_t *total;             // total entries of the group
+    uint32_t *pair_sum;          // HB_NPAIRS: entries of each letter pair's cells
+    uint32_t *out;               // {entries, cells with entries} of the group
 };
-// pass 0: count; pass 1: exclusive scan + total; pass 2: fill cells, entries, pv
-hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, int32_t qlen_max,
-                         const int8_t *mat32, int32_t threshold, int pass, hipStream_t st);
+// fill = false: counts (cells[].y, pv, pair_sum); true: starts, entries, out
+hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, const int8_t *mat32,
+                         int32_t threshold, bool fill, hipStream_t st);
 hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int block_threads,
                           size_t lds_bytes, hipStream_t st);
 // Sets the kernel's dynamic-LDS limit and returns its occupancy (call before

@@ -100,76 +100,156 @@ __global__ void check_residues_kernel(const uint8_t *res, uint64_t n, uint32_t *
 // ---------------------------------------------------------------- lookup table
 // Cell w = (a<<10)|(b<<5)|c holds query offset q (a word inside one context)
 // when M[q0][a]+M[q1][b]+M[q2][c] >= T, or when w is the query word itself
-// (an exact word always seeds, also below T).  One thread per cell, query
-// offsets visited ascending, so each cell lists them ascending (as
-// lut_sorting leaves them, h_blast.cu:165-194).  grid.y = group.
-template <int PASS>
+// (an exact word always seeds, also below T), offsets ascending in each cell
+// and the cells' lists one after another (as lut_sorting leaves them,
+// h_blast.cu:165-194).  grid.y = group.
+//
+// One wavefront builds the 32 cells of one letter pair (a, b).  It tests 64
+// query words at a time on M[q0][a] + M[q1][b] + (largest score of q2), which
+// leaves a few percent of them, keeps those in order in LDS and then scores
+// two of them a step on all third letters (lane c of each half).  A thread
+// per cell that scored every query word against its cell did 784 x 28 x qlen
+// steps twice; this does 784 x (qlen / 64 + candidates / 2), so the tables
+// are bound by the latency of a wavefront's steps: both passes together 12 us
+// instead of 39 (with the scan of the counts between them) for 60 residues,
+// 11 us instead of 119 for 350, 97 us instead of 2.25 ms for 8,001, 73 us
+// instead of 777 for 28 groups of 768.  The count pass leaves each pair's
+// sum, from which each wavefront of the fill pass adds up where its cells
+// start.
+constexpr uint32_t kLutList = 2 * HB_WAVE + 8;   // candidates a wavefront keeps, read in eights
+
+template <bool FILL>
 __global__ __launch_bounds__(256) void lut_kernel(const hb_lut_job *jobs, const int8_t *mat32,
                                                   int32_t threshold)
 {
-    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ __align__(16) int8_t sm[1024];   // 32x32
+    __shared__ int8_t top[32];                  // largest score of each letter's row
+    __shared__ int8_t cols[256 / HB_WAVE][64];  // the pair's columns M[.][a], M[.][b]
+    __shared__ uint2 lists[256 / HB_WAVE][kLutList];
     const hb_lut_job J = jobs[blockIdx.y];
-    int8_t *sm = reinterpret_cast<int8_t *>(lds);        // 32x32
-    uint8_t *sq = lds + 1024;                              // qlen bytes
-    for (int i = threadIdx.x; i < 1024; i += blockDim.x) sm[i] = mat32[i];
-    for (int i = threadIdx.x; i < J.qlen; i += blockDim.x) sq[i] = J.qflag[i];
+    const int lane = threadIdx.x & (HB_WAVE - 1), wid = threadIdx.x / HB_WAVE;
+    const uint32_t c = (uint32_t)lane & 31u, half = (uint32_t)lane >> 5;
+    reinterpret_cast<uint32_t *>(sm)[threadIdx.x] =
+        reinterpret_cast<const uint32_t *>(mat32)[threadIdx.x];
     __syncthreads();
-    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t a = w >> 10, b = (w >> 5) & 31, c = w & 31;
-    uint32_t n = 0;
-    if (a < HB_ALPHA && b < HB_ALPHA && c < HB_ALPHA) {
-        uint32_t k = PASS == 2 ? J.count_start[w] : 0;
-        for (int32_t q = 0; q + 3 <= J.qlen; ++q) {
-            const uint8_t f0 = sq[q];
-            if (!(f0 & 0x80)) continue;
-            const uint32_t q0 = f0 & 31, q1 = sq[q + 1] & 31, q2 = sq[q + 2] & 31;
-            const int32_t sc = sm[(q0 << 5) | a] + sm[(q1 << 5) | b] + sm[(q2 << 5) | c];
-            const bool self = (q0 == a) & (q1 == b) & (q2 == c);
-            if (sc >= threshold || self) {
-                if (PASS == 2) J.entries[k++] = (uint32_t)q;
-                ++n;
+    const uint32_t p = blockIdx.x * (256 / HB_WAVE) + (uint32_t)wid;
+    const uint32_t a = p >> 5, b = p & 31;
+    if (threadIdx.x < 32) {
+        int8_t m = sm[threadIdx.x << 5];
+        for (int i = 1; i < HB_ALPHA; ++i) m = max(m, sm[(threadIdx.x << 5) | i]);
+        top[threadIdx.x] = m;
+    }
+    cols[wid][lane] = sm[(c << 5) | (half ? b : a)];
+    __syncthreads();
+    const int8_t *ca = cols[wid], *cb = cols[wid] + 32;
+    uint2 *list = lists[wid];
+    const uint32_t w = (p << 5) | c;
+    const bool valid = a < HB_ALPHA && b < HB_ALPHA;
+
+    uint32_t k = 0;   // FILL: the next entry of cell c; else: its entries (of this half)
+    if (FILL) {
+        uint32_t before = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < HB_NPAIRS / HB_WAVE; ++i) {
+            const uint32_t j = i * HB_WAVE + (uint32_t)lane;
+            const uint32_t v = J.pair_sum[j];
+            before += j < p ? v : 0u;
+        }
+        before = lane63(wave_incl_add(before));
+        const uint32_t n = J.cells[w].y;
+        const uint32_t incl = wave_incl_add(half ? 0u : n);
+        k = before + (uint32_t)__shfl((int)(incl - n), (int)c, HB_WAVE);
+        if (half == 0) J.cells[w] = make_uint2(k, n);
+        if (p == HB_NPAIRS - 1) {   // no word: this wavefront sums up the table
+            uint32_t used = 0;
+            for (uint32_t j = (uint32_t)lane; j < HB_PV_WORDS; j += HB_WAVE)
+                used += (uint32_t)__popc(J.pv[j]);
+            used = lane63(wave_incl_add(used));
+            if (lane == 0) {
+                J.out[0] = before;
+                J.out[1] = used;
             }
         }
     }
-    if (PASS == 0) {
-        J.count_start[w] = n;
-    } else {
-        J.cells[w] = make_uint2(J.count_start[w], n);
-        const uint64_t m = __ballot(n != 0);
-        const int lane = threadIdx.x & 63;
-        if (lane == 0) J.pv[w >> 5] = (uint32_t)m;
-        if (lane == 32) J.pv[w >> 5] = (uint32_t)(m >> 32);
-    }
-}
 
-// Exclusive scan of one group's HB_NCELLS counts in place; [HB_NCELLS] and
-// *total receive the number of entries.  grid.y = group.
-__global__ __launch_bounds__(1024) void lut_scan_kernel(const hb_lut_job *jobs)
-{
-    __shared__ uint32_t part[1024];
-    const hb_lut_job J = jobs[blockIdx.y];
-    uint32_t *cnt = J.count_start;
-    const int t = threadIdx.x;
-    const int per = HB_NCELLS / 1024;
-    uint32_t s = 0;
-    for (int i = 0; i < per; ++i) s += cnt[t * per + i];
-    part[t] = s;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const uint32_t v = t >= o ? part[t - o] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    // Scores the n kept candidates {q, (T - partial + 1024) << 16 | self << 8 |
+    // q2}, eight a step so that their LDS reads overlap: of each two the lower
+    // half's precedes the upper half's.
+    auto score = [&](uint32_t n) {
+        for (uint32_t j = 0; j < n; j += 8) {
+            uint2 e[4];
+            int32_t s[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) e[u] = list[j + 2 * u + half];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[u] = sm[((e[u].y & 31u) << 5) | c];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool hit = j + 2 * u + half < n && c < HB_ALPHA &&
+                                 (s[u] + 1024 >= (int32_t)(e[u].y >> 16) ||
+                                  (((e[u].y >> 8) & 1u) && (e[u].y & 31u) == c));
+                if (FILL) {
+                    const uint64_t m = ballot(hit);
+                    const uint32_t lo = (uint32_t)(m >> c) & 1u, hi = (uint32_t)(m >> (32 + c)) & 1u;
+                    const uint32_t at = k + (half ? lo : 0u);
+                    if (hit && at < J.cap) J.entries[at] = e[u].x;
+                    k += lo + hi;
+                } else {
+                    k += hit;
+                }
+            }
+        }
+    };
+    if (valid) {
+        uint32_t n = 0;   // candidates kept (wave-uniform)
+        // 256 words a step, the next step's loaded ahead (words[] is padded
+        // with words that seed nothing to a multiple of 256)
+        uint16_t nx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nx[i] = J.words[i * HB_WAVE + lane];
+        for (uint32_t q0 = 0; q0 < J.n_words; q0 += 4 * HB_WAVE) {
+            uint16_t cur[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cur[i] = nx[i];
+            if (q0 + 4 * HB_WAVE < J.n_words)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    nx[i] = J.words[q0 + (uint32_t)((4 + i) * HB_WAVE + lane)];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t v = cur[i];
+                const uint32_t l0 = v & 31u, l1 = (v >> 5) & 31u, l2 = (v >> 10) & 31u;
+                const int32_t need = threshold - ca[l0] - cb[l1];
+                const bool self = l0 == a && l1 == b;
+                const uint64_t m = ballot((v & 0x8000u) && (top[l2] >= need || self));
+                if (m) {
+                    if (lane_bit(m))
+                        list[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                            make_uint2(q0 + (uint32_t)(i * HB_WAVE + lane),
+                                       (uint32_t)(need + 1024) << 16 | (uint32_t)self << 8 | l2);
+                    n += (uint32_t)__popcll(m);
+                    if (n >= HB_WAVE) {
+                        wave_lds_sync();
+                        score(n);
+                        n = 0;
+                        wave_lds_sync();
+                    }
+                }
+            }
+        }
+        wave_lds_sync();
+        score(n);
     }
-    uint32_t run = part[t] - s;
-    for (int i = 0; i < per; ++i) {
-        const uint32_t v = cnt[t * per + i];
-        cnt[t * per + i] = run;
-        run += v;
-    }
-    if (t == 1023) {
-        cnt[HB_NCELLS] = run;
-        *J.total = run;
+    if (!FILL) {
+        k += (uint32_t)__shfl_xor((int)k, 32, HB_WAVE);
+        const uint64_t m = ballot(k != 0);
+        const uint32_t sum = lane63(wave_incl_add(half ? 0u : k));
+        if (half == 0) J.cells[w] = make_uint2(0, k);
+        if (lane == 0) {
+            J.pv[p] = (uint32_t)m;
+            J.pair_sum[p] = sum;
+        }
     }
 }
 
@@ -386,7 +466,6 @@ struct WaveScan {
     // counter.
     const HB_GLOBAL uint64_t *cells;   // {start, count} as one 64-bit word
     const HB_GLOBAL uint32_t *entries;
-    uint32_t n_entries;
     int32_t qlen;
     int32_t n_ctx;
     int32_t ctx_base;
@@ -1081,7 +1160,6 @@ __device__ __forceinline__ void bind_group(WaveScan<GS> &w, const hb_group_desc 
 {
     w.cells = (const HB_GLOBAL uint64_t *)G.cells;
     w.entries = (const HB_GLOBAL uint32_t *)G.entries;
-    w.n_entries = G.n_entries > 0 ? G.n_entries : 1u;
     w.qlen = G.qlen;
     w.n_ctx = G.n_ctx;
     w.ctx_base = G.ctx_base;
@@ -1650,25 +1728,16 @@ hipError_t hb_launch_check_residues(const uint8_t *res, uint64_t n, uint32_t *fl
     return hipGetLastError();
 }
 
-hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, int32_t qlen_max,
-                         const int8_t *mat32, int32_t threshold, int pass, hipStream_t st)
+hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, const int8_t *mat32,
+                         int32_t threshold, bool fill, hipStream_t st)
 {
     if (n_jobs <= 0) return hipSuccess;
-    const size_t lds = 1024 + (size_t)((qlen_max + 15) & ~15);
-    if (pass == 1) {
-        hipLaunchKernelGGL(lut_scan_kernel, dim3(1, n_jobs), dim3(1024), 0, st, jobs_dev);
-        return hipGetLastError();
-    }
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(pass == 0 ? lut_kernel<0>
-                                                                                : lut_kernel<2>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    if (pass == 0)
-        hipLaunchKernelGGL(lut_kernel<0>, dim3(HB_NCELLS / 256, n_jobs), dim3(256), lds, st,
-                           jobs_dev, mat32, threshold);
-    else
-        hipLaunchKernelGGL(lut_kernel<2>, dim3(HB_NCELLS / 256, n_jobs), dim3(256), lds, st,
-                           jobs_dev, mat32, threshold);
+    // three scores lie in [-384, 381]: a threshold past that range acts as its
+    // end does, and the kernel's sums stay small
+    const int32_t t = threshold < -400 ? -400 : threshold > 400 ? 400 : threshold;
+    const dim3 grid(HB_NPAIRS / (256 / HB_WAVE), n_jobs), block(256);
+    if (fill) hipLaunchKernelGGL(lut_kernel<true>, grid, block, 0, st, jobs_dev, mat32, t);
+    else hipLaunchKernelGGL(lut_kernel<false>, grid, block, 0, st, jobs_dev, mat32, t);
     return hipGetLastError();
 }
 

@@ -37,6 +37,8 @@ struct hb_ctx {
     std::mutex pin_mu;
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+    // small page-locked buffers for uploads and read-backs (kept, bounded)
+    std::vector<std::pair<void *, size_t>> pins;
     // device address of this GPU's hb_scan_noalloc scratch
     unsigned char *scratch_dev = nullptr;
 };
@@ -44,6 +46,11 @@ struct hb_ctx {
 // Copies device bytes to pageable host memory through the context's pinned
 // staging buffer (DMA at full link speed, then a multi-threaded host copy).
 int hb_copy_out(hb_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t st);
+
+// A page-locked buffer of at least *bytes (set to its size) from the
+// context's list, and back to it; null when out of memory.
+void *hb_pin_get(hb_ctx *c, size_t *bytes);
+void hb_pin_put(hb_ctx *c, void *p, size_t bytes);
 
 void *hb_pool_get(hb_ctx *c, size_t bytes);
 void hb_pool_put(hb_ctx *c, void *p, size_t bytes);
@@ -86,15 +93,15 @@ int hb_check_query(const uint8_t *seq, int32_t len, int32_t n_ctx, const int32_t
                    const int32_t *ctx_len, const int32_t *xdrop);
 
 // Device lookup tables and group descriptors for a set of concatenated
-// queries, all in two allocations (fixed-size tables + entries), taken from
+// queries, in two allocations (tables and inputs, entries), taken from
 // and returned to the context's buffer pool.
 struct hb_group_set {
     hb_ctx *ctx = nullptr;
     std::vector<hb_group_desc> desc;   // host copy
-    hb_group_desc *d_desc = nullptr;   // device copy
-    void *d_fixed = nullptr;           // cells, starts, pv, query, ctx, qflag per group
+    hb_group_desc *d_desc = nullptr;   // device copy, inside d_fixed
+    void *d_fixed = nullptr;           // cells, pv, pair sums per group; the uploaded inputs; totals
     uint32_t *d_entries = nullptr;
-    int8_t *d_mat = nullptr;
+    int8_t *d_mat = nullptr;           // inside d_fixed
     size_t fixed_bytes = 0, entries_bytes = 0;
     int32_t qlen_pad_max = 0, ctx_pad_max = 4, diag_len_max = 64;
     std::vector<uint32_t> n_entries, n_cells_used;

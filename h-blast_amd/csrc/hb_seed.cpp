@@ -71,6 +71,38 @@ void hb_pool_put(hb_ctx *c, void *p, size_t bytes)
     }
 }
 
+void *hb_pin_get(hb_ctx *c, size_t *bytes)
+{
+    {
+        std::lock_guard<std::mutex> lk(c->pin_mu);
+        for (size_t i = 0; i < c->pins.size(); ++i)
+            if (c->pins[i].second >= *bytes) {
+                void *p = c->pins[i].first;
+                *bytes = c->pins[i].second;
+                c->pins.erase(c->pins.begin() + (long)i);
+                return p;
+            }
+    }
+    *bytes = (*bytes + 0x3ffff) & ~(size_t)0x3ffff;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, *bytes, hipHostMallocDefault) != hipSuccess) return nullptr;
+    return p;
+}
+
+// At most 8 buffers of up to 16 MiB are kept.
+void hb_pin_put(hb_ctx *c, void *p, size_t bytes)
+{
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(c->pin_mu);
+        if (c->pins.size() < 8 && bytes <= ((size_t)16 << 20)) {
+            c->pins.emplace_back(p, bytes);
+            return;
+        }
+    }
+    hipHostFree(p);
+}
+
 int hb_copy_out(hb_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t st)
 {
     if (bytes == 0) return HB_OK;
@@ -146,18 +178,21 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 void hb_group_set_free(hb_group_set *g)
 {
     if (!g || !g->ctx) return;
-    hb_pool_put(g->ctx, g->d_desc, g->desc.size() * sizeof(hb_group_desc));
     hb_pool_put(g->ctx, g->d_fixed, g->fixed_bytes);
     hb_pool_put(g->ctx, g->d_entries, g->entries_bytes);
-    hb_pool_put(g->ctx, g->d_mat, 1024);
     g->d_desc = nullptr;
     g->d_fixed = nullptr;
     g->d_entries = nullptr;
     g->d_mat = nullptr;
 }
 
-// Lookup tables of all groups are built together: count pass, per-group
-// exclusive scan, one read-back of the totals, entries allocation, fill pass.
+// Lookup tables of all groups are built together: one upload of the inputs,
+// count pass, fill pass, one read-back of the totals.  The entries get room
+// for kEntriesPerWord of each query word (BLOSUM62 at threshold 11 gives 30
+// on average); tables that turn out larger are filled again with the room
+// they need.
+static constexpr size_t kEntriesPerWord = 64;
+
 int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
                        const std::vector<int32_t> &ctx_base, const hb_resolved_params &p,
                        hipStream_t st, hb_group_set *out)
@@ -166,140 +201,127 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
     if (n == 0 || ctx_base.size() != n) return HB_ERR_ARG;
     out->ctx = c;
     out->desc.assign(n, hb_group_desc{});
-    // per-group layout inside d_fixed
-    const size_t cells_b = HB_NCELLS * sizeof(uint2);
-    const size_t start_b = align256((HB_NCELLS + 1) * sizeof(uint32_t));
-    const size_t pv_b = HB_PV_WORDS * sizeof(uint32_t);
-    std::vector<size_t> off(n + 1, 0);
-    int32_t qlen_max = 0;
+    // d_fixed: the groups' tables, the uploaded inputs (score matrix, jobs,
+    // descriptors, then each group's query, contexts and words), the totals
+    const size_t cells_b = HB_NCELLS * sizeof(uint2), pv_b = HB_PV_WORDS * sizeof(uint32_t);
+    const size_t table_b = cells_b + pv_b + HB_NPAIRS * sizeof(uint32_t);
+    const size_t o_jobs = 1024, o_desc = o_jobs + align256(n * sizeof(hb_lut_job));
+    const size_t o_groups = o_desc + align256(n * sizeof(hb_group_desc));
+    auto query_b = [&](size_t g) { return align256((qs[g].seq.size() + 15) & ~(size_t)15); };
+    auto ctx_b = [&](size_t g) { return align256(3 * qs[g].ctx_off.size() * sizeof(int32_t)); };
+    auto n_words = [&](size_t g) { return (qs[g].seq.size() + 255) & ~(size_t)255; };
+    size_t in_b = o_groups, ent_cap = 0;
     for (size_t g = 0; g < n; ++g) {
         const int32_t qlen = (int32_t)qs[g].seq.size();
-        const int32_t qpad = (qlen + 15) & ~15;
-        const int32_t nctx = (int32_t)qs[g].ctx_off.size();
-        const size_t bytes = cells_b + start_b + pv_b + align256(qpad) +
-                             align256(3 * (size_t)nctx * sizeof(int32_t)) + align256(qlen) + 256;
-        off[g + 1] = off[g] + bytes;
-        qlen_max = std::max(qlen_max, qlen);
-        out->qlen_pad_max = std::max(out->qlen_pad_max, qpad);
-        out->ctx_pad_max = std::max(out->ctx_pad_max, hb_ctx_pad(nctx));
+        in_b += query_b(g) + ctx_b(g) + n_words(g) * sizeof(uint16_t);
+        ent_cap += kEntriesPerWord * (size_t)qlen;
+        out->qlen_pad_max = std::max(out->qlen_pad_max, (qlen + 15) & ~15);
+        out->ctx_pad_max = std::max(out->ctx_pad_max, hb_ctx_pad((int32_t)qs[g].ctx_off.size()));
         out->diag_len_max = std::max(out->diag_len_max, (qlen + p.window + 63) & ~63);
     }
-    out->fixed_bytes = off[n];
-    // host image of the inputs (query, ctx, qflag) and the job table
-    std::vector<uint8_t> img(out->fixed_bytes, 0);
-    std::vector<hb_lut_job> jobs(n);
+    const size_t in_o = n * table_b, tot_o = in_o + in_b, tot_b = 2 * n * sizeof(uint32_t);
+    out->fixed_bytes = tot_o + align256(tot_b);
+    out->entries_bytes = ent_cap * sizeof(uint32_t);
+    size_t pin_b = in_b + tot_b;
+    uint8_t *pin = static_cast<uint8_t *>(hb_pin_get(c, &pin_b));
     out->d_fixed = hb_pool_get(c, out->fixed_bytes);
-    out->d_mat = static_cast<int8_t *>(hb_pool_get(c, 1024));
-    out->d_desc = static_cast<hb_group_desc *>(hb_pool_get(c, n * sizeof(hb_group_desc)));
-    if (!out->d_fixed || !out->d_mat || !out->d_desc) {
-        hb_group_set_free(out);
-        return HB_ERR_NOMEM;
-    }
-    uint8_t *base = static_cast<uint8_t *>(out->d_fixed);
+    out->d_entries = static_cast<uint32_t *>(hb_pool_get(c, out->entries_bytes));
+    auto done = [&](int rc) {
+        if (rc) {
+            hipStreamSynchronize(st);
+            hb_group_set_free(out);
+        }
+        hb_pin_put(c, pin, pin_b);
+        return rc;
+    };
+    if (!pin || !out->d_fixed || !out->d_entries) return done(HB_ERR_NOMEM);
+    uint8_t *base = static_cast<uint8_t *>(out->d_fixed), *in = base + in_o;
+    out->d_mat = reinterpret_cast<int8_t *>(in);
+    out->d_desc = reinterpret_cast<hb_group_desc *>(in + o_desc);
+    hb_lut_job *jobs = reinterpret_cast<hb_lut_job *>(pin + o_jobs);
+    const hb_lut_job *d_jobs = reinterpret_cast<const hb_lut_job *>(in + o_jobs);
+    uint32_t *totals = reinterpret_cast<uint32_t *>(pin + in_b);
+    memset(pin, 0, in_b);
+    memcpy(pin, p.mat32, 1024);
+    size_t o = o_groups, e = 0;
     for (size_t g = 0; g < n; ++g) {
         const hb_concat &Q = qs[g];
         const int32_t qlen = (int32_t)Q.seq.size();
-        const int32_t qpad = (qlen + 15) & ~15;
         const int32_t nctx = (int32_t)Q.ctx_off.size();
-        size_t o = off[g];
-        uint2 *cells = reinterpret_cast<uint2 *>(base + o);
-        o += cells_b;
-        uint32_t *start = reinterpret_cast<uint32_t *>(base + o);
-        o += start_b;
-        uint32_t *pv = reinterpret_cast<uint32_t *>(base + o);
-        o += pv_b;
-        const size_t q_o = o;
-        memcpy(&img[q_o], Q.seq.data(), (size_t)qlen);
-        o += align256(qpad);
-        const size_t c_o = o;
-        int32_t *cimg = reinterpret_cast<int32_t *>(&img[c_o]);
+        const size_t q_o = o, c_o = q_o + query_b(g), w_o = c_o + ctx_b(g);
+        o = w_o + n_words(g) * sizeof(uint16_t);
+        memcpy(pin + q_o, Q.seq.data(), (size_t)qlen);
+        int32_t *cimg = reinterpret_cast<int32_t *>(pin + c_o);
+        uint16_t *words = reinterpret_cast<uint16_t *>(pin + w_o);
         for (int32_t k = 0; k < nctx; ++k) {
             cimg[k] = Q.ctx_off[k];
             cimg[nctx + k] = Q.xdrop[k];
             cimg[2 * nctx + k] = Q.cutoff[k];
+            // masked residues seed no word (NCBI builds its table over the
+            // unmasked segments only)
+            for (int32_t w = Q.ctx_off[k]; w + 3 <= Q.ctx_off[k] + Q.ctx_len[k]; ++w)
+                if (Q.mask.empty() || !(Q.mask[w] | Q.mask[w + 1] | Q.mask[w + 2]))
+                    words[w] = (uint16_t)(0x8000u | Q.seq[w] | Q.seq[w + 1] << 5 | Q.seq[w + 2] << 10);
         }
-        o += align256(3 * (size_t)nctx * sizeof(int32_t));
-        const size_t f_o = o;
-        uint8_t *qf = &img[f_o];
-        for (int32_t i = 0; i < qlen; ++i) qf[i] = Q.seq[i];
-        for (int32_t k = 0; k < nctx; ++k)
-            for (int32_t w = Q.ctx_off[k]; w + 3 <= Q.ctx_off[k] + Q.ctx_len[k]; ++w) qf[w] |= 0x80;
-        // masked residues seed no word (NCBI builds its table over the
-        // unmasked segments only)
-        if (!Q.mask.empty())
-            for (int32_t w = 0; w + 3 <= qlen; ++w)
-                if (Q.mask[w] | Q.mask[w + 1] | Q.mask[w + 2]) qf[w] &= 0x7f;
-        o += align256(qlen);
-        uint32_t *total = reinterpret_cast<uint32_t *>(base + o);
+        uint8_t *t = base + g * table_b;
         hb_group_desc &D = out->desc[g];
-        D.cells = cells;
-        D.pv = pv;
-        D.query = base + q_o;
-        D.ctx = reinterpret_cast<const int32_t *>(base + c_o);
+        D.cells = reinterpret_cast<uint2 *>(t);
+        D.pv = reinterpret_cast<uint32_t *>(t + cells_b);
+        D.entries = out->d_entries + e;
+        D.query = in + q_o;
+        D.ctx = reinterpret_cast<const int32_t *>(in + c_o);
         D.qlen = qlen;
-        D.qlen_pad = qpad;
+        D.qlen_pad = (qlen + 15) & ~15;
         D.n_ctx = nctx;
         D.diag_len = (qlen + p.window + 63) & ~63;
         D.ctx_base = ctx_base[g];
-        jobs[g].qflag = base + f_o;
-        jobs[g].qlen = qlen;
-        jobs[g].count_start = start;
-        jobs[g].cells = cells;
-        jobs[g].pv = pv;
-        jobs[g].total = total;
+        hb_lut_job &J = jobs[g];
+        J.words = reinterpret_cast<const uint16_t *>(in + w_o);
+        J.n_words = (uint32_t)n_words(g);
+        J.cap = (uint32_t)(kEntriesPerWord * (size_t)qlen);
+        J.entries = out->d_entries + e;
+        J.cells = reinterpret_cast<uint2 *>(t);
+        J.pv = reinterpret_cast<uint32_t *>(t + cells_b);
+        J.pair_sum = reinterpret_cast<uint32_t *>(t + cells_b + pv_b);
+        J.out = reinterpret_cast<uint32_t *>(base + tot_o) + 2 * g;
+        e += J.cap;
     }
-    hb_lut_job *d_jobs = static_cast<hb_lut_job *>(hb_pool_get(c, n * sizeof(hb_lut_job)));
-    auto fail = [&](int rc) {
-        hipStreamSynchronize(st);
-        hb_pool_put(c, d_jobs, n * sizeof(hb_lut_job));
-        hb_group_set_free(out);
-        return rc;
+    memcpy(pin + o_desc, out->desc.data(), n * sizeof(hb_group_desc));
+    auto upload_fill = [&](bool count) {
+        return hipMemcpyAsync(in, pin, in_b, hipMemcpyHostToDevice, st) == hipSuccess &&
+               (!count || hb_launch_lut(d_jobs, (int)n, out->d_mat, p.threshold, false, st) ==
+                              hipSuccess) &&
+               hb_launch_lut(d_jobs, (int)n, out->d_mat, p.threshold, true, st) == hipSuccess &&
+               hipMemcpyAsync(totals, base + tot_o, tot_b, hipMemcpyDeviceToHost, st) ==
+                   hipSuccess &&
+               hipStreamSynchronize(st) == hipSuccess;
     };
-    if (!d_jobs) return fail(HB_ERR_NOMEM);
-    // inputs: copy each group's query/ctx/qflag span (the tables are written on the device)
-    for (size_t g = 0; g < n; ++g) {
-        // query, context table and qflag are contiguous in the group's span
-        const size_t q_o = (size_t)(out->desc[g].query - base);
-        const size_t end = (size_t)(jobs[g].qflag - base) + align256(jobs[g].qlen);
-        if (hipMemcpyAsync(base + q_o, &img[q_o], end - q_o, hipMemcpyHostToDevice, st) !=
-            hipSuccess)
-            return fail(HB_ERR_DEVICE);
-    }
-    if (hipMemcpyAsync(out->d_mat, p.mat32, 1024, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemcpyAsync(d_jobs, jobs.data(), n * sizeof(hb_lut_job), hipMemcpyHostToDevice, st) !=
-            hipSuccess ||
-        hb_launch_lut(d_jobs, (int)n, qlen_max, out->d_mat, p.threshold, 0, st) != hipSuccess ||
-        hb_launch_lut(d_jobs, (int)n, qlen_max, out->d_mat, p.threshold, 1, st) != hipSuccess)
-        return fail(HB_ERR_DEVICE);
-    std::vector<uint32_t> totals(n);
-    for (size_t g = 0; g < n; ++g)
-        if (hipMemcpyAsync(&totals[g], jobs[g].total, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           st) != hipSuccess)
-            return fail(HB_ERR_DEVICE);
-    if (hipStreamSynchronize(st) != hipSuccess) return fail(HB_ERR_DEVICE);
-    size_t ent_total = 0;
-    for (uint32_t t : totals) ent_total += t;
-    out->entries_bytes = std::max<size_t>(ent_total, 1) * sizeof(uint32_t);
-    out->d_entries = static_cast<uint32_t *>(hb_pool_get(c, out->entries_bytes));
-    if (!out->d_entries) return fail(HB_ERR_NOMEM);
-    size_t e = 0;
+    if (!upload_fill(true)) return done(HB_ERR_DEVICE);
     out->n_entries.resize(n);
+    out->n_cells_used.resize(n);
+    bool fits = true;
+    size_t need = 0;
     for (size_t g = 0; g < n; ++g) {
-        jobs[g].entries = out->d_entries + e;
-        out->desc[g].entries = out->d_entries + e;
-        out->desc[g].n_entries = totals[g];
-        out->n_entries[g] = totals[g];
-        e += totals[g];
+        out->n_entries[g] = totals[2 * g];
+        out->n_cells_used[g] = totals[2 * g + 1];
+        fits &= totals[2 * g] <= jobs[g].cap;
+        need += totals[2 * g];
     }
-    if (hipMemcpyAsync(d_jobs, jobs.data(), n * sizeof(hb_lut_job), hipMemcpyHostToDevice, st) !=
-            hipSuccess ||
-        hb_launch_lut(d_jobs, (int)n, qlen_max, out->d_mat, p.threshold, 2, st) != hipSuccess ||
-        hipMemcpyAsync(out->d_desc, out->desc.data(), n * sizeof(hb_group_desc),
-                       hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-        return fail(HB_ERR_DEVICE);
-    hb_pool_put(c, d_jobs, n * sizeof(hb_lut_job));
-    return HB_OK;
+    if (!fits) {
+        hb_pool_put(c, out->d_entries, out->entries_bytes);
+        out->entries_bytes = need * sizeof(uint32_t);
+        out->d_entries = static_cast<uint32_t *>(hb_pool_get(c, out->entries_bytes));
+        if (!out->d_entries) return done(HB_ERR_NOMEM);
+        e = 0;
+        for (size_t g = 0; g < n; ++g) {
+            out->desc[g].entries = jobs[g].entries = out->d_entries + e;
+            jobs[g].cap = out->n_entries[g];
+            e += out->n_entries[g];
+        }
+        memcpy(pin + o_desc, out->desc.data(), n * sizeof(hb_group_desc));
+        if (!upload_fill(false)) return done(HB_ERR_DEVICE);
+    }
+    return done(HB_OK);
 }
 
 // Picks wavefronts per workgroup and the staging ring size: the most
@@ -390,7 +412,6 @@ struct hb_query {
     hb_ctx *ctx = nullptr;
     hb_resolved_params p;
     hb_group_set gs;
-    uint32_t n_cells_used = 0;
     std::vector<int32_t> ctx_off, ctx_len;   // host copies (gapped stage)
     int mode = HB_STATE_AUTO;   // requested placement of the diagonal state
     bool lds_fits = true;       // the LDS layout can hold the diagonal words
@@ -515,6 +536,7 @@ int hb_destroy(hb_ctx *c)
     if (c->stream) hipStreamSynchronize(c->stream);
     for (auto &b : c->pool) hipFree(b.first);
     if (c->pinned) hipHostFree(c->pinned);
+    for (auto &b : c->pins) hipHostFree(b.first);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
     return HB_OK;
@@ -955,13 +977,6 @@ int hb_query_prepare_masked(hb_ctx *c, const uint8_t *seq, int32_t len, int32_t 
         delete q;
         return rc;
     }
-    std::vector<uint32_t> pv(HB_PV_WORDS);
-    if (hipMemcpy(pv.data(), q->gs.desc[0].pv, HB_PV_WORDS * 4, hipMemcpyDeviceToHost) !=
-        hipSuccess) {
-        hb_query_free(q);
-        return HB_ERR_DEVICE;
-    }
-    for (uint32_t w : pv) q->n_cells_used += (uint32_t)__builtin_popcount(w);
     *out = q;
     return HB_OK;
 }
@@ -1012,7 +1027,7 @@ int hb_query_lut_info(const hb_query *q, uint32_t *n_entries, uint32_t *n_cells_
 {
     if (!q) return HB_ERR_ARG;
     if (n_entries) *n_entries = q->gs.n_entries[0];
-    if (n_cells_used) *n_cells_used = q->n_cells_used;
+    if (n_cells_used) *n_cells_used = q->gs.n_cells_used[0];
     return HB_OK;
 }
 
