@@ -15,7 +15,7 @@ namespace {
 
 struct Class {
     int32_t g_begin = 0, g_end = 0;   // groups [g_begin, g_end) of the group set
-    int32_t qlen_pad_max = 0, ctx_pad_max = 4, diag_len_max = 64;
+    int32_t qlen_pad_max = 0, ctx_pad_max = 4, diag_len_max = 64, shift_max = 0;
     hb_launch_cfg cfg;
     uint32_t tiles_per_item = 1;
     int place = HB_PLACE_LDS;          // where the diagonal state goes
@@ -155,7 +155,7 @@ static void make_groups(hb_batch *b, int32_t target, std::vector<hb_concat> *gro
             }
         }
         if (masked) G.mask.resize(G.seq.size(), 0);
-        diag->push_back(((int32_t)G.seq.size() + b->p.window + 63) & ~63);
+        diag->push_back(hb_diag_len((int32_t)G.seq.size(), b->p.window, 0));
         groups->push_back(std::move(G));
     }
 }
@@ -176,12 +176,12 @@ static void size_items(hb_batch *b, uint32_t n_tiles)
 
 // Wavefronts per CU that the scan reaches with one class's LDS layout
 // (0 when no configuration fits).
-static int class_waves(hb_batch *b, int32_t qlen_pad, int32_t ctx_pad, int32_t diag_len)
+static int class_waves(hb_batch *b, bool split, int32_t qlen_pad, int32_t ctx_pad, int32_t diag_len)
 {
     const int place = hb_state_choose(b->ctx, diag_len, hb_scan_fixed_lds(qlen_pad, ctx_pad),
                                       b->db->max_len, b->p.window);
     hb_launch_cfg cfg;
-    if (hb_scan_config(b->ctx, true, qlen_pad, ctx_pad, diag_len, 1u << 30, &cfg, place,
+    if (hb_scan_config(b->ctx, true, split, qlen_pad, ctx_pad, diag_len, 1u << 30, &cfg, place,
                        b->g_ring, b->g_waves) != HB_OK)
         return 0;
     return cfg.blocks / std::max(b->ctx->n_cu, 1) * cfg.waves;
@@ -206,7 +206,7 @@ static int build(hb_batch *b, int32_t target)
     for (const hb_concat &G : groups)
         if (!hb_query_lds_ok(b->ctx, (int32_t)G.seq.size(), (int32_t)G.ctx_off.size()))
             return HB_ERR_UNSUPPORTED;
-    int rc = hb_group_set_build(b->ctx, groups, ctx_base, b->p, b->st, &b->gs);
+    int rc = hb_group_set_build(b->ctx, groups, ctx_base, b->p, true, b->st, &b->gs);
     if (rc) return rc;
     const int32_t ng = (int32_t)groups.size();
     for (int32_t g = 0; g < ng;) {
@@ -217,12 +217,16 @@ static int build(hb_batch *b, int32_t target)
         while (g < ng && diag[g] <= lim) {
             const int32_t qp = std::max(c.qlen_pad_max, b->gs.desc[g].qlen_pad);
             const int32_t cp = std::max(c.ctx_pad_max, hb_ctx_pad(b->gs.desc[g].n_ctx));
-            const int32_t dl = std::max(c.diag_len_max, diag[g]);
+            const int32_t dl = std::max(c.diag_len_max, b->gs.desc[g].diag_len);
+            const int32_t sh = std::max(c.shift_max, b->gs.desc[g].shift);
             if (w0 < 0) {
-                w0 = class_waves(b, qp, cp, dl);
+                w0 = class_waves(b, sh > 0, qp, cp, dl);
+            } else if ((sh > 0) != (c.shift_max > 0)) {
+                break;   // the scan of split diagonals is a kernel of its own
             } else if (qp != c.qlen_pad_max || cp != c.ctx_pad_max || dl != c.diag_len_max) {
-                if (class_waves(b, qp, cp, dl) < w0) break;
+                if (class_waves(b, sh > 0, qp, cp, dl) < w0) break;
             }
+            c.shift_max = sh;
             c.qlen_pad_max = qp;
             c.ctx_pad_max = cp;
             c.diag_len_max = dl;
@@ -238,8 +242,11 @@ static int build(hb_batch *b, int32_t target)
         c.place = hb_state_choose(b->ctx, c.diag_len_max,
                                   hb_scan_fixed_lds(c.qlen_pad_max, c.ctx_pad_max),
                                   b->db->max_len, b->p.window);
-        rc = hb_scan_config(b->ctx, true, c.qlen_pad_max, c.ctx_pad_max, c.diag_len_max,
-                            n_groups * b->db->n_tiles, &c.cfg, c.place, b->g_ring, b->g_waves);
+        rc = hb_scan_config(b->ctx, true, c.shift_max > 0, c.qlen_pad_max, c.ctx_pad_max,
+                            c.diag_len_max,
+                            (uint32_t)std::min<uint64_t>(
+                                1u << 30, ((uint64_t)n_groups * b->db->n_tiles) << c.shift_max),
+                            &c.cfg, c.place, b->g_ring, b->g_waves);
         if (rc) return rc;
         if (c.place == HB_PLACE_GLOBAL) {
             c.gstate_bytes =
@@ -292,6 +299,7 @@ static int enqueue(hb_batch *b, uint32_t t_begin, uint32_t t_end)
         a.qlen_pad_max = C.qlen_pad_max;
         a.ctx_pad_max = C.ctx_pad_max;
         a.diag_len_max = C.diag_len_max;
+        a.split = C.shift_max > 0;
         a.wave_lds = (uint32_t)hb_scan_wave_lds(C.diag_len_max, C.cfg.ring,
                                                 hb_state_bytes(C.place));
         a.ring = (uint32_t)C.cfg.ring;
@@ -422,7 +430,10 @@ static int autotune(hb_batch *b, int32_t *best)
     float best_ms = 0, ms = 0;
     *best = 0;
     b->tune_candidates = 0;
-    for (int32_t cand : {512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192}) {
+    // (groups of 6,144 and 8,192 residues were 6-18% slower than 2,048 or
+    // 4,096 with 48 and with 400 queries: the workgroups' copies of the query
+    // leave the rings too little LDS)
+    for (int32_t cand : {512, 768, 1024, 1536, 2048, 3072, 4096}) {
         int rc = time_candidate(b, cand, t0, span, &ms);
         if (rc) return rc;
         if (ms >= 0 && (*best == 0 || ms < best_ms)) {

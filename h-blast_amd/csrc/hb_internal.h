@@ -22,6 +22,9 @@
 #define HB_QUEUE_STRIDE 32  // words between two queues' counters (a 128-byte line each)
 #define HB_QUEUE_WORDS (HB_QUEUES * HB_QUEUE_STRIDE)
 #define HB_BLOCK 256        // at most 4 wavefronts per workgroup
+#define HB_BLOCK_SPLIT 1024 // ... 16 in a plain scan of split diagonals: a workgroup holds the
+                            // whole (long) query
+#define HB_SHIFT_MAX 5      // at most 32 classes of diagonals
 // Diagonal state kept in LDS: one 32-bit word per diagonal, 23-bit positions
 // between resets (hb_scan_args::state_limit), so the longest subject and
 // its successor must fit: 2 * (longest + window) + 64 < 2^23.
@@ -34,7 +37,7 @@
 // contexts) with its lookup table.  The plain path scans one group; the
 // batched path scans many groups in one launch.
 struct hb_group_desc {
-    const uint2 *cells;          // HB_NCELLS cells {start, count}
+    const uint2 *cells;          // HB_NCELLS << shift cells {start, count}
     const uint32_t *entries;     // query offsets, ascending per cell
     const uint32_t *pv;          // HB_PV_WORDS presence bits
     const uint8_t *query;        // qlen_pad bytes (zero padded)
@@ -42,9 +45,14 @@ struct hb_group_desc {
     int32_t qlen;
     int32_t qlen_pad;            // multiple of 16
     int32_t n_ctx;
-    int32_t diag_len;            // >= qlen + window, multiple of 64
+    int32_t diag_len;            // diagonals of one class, multiple of 64:
+                                 // diag_len << shift >= qlen + window
     int32_t ctx_base;            // added to context indices in HSP records
-    int32_t pad[3];
+    // the diagonals q - s are dealt to 2^shift classes by their value mod
+    // 2^shift, and the cells hold each class apart: cell (w << shift | c) the
+    // offsets q = c mod 2^shift of word w
+    int32_t shift;
+    int32_t pad[2];
 };
 
 // Kernel arguments of the scan.
@@ -70,6 +78,7 @@ struct hb_scan_args {
     int32_t qlen_pad_max;
     int32_t ctx_pad_max;         // multiple of 4
     int32_t diag_len_max;
+    int32_t split;               // some group has shift > 0
     uint32_t wave_lds;           // LDS bytes per wave
     uint32_t ring;               // staging ring bytes per wave (multiple of 16): subjects up
                                  // to this length are staged in LDS
@@ -115,6 +124,12 @@ static inline size_t hb_scan_fixed_lds(int32_t qlen_pad, int32_t ctx_pad)
     return 1024 + 12 * (size_t)ctx_pad + qlen_pad;
 }
 
+// Threads of a scan workgroup at most.
+static inline int hb_block_max(bool multi, bool split, bool gstate)
+{
+    return split && !multi && !gstate ? HB_BLOCK_SPLIT : HB_BLOCK;
+}
+
 // Kernel launchers (hb_kernels.hip).
 // Copies every subject's residues (res at offs[oid]) to its processing-order
 // place in out (the record's offset), one workgroup per tile.
@@ -125,17 +140,18 @@ hipError_t hb_launch_check_residues(const uint8_t *res, uint64_t n, uint32_t *fl
                                     hipStream_t st);
 // Lookup tables of n groups (grid.y = group).
 struct hb_lut_job {
-    // per query offset q: letters q | q+1 << 5 | q+2 << 10, and 0x8000 when
-    // the word seeds (inside one context, unmasked); n_words is qlen rounded
-    // up to a multiple of 256, the words past qlen are 0
+    // for the offsets q = i << shift | cls, i ascending: letters q | q+1 << 5 |
+    // q+2 << 10, and 0x8000 when the word seeds (inside one context, unmasked);
+    // n_words is a multiple of 256, the words past the query are 0
     const uint16_t *words;
     uint32_t n_words;
-    uint32_t cap;                // room in entries[]: none is written past it
+    uint32_t first, cap;         // this job's entries: first .. first + cap - 1 at most
+    uint32_t shift, cls;
     uint32_t *entries;
-    uint2 *cells;
-    uint32_t *pv;
+    uint2 *cells;                // class cls's first cell; the next is 1 << shift further
+    uint32_t *pv;                // (the classes' follow one another)
     uint32_t *pair_sum;          // HB_NPAIRS: entries of each letter pair's cells
-    uint32_t *out;               // {entries, cells with entries} of the group
+    uint32_t *out;               // {entries, in class 0's: cells with entries in any class}
 };
 // fill = false: counts (cells[].y, pv, pair_sum); true: starts, entries, out
 hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, const int8_t *mat32,
@@ -146,7 +162,7 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
 // launching or capturing a launch with that LDS size).
 // Raises both scan kernels' dynamic LDS limit to max_lds (once per context).
 hipError_t hb_scan_allow_lds(size_t max_lds);
-hipError_t hb_scan_occupancy(bool multi, bool gstate, size_t lds_bytes,
+hipError_t hb_scan_occupancy(bool multi, bool gstate, bool split, size_t lds_bytes,
                              int block_threads, int *blocks_per_cu);
 hipError_t hb_launch_copy(void *dst, const void *src, uint64_t bytes, hipStream_t st);
 hipError_t hb_launch_fill_u32(uint32_t *dst, uint32_t value, uint32_t n, hipStream_t st);

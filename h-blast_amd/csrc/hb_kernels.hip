@@ -102,7 +102,8 @@ __global__ void check_residues_kernel(const uint8_t *res, uint64_t n, uint32_t *
 // when M[q0][a]+M[q1][b]+M[q2][c] >= T, or when w is the query word itself
 // (an exact word always seeds, also below T), offsets ascending in each cell
 // and the cells' lists one after another (as lut_sorting leaves them,
-// h_blast.cu:165-194).  grid.y = group.
+// h_blast.cu:165-194).  grid.y = job: one per group, or one per class of query
+// offsets (hb_lut_job::cls) of a group whose scan splits the diagonals.
 //
 // One wavefront builds the 32 cells of one letter pair (a, b).  It tests 64
 // query words at a time on M[q0][a] + M[q1][b] + (largest score of q2), which
@@ -156,14 +157,18 @@ __global__ __launch_bounds__(256) void lut_kernel(const hb_lut_job *jobs, const 
             before += j < p ? v : 0u;
         }
         before = lane63(wave_incl_add(before));
-        const uint32_t n = J.cells[w].y;
+        const uint32_t n = J.cells[(size_t)w << J.shift].y;
         const uint32_t incl = wave_incl_add(half ? 0u : n);
-        k = before + (uint32_t)__shfl((int)(incl - n), (int)c, HB_WAVE);
-        if (half == 0) J.cells[w] = make_uint2(k, n);
+        k = J.first + before + (uint32_t)__shfl((int)(incl - n), (int)c, HB_WAVE);
+        if (half == 0) J.cells[(size_t)w << J.shift] = make_uint2(k, n);
         if (p == HB_NPAIRS - 1) {   // no word: this wavefront sums up the table
             uint32_t used = 0;
-            for (uint32_t j = (uint32_t)lane; j < HB_PV_WORDS; j += HB_WAVE)
-                used += (uint32_t)__popc(J.pv[j]);
+            if (J.cls == 0)   // cells that any class has entries in
+                for (uint32_t j = (uint32_t)lane; j < HB_PV_WORDS; j += HB_WAVE) {
+                    uint32_t m = 0;
+                    for (uint32_t i = 0; i < 1u << J.shift; ++i) m |= J.pv[i * HB_PV_WORDS + j];
+                    used += (uint32_t)__popc(m);
+                }
             used = lane63(wave_incl_add(used));
             if (lane == 0) {
                 J.out[0] = before;
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(256) void lut_kernel(const hb_lut_job *jobs, const 
                     const uint64_t m = ballot(hit);
                     const uint32_t lo = (uint32_t)(m >> c) & 1u, hi = (uint32_t)(m >> (32 + c)) & 1u;
                     const uint32_t at = k + (half ? lo : 0u);
-                    if (hit && at < J.cap) J.entries[at] = e[u].x;
+                    if (hit && at < J.first + J.cap) J.entries[at] = e[u].x;
                     k += lo + hi;
                 } else {
                     k += hit;
@@ -226,7 +231,7 @@ __global__ __launch_bounds__(256) void lut_kernel(const hb_lut_job *jobs, const 
                     if (lane_bit(m))
                         list[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
-                            make_uint2(q0 + (uint32_t)(i * HB_WAVE + lane),
+                            make_uint2((q0 + (uint32_t)(i * HB_WAVE + lane)) << J.shift | J.cls,
                                        (uint32_t)(need + 1024) << 16 | (uint32_t)self << 8 | l2);
                     n += (uint32_t)__popcll(m);
                     if (n >= HB_WAVE) {
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(256) void lut_kernel(const hb_lut_job *jobs, const 
         k += (uint32_t)__shfl_xor((int)k, 32, HB_WAVE);
         const uint64_t m = ballot(k != 0);
         const uint32_t sum = lane63(wave_incl_add(half ? 0u : k));
-        if (half == 0) J.cells[w] = make_uint2(0, k);
+        if (half == 0) J.cells[(size_t)w << J.shift] = make_uint2(0, k);
         if (lane == 0) {
             J.pv[p] = (uint32_t)m;
             J.pair_sum[p] = sum;
@@ -454,7 +459,7 @@ template <> struct DiagWord<true> {   // no marker bits: the markers are in an L
 static_assert(HB_LDS_POS_LIMIT <= (1 << 23) && HB_GLOBAL_POS_LIMIT <= (1 << 28),
               "positions (< limit + longest subject) must stay below kP");
 
-template <bool G>
+template <bool G, bool SPLIT>
 struct WaveScan {
     using W = DiagWord<G>;
     using word_t = typename W::T;
@@ -471,6 +476,10 @@ struct WaveScan {
     int32_t ctx_base;
     int32_t D;
     uint32_t dmul;     // ceil(2^32 / D): x mod D by a multiply-high
+    // SPLIT: the diagonals q - s are dealt to 2^shift classes by their value
+    // mod 2^shift; a scan of a subject takes the hits of one class, whose
+    // diagonals have the indices floor((q - s) / 2^shift) mod D
+    uint32_t shift, cls;
     // LDS tables
     const int8_t *mat;
     const uint8_t *qry;
@@ -508,6 +517,11 @@ struct WaveScan {
     }
     __device__ __forceinline__ uint32_t diag_of(uint32_t q, int32_t so) const
     {
+        if (SPLIT) {   // the hit's class is that of its diagonal
+            const uint32_t k = (q - (uint32_t)so) & ((1u << shift) - 1);
+            so = (int32_t)(((uint32_t)so + k) >> shift);
+            q >>= shift;
+        }
         const int32_t d = (int32_t)q - (int32_t)mod_d((uint32_t)so);
         return (uint32_t)(d < 0 ? d + D : d);
     }
@@ -786,6 +800,22 @@ struct WaveScan {
         retire_all();
     }
 
+    // A subject's counters (SPLIT: added up over its classes).
+    __device__ __forceinline__ void put_stats(uint32_t oid, uint32_t h, uint32_t e, uint32_t hs) const
+    {
+        if (!a->stats) return;
+        uint32_t *st = a->stats + 3 * (size_t)oid;
+        if (SPLIT && shift) {
+            atomicAdd(&st[0], h);
+            if (e) atomicAdd(&st[1], e);
+            if (hs) atomicAdd(&st[2], hs);
+        } else {
+            st[0] = h;
+            st[1] = e;
+            st[2] = hs;
+        }
+    }
+
     // Writes the counters of every staged subject and empties the ring.
     __device__ __forceinline__ void retire_all()
     {
@@ -797,11 +827,7 @@ struct WaveScan {
             h = B.x;
             e = B.y;
             hs = B.z;
-            if (a->stats) {
-                a->stats[3 * (size_t)A.x + 0] = h;
-                a->stats[3 * (size_t)A.x + 1] = e;
-                a->stats[3 * (size_t)A.x + 2] = hs;
-            }
+            put_stats(A.x, h, e, hs);
         }
         tot_hits += h;
         tot_ext += e;
@@ -834,11 +860,7 @@ struct WaveScan {
         // wave-uniform, so that the ring state stays uniform
         const uint32_t t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.w);
         if (lane == 0) {
-            if (a->stats) {
-                a->stats[3 * (size_t)A.x + 0] = B.x;
-                a->stats[3 * (size_t)A.x + 1] = B.y;
-                a->stats[3 * (size_t)A.x + 2] = B.z;
-            }
+            put_stats(A.x, B.x, B.y, B.z);
             tot_hits += B.x;
             tot_ext += B.y;
             tot_hsp += B.z;
@@ -909,7 +931,8 @@ struct WaveScan {
         uint32_t excl;
         int32_t eb;
         uint32_t H;
-        int32_t s0, s0m;   // first position, and it mod D
+        int32_t s0, s0m;   // first position, and it mod D (SPLIT: s0 >> shift, s0 is a
+                           // multiple of 64)
     };
 
     // The {start, count} cell of the word at position s0 + lane (0 past the
@@ -922,7 +945,8 @@ struct WaveScan {
         const int32_t s = s0 + lane;
         uint64_t c2 = 0;
         if (s + 3 <= slen) {
-            const uint32_t idx = ((uint32_t)S[s] << 10) | ((uint32_t)S[s + 1] << 5) | S[s + 2];
+            uint32_t idx = ((uint32_t)S[s] << 10) | ((uint32_t)S[s + 1] << 5) | S[s + 2];
+            if (SPLIT) idx = (idx << shift) | (((uint32_t)s + cls) & ((1u << shift) - 1));
             c2 = cells[idx];
         }
         return c2;
@@ -966,6 +990,7 @@ struct WaveScan {
         B = A;
         bool hasB = false;        // B holds the window after A
         int32_t nxt = 0, nxtm = 0;   // the next window to load, and it mod D
+        const int32_t step = SPLIT ? HB_WAVE >> shift : HB_WAVE;   // of nxtm
         uint32_t r = 0;           // hits of A already taken
         uint32_t c = 0;           // carried hits, in lanes 0..c-1
         uint32_t cq = 0, cd = 0;
@@ -987,7 +1012,7 @@ struct WaveScan {
                     make_window(cell_at(S, slen, nxt), nxt, nxtm, A);
                     hits += A.H;
                     nxt += HB_WAVE;
-                    nxtm += HB_WAVE;
+                    nxtm += step;
                     if (nxtm >= D) nxtm -= D;
                 }
                 r = 0;
@@ -1000,7 +1025,7 @@ struct WaveScan {
                 hits += B.H;
                 hasB = true;
                 nxt += HB_WAVE;
-                nxtm += HB_WAVE;
+                nxtm += step;
                 if (nxtm >= D) nxtm -= D;
             }
             const uint32_t t1 = min((uint32_t)HB_WAVE, A.H - r);
@@ -1034,8 +1059,9 @@ struct WaveScan {
                 const int32_t ebb = __builtin_amdgcn_ds_bpermute(p4, B.eb);
                 eb = p >= 64 ? ebb : eb;
             }
-            // (s0 + p) mod D, p < 128 <= 2 D
-            int32_t smp = A.s0m + (int32_t)p;
+            // (s0 + p) mod D, p < 128 <= 2 D (SPLIT: of the diagonal's position
+            // in its class, (s0 + p + cls) >> shift)
+            int32_t smp = A.s0m + (int32_t)(SPLIT ? (p + cls) >> shift : p);
             if (smp >= D) smp -= D;
             if (smp >= D) smp -= D;
             const uint32_t flat = (uint32_t)lane >= t1 ? (uint32_t)lane - t1 : (uint32_t)lane + r;
@@ -1069,7 +1095,7 @@ struct WaveScan {
                 }
             }
             stage();
-            int32_t dn = (int32_t)qn - smp;
+            int32_t dn = (int32_t)(SPLIT ? qn >> shift : qn) - smp;
             if (dn < 0) dn += D;
             const bool isc = (uint32_t)lane < c;
             const uint32_t q = isc ? cq : qn;
@@ -1155,8 +1181,8 @@ __device__ __forceinline__ void load_group(const hb_scan_args &a, const hb_group
     }
 }
 
-template <bool GS>
-__device__ __forceinline__ void bind_group(WaveScan<GS> &w, const hb_group_desc &G)
+template <bool GS, bool SPLIT>
+__device__ __forceinline__ void bind_group(WaveScan<GS, SPLIT> &w, const hb_group_desc &G)
 {
     w.cells = (const HB_GLOBAL uint64_t *)G.cells;
     w.entries = (const HB_GLOBAL uint32_t *)G.entries;
@@ -1165,12 +1191,14 @@ __device__ __forceinline__ void bind_group(WaveScan<GS> &w, const hb_group_desc 
     w.ctx_base = G.ctx_base;
     w.D = G.diag_len;
     w.dmul = (uint32_t)(0xffffffffu / (uint32_t)G.diag_len) + 1u;
+    w.shift = (uint32_t)G.shift;
+    w.cls = 0;
 }
 
 // Scans the subjects of one tile (at most 64): lane j holds the record of
 // subject j, so that the records cost one load per tile.
-template <bool GS>
-__device__ __forceinline__ void scan_tile(WaveScan<GS> &w, const hb_scan_args &a, uint32_t t)
+template <bool GS, bool SPLIT>
+__device__ __forceinline__ void scan_tile(WaveScan<GS, SPLIT> &w, const hb_scan_args &a, uint32_t t)
 {
     const uint32_t s0 = a.tiles[t], ns = a.tiles[t + 1] - s0;
     uint4 rec = make_uint4(0, 0, 0, 0);
@@ -1189,25 +1217,29 @@ __device__ __forceinline__ void scan_tile(WaveScan<GS> &w, const hb_scan_args &a
 // per wavefront of the grid) instead of LDS, for queries (groups) whose
 // state does not fit LDS or would leave it too few wavefronts, and for
 // databases whose subjects are too long for the LDS word's positions.
+// SPLIT: some group's diagonals are dealt to classes (hb_group_desc::shift):
+// an item is scanned once per class, for the hits of that class only.  A
+// launch's LDS then holds one class's diagonals per wavefront, 16 wavefronts
+// a CU where 8,001 residues left room for 4.
 // Every scan kernel keeps a register budget for four wavefronts per SIMD
 // (128 VGPRs), the most a 1000-residue query's LDS leaves room for: at five
 // (96 VGPRs) the many-group kernel spills to scratch, and 20 wavefronts per
 // CU measured slower than 16 where the LDS would allow them.
-template <bool MULTI, bool GSTATE>
+template <bool MULTI, bool GSTATE, bool SPLIT>
 __device__ __forceinline__ void scan_body(const hb_scan_args &a);
 
-template <bool MULTI, bool GSTATE>
-__global__ __launch_bounds__(HB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void hb_scan_kernel(hb_scan_args a)
+template <bool MULTI, bool SPLIT>
+__global__ __launch_bounds__(SPLIT && !MULTI ? HB_BLOCK_SPLIT : HB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void hb_scan_kernel(hb_scan_args a)
 {
-    scan_body<MULTI, GSTATE>(a);
+    scan_body<MULTI, false, SPLIT>(a);
 }
 template <bool MULTI>
 __global__ __launch_bounds__(HB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void hb_scan_kernel_g(hb_scan_args a)
 {
-    scan_body<MULTI, true>(a);
+    scan_body<MULTI, true, true>(a);
 }
 
-template <bool MULTI, bool GSTATE>
+template <bool MULTI, bool GSTATE, bool SPLIT>
 __device__ __forceinline__ void scan_body(const hb_scan_args &a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1223,7 +1255,7 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
     for (int i = threadIdx.x; i < 256; i += blockDim.x)
         reinterpret_cast<uint32_t *>(sm_mat)[i] = reinterpret_cast<const uint32_t *>(a.mat32)[i];
 
-    WaveScan<GSTATE> w;
+    WaveScan<GSTATE, SPLIT> w;
     w.a = &a;
     w.mat = sm_mat;
     w.qry = sm_q;
@@ -1270,13 +1302,19 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
         const uint32_t n_q = min((uint32_t)gridDim.x, (uint32_t)HB_QUEUES);
         const uint32_t k = blockIdx.x % n_q;
         const uint32_t wpb = blockDim.x / HB_WAVE;
-        const uint32_t len = n_tiles > k ? (n_tiles - k + n_q - 1) / n_q : 0u;
+        const uint32_t n_items = SPLIT ? n_tiles << w.shift : n_tiles;   // a tile's classes in a row
+        const uint32_t len = n_items > k ? (n_items - k + n_q - 1) / n_q : 0u;
         const uint32_t first = (gridDim.x - k + n_q - 1) / n_q * wpb;   // the queue's wavefronts
         uint32_t i = (blockIdx.x / n_q) * wpb + (uint32_t)wid;
         while (i < len) {
             uint32_t nx = 0;   // popped ahead: the atomic overlaps the tile's work
             if (lane == 0) nx = atomicAdd(a.work_counter + HB_QUEUE_STRIDE * k, 1u);
-            scan_tile(w, a, a.tile_begin + k + i * n_q);
+            uint32_t t = k + i * n_q;
+            if (SPLIT) {
+                w.cls = t & ((1u << w.shift) - 1);
+                t >>= w.shift;
+            }
+            scan_tile(w, a, a.tile_begin + t);
             i = first + (uint32_t)__builtin_amdgcn_readfirstlane((int)nx);
         }
         w.template finish<true>(w.ring);
@@ -1290,8 +1328,11 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
         // own and meet only where the group changes.
         const uint32_t n_s = a.n_streams, n_q = a.n_queues, tpi = a.tiles_per_item;
         const uint32_t stream = blockIdx.x % n_s, k = (blockIdx.x / n_s) % n_q;
-        const uint32_t n_items = (n_tiles + tpi - 1) / tpi;
-        const uint32_t len = n_items > k ? (n_items - k + n_q - 1) / n_q : 0u;
+        // items of this workgroup's queue in a group whose scan has 2^shift classes
+        auto queue_len = [&](int32_t shift) {
+            const uint32_t n = ((n_tiles + tpi - 1) / tpi) << (SPLIT ? shift : 0);
+            return n > k ? (n - k + n_q - 1) / n_q : 0u;
+        };
         const uint32_t n_own = (a.n_groups - stream + n_s - 1) / n_s;
         uint32_t pos = 0;   // candidates already passed over (wavefront 0)
         for (;;) {
@@ -1304,7 +1345,8 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
                     if (p < n_own + a.n_groups)
                         left = __hip_atomic_load(
                                    &a.work_counter[(size_t)gp * HB_QUEUE_WORDS + HB_QUEUE_STRIDE * k],
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < len;
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                               queue_len(SPLIT ? a.groups[gp].shift : 0);
                     const uint64_t m = ballot(left);
                     if (m) {
                         const int f = (int)__builtin_ctzll(m);
@@ -1324,13 +1366,19 @@ __device__ __forceinline__ void scan_body(const hb_scan_args &a)
             w.clear_words();
             __syncthreads();
             uint32_t *ctr = a.work_counter + (size_t)g * HB_QUEUE_WORDS + HB_QUEUE_STRIDE * k;
+            const uint32_t len = queue_len(G.shift);
             uint32_t i = 0;
             if (lane == 0) i = atomicAdd(ctr, 1u);
             i = (uint32_t)__builtin_amdgcn_readfirstlane((int)i);
             while (i < len) {
                 uint32_t nx = 0;
                 if (lane == 0) nx = atomicAdd(ctr, 1u);
-                const uint32_t t0 = a.tile_begin + (k + i * n_q) * tpi;
+                uint32_t it = k + i * n_q;
+                if (SPLIT) {
+                    w.cls = it & ((1u << w.shift) - 1);
+                    it >>= w.shift;
+                }
+                const uint32_t t0 = a.tile_begin + it * tpi;
                 const uint32_t t1 = min(t0 + tpi, a.tile_end);
                 for (uint32_t t = t0; t < t1; ++t) scan_tile(w, a, t);
                 i = (uint32_t)__builtin_amdgcn_readfirstlane((int)nx);
@@ -1741,12 +1789,14 @@ hipError_t hb_launch_lut(const hb_lut_job *jobs_dev, int n_jobs, const int8_t *m
     return hipGetLastError();
 }
 
-// Instantiations: (MULTI, GSTATE).
-static const void *scan_fn(bool multi, bool gstate)
+static const void *scan_fn(bool multi, bool gstate, bool split)
 {
     if (gstate)
         return multi ? reinterpret_cast<const void *>(hb_scan_kernel_g<true>)
                      : reinterpret_cast<const void *>(hb_scan_kernel_g<false>);
+    if (split)
+        return multi ? reinterpret_cast<const void *>(hb_scan_kernel<true, true>)
+                     : reinterpret_cast<const void *>(hb_scan_kernel<false, true>);
     return multi ? reinterpret_cast<const void *>(hb_scan_kernel<true, false>)
                  : reinterpret_cast<const void *>(hb_scan_kernel<false, false>);
 }
@@ -1754,16 +1804,20 @@ static const void *scan_fn(bool multi, bool gstate)
 hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int block_threads,
                           size_t lds_bytes, hipStream_t st)
 {
-    if (block_threads < HB_WAVE || block_threads > HB_BLOCK || block_threads % HB_WAVE)
+    const bool g = a.gstate != nullptr, split = a.split != 0;
+    const int top = hb_block_max(multi, split, g);
+    if (block_threads < HB_WAVE || block_threads > top || block_threads % HB_WAVE)
         return hipErrorInvalidValue;
     if (a.ring % 16 || a.wave_lds % 16 || a.state_limit <= 0) return hipErrorInvalidValue;
-    const bool g = a.gstate != nullptr;
     const dim3 grid(n_blocks), block(block_threads);
-    if (multi) {
-        if (g) hipLaunchKernelGGL(hb_scan_kernel_g<true>, grid, block, lds_bytes, st, a);
-        else hipLaunchKernelGGL((hb_scan_kernel<true, false>), grid, block, lds_bytes, st, a);
+    if (g) {
+        if (multi) hipLaunchKernelGGL(hb_scan_kernel_g<true>, grid, block, lds_bytes, st, a);
+        else hipLaunchKernelGGL(hb_scan_kernel_g<false>, grid, block, lds_bytes, st, a);
+    } else if (split) {
+        if (multi) hipLaunchKernelGGL((hb_scan_kernel<true, true>), grid, block, lds_bytes, st, a);
+        else hipLaunchKernelGGL((hb_scan_kernel<false, true>), grid, block, lds_bytes, st, a);
     } else {
-        if (g) hipLaunchKernelGGL(hb_scan_kernel_g<false>, grid, block, lds_bytes, st, a);
+        if (multi) hipLaunchKernelGGL((hb_scan_kernel<true, false>), grid, block, lds_bytes, st, a);
         else hipLaunchKernelGGL((hb_scan_kernel<false, false>), grid, block, lds_bytes, st, a);
     }
     return hipGetLastError();
@@ -1771,8 +1825,8 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
 
 hipError_t hb_scan_allow_lds(size_t max_lds)
 {
-    for (int k = 0; k < 4; ++k) {
-        const void *fn = scan_fn((k & 1) != 0, (k & 2) != 0);
+    for (int k = 0; k < 6; ++k) {
+        const void *fn = scan_fn((k & 1) != 0, k >= 4, (k & 2) != 0);
         hipFuncAttributes fa;
         hipError_t e = hipFuncGetAttributes(&fa, fn);
         if (e != hipSuccess) return e;
@@ -1784,9 +1838,9 @@ hipError_t hb_scan_allow_lds(size_t max_lds)
     return hipSuccess;
 }
 
-hipError_t hb_scan_occupancy(bool multi, bool gstate, size_t lds_bytes, int block_threads,
-                             int *blocks_per_cu)
+hipError_t hb_scan_occupancy(bool multi, bool gstate, bool split, size_t lds_bytes,
+                             int block_threads, int *blocks_per_cu)
 {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, scan_fn(multi, gstate),
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, scan_fn(multi, gstate, split),
                                                         block_threads, lds_bytes);
 }

@@ -104,11 +104,12 @@ struct hb_group_set {
     int8_t *d_mat = nullptr;           // inside d_fixed
     size_t fixed_bytes = 0, entries_bytes = 0;
     int32_t qlen_pad_max = 0, ctx_pad_max = 4, diag_len_max = 64;
+    int32_t split = 0;                 // some group's diagonals are split into classes
     std::vector<uint32_t> n_entries, n_cells_used;
 };
 int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &queries,
                        const std::vector<int32_t> &ctx_base, const hb_resolved_params &p,
-                       hipStream_t st, hb_group_set *out);
+                       bool multi, hipStream_t st, hb_group_set *out);
 void hb_group_set_free(hb_group_set *g);
 
 // Launch configuration of the scan for a given LDS layout.
@@ -153,9 +154,17 @@ size_t hb_gstate_bytes_max(const hb_ctx *c, int32_t D);
 // place: where the diagonal state goes (LDS bytes per diagonal follow).
 // ring_cap > 0 caps the staging ring, waves > 0 fixes the wavefronts per
 // workgroup (autotuner constraints; HB_ERR_UNSUPPORTED if nothing fits).
-int hb_scan_config(hb_ctx *c, bool multi, int32_t qlen_pad_max, int32_t ctx_pad_max,
+int hb_scan_config(hb_ctx *c, bool multi, bool split, int32_t qlen_pad_max, int32_t ctx_pad_max,
                    int32_t diag_len_max, uint32_t work_items, hb_launch_cfg *cfg,
                    int place = HB_PLACE_LDS, int32_t ring_cap = 0, int32_t waves = 0);
+// The classes of diagonals (2^shift) of a plain scan, or of a many-group one
+// (multi), for a concatenated query, and the diagonals of one class (a multiple
+// of 64).
+int32_t hb_diag_shift(const hb_ctx *c, bool multi, int32_t qlen, int32_t n_ctx, int32_t window);
+static inline int32_t hb_diag_len(int32_t qlen, int32_t window, int32_t shift)
+{
+    return ((((qlen + window + (1 << shift) - 1) >> shift) + 63) & ~63);
+}
 
 // Asynchronous steps of a batch (hb_batch.cpp), used by the serving loop:
 // the batch runs on the given stream (nullptr: the context's); launch

@@ -195,7 +195,7 @@ static constexpr size_t kEntriesPerWord = 64;
 
 int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
                        const std::vector<int32_t> &ctx_base, const hb_resolved_params &p,
-                       hipStream_t st, hb_group_set *out)
+                       bool multi, hipStream_t st, hb_group_set *out)
 {
     const size_t n = qs.size();
     if (n == 0 || ctx_base.size() != n) return HB_ERR_ARG;
@@ -203,23 +203,36 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
     out->desc.assign(n, hb_group_desc{});
     // d_fixed: the groups' tables, the uploaded inputs (score matrix, jobs,
     // descriptors, then each group's query, contexts and words), the totals
+    // (a job and its tables per class of a group's diagonals)
     const size_t cells_b = HB_NCELLS * sizeof(uint2), pv_b = HB_PV_WORDS * sizeof(uint32_t);
     const size_t table_b = cells_b + pv_b + HB_NPAIRS * sizeof(uint32_t);
-    const size_t o_jobs = 1024, o_desc = o_jobs + align256(n * sizeof(hb_lut_job));
+    std::vector<int32_t> shift(n);
+    size_t nj = 0;
+    for (size_t g = 0; g < n; ++g) {
+        shift[g] = hb_diag_shift(c, multi, (int32_t)qs[g].seq.size(),
+                                 (int32_t)qs[g].ctx_off.size(), p.window);
+        nj += (size_t)1 << shift[g];
+    }
+    const size_t o_jobs = 1024, o_desc = o_jobs + align256(nj * sizeof(hb_lut_job));
     const size_t o_groups = o_desc + align256(n * sizeof(hb_group_desc));
     auto query_b = [&](size_t g) { return align256((qs[g].seq.size() + 15) & ~(size_t)15); };
     auto ctx_b = [&](size_t g) { return align256(3 * qs[g].ctx_off.size() * sizeof(int32_t)); };
-    auto n_words = [&](size_t g) { return (qs[g].seq.size() + 255) & ~(size_t)255; };
+    // words and entries of one class
+    auto class_words = [&](size_t g) {
+        return (qs[g].seq.size() + ((size_t)1 << shift[g]) - 1) >> shift[g];
+    };
+    auto n_words = [&](size_t g) { return (class_words(g) + 255) & ~(size_t)255; };
     size_t in_b = o_groups, ent_cap = 0;
     for (size_t g = 0; g < n; ++g) {
         const int32_t qlen = (int32_t)qs[g].seq.size();
-        in_b += query_b(g) + ctx_b(g) + n_words(g) * sizeof(uint16_t);
-        ent_cap += kEntriesPerWord * (size_t)qlen;
+        in_b += query_b(g) + ctx_b(g) + (n_words(g) * sizeof(uint16_t) << shift[g]);
+        ent_cap += kEntriesPerWord * class_words(g) << shift[g];
         out->qlen_pad_max = std::max(out->qlen_pad_max, (qlen + 15) & ~15);
         out->ctx_pad_max = std::max(out->ctx_pad_max, hb_ctx_pad((int32_t)qs[g].ctx_off.size()));
-        out->diag_len_max = std::max(out->diag_len_max, (qlen + p.window + 63) & ~63);
+        out->diag_len_max = std::max(out->diag_len_max, hb_diag_len(qlen, p.window, shift[g]));
+        out->split |= shift[g] > 0;
     }
-    const size_t in_o = n * table_b, tot_o = in_o + in_b, tot_b = 2 * n * sizeof(uint32_t);
+    const size_t in_o = nj * table_b, tot_o = in_o + in_b, tot_b = 2 * nj * sizeof(uint32_t);
     out->fixed_bytes = tot_o + align256(tot_b);
     out->entries_bytes = ent_cap * sizeof(uint32_t);
     size_t pin_b = in_b + tot_b;
@@ -243,13 +256,15 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
     uint32_t *totals = reinterpret_cast<uint32_t *>(pin + in_b);
     memset(pin, 0, in_b);
     memcpy(pin, p.mat32, 1024);
-    size_t o = o_groups, e = 0;
+    size_t o = o_groups, e = 0, j = 0;
     for (size_t g = 0; g < n; ++g) {
         const hb_concat &Q = qs[g];
         const int32_t qlen = (int32_t)Q.seq.size();
         const int32_t nctx = (int32_t)Q.ctx_off.size();
         const size_t q_o = o, c_o = q_o + query_b(g), w_o = c_o + ctx_b(g);
-        o = w_o + n_words(g) * sizeof(uint16_t);
+        const uint32_t sh = (uint32_t)shift[g], nc = 1u << sh;
+        const size_t nw = n_words(g);
+        o = w_o + nw * nc * sizeof(uint16_t);
         memcpy(pin + q_o, Q.seq.data(), (size_t)qlen);
         int32_t *cimg = reinterpret_cast<int32_t *>(pin + c_o);
         uint16_t *words = reinterpret_cast<uint16_t *>(pin + w_o);
@@ -261,62 +276,79 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
             // unmasked segments only)
             for (int32_t w = Q.ctx_off[k]; w + 3 <= Q.ctx_off[k] + Q.ctx_len[k]; ++w)
                 if (Q.mask.empty() || !(Q.mask[w] | Q.mask[w + 1] | Q.mask[w + 2]))
-                    words[w] = (uint16_t)(0x8000u | Q.seq[w] | Q.seq[w + 1] << 5 | Q.seq[w + 2] << 10);
+                    words[(w & (nc - 1)) * nw + (w >> sh)] =
+                        (uint16_t)(0x8000u | Q.seq[w] | Q.seq[w + 1] << 5 | Q.seq[w + 2] << 10);
         }
-        uint8_t *t = base + g * table_b;
+        uint8_t *t = base + j * table_b;   // nc classes' cells, presence bits, pair sums
         hb_group_desc &D = out->desc[g];
         D.cells = reinterpret_cast<uint2 *>(t);
-        D.pv = reinterpret_cast<uint32_t *>(t + cells_b);
+        D.pv = reinterpret_cast<uint32_t *>(t + nc * cells_b);
         D.entries = out->d_entries + e;
         D.query = in + q_o;
         D.ctx = reinterpret_cast<const int32_t *>(in + c_o);
         D.qlen = qlen;
         D.qlen_pad = (qlen + 15) & ~15;
         D.n_ctx = nctx;
-        D.diag_len = (qlen + p.window + 63) & ~63;
+        D.diag_len = hb_diag_len(qlen, p.window, shift[g]);
         D.ctx_base = ctx_base[g];
-        hb_lut_job &J = jobs[g];
-        J.words = reinterpret_cast<const uint16_t *>(in + w_o);
-        J.n_words = (uint32_t)n_words(g);
-        J.cap = (uint32_t)(kEntriesPerWord * (size_t)qlen);
-        J.entries = out->d_entries + e;
-        J.cells = reinterpret_cast<uint2 *>(t);
-        J.pv = reinterpret_cast<uint32_t *>(t + cells_b);
-        J.pair_sum = reinterpret_cast<uint32_t *>(t + cells_b + pv_b);
-        J.out = reinterpret_cast<uint32_t *>(base + tot_o) + 2 * g;
-        e += J.cap;
+        D.shift = shift[g];
+        const uint32_t cap = (uint32_t)(kEntriesPerWord * class_words(g));
+        for (uint32_t k = 0; k < nc; ++k, ++j) {
+            hb_lut_job &J = jobs[j];
+            J.words = reinterpret_cast<const uint16_t *>(in + w_o) + k * nw;
+            J.n_words = (uint32_t)nw;
+            J.first = k * cap;
+            J.cap = cap;
+            J.shift = sh;
+            J.cls = k;
+            J.entries = out->d_entries + e;
+            J.cells = reinterpret_cast<uint2 *>(t) + k;
+            J.pv = reinterpret_cast<uint32_t *>(t + nc * cells_b + k * pv_b);
+            J.pair_sum = reinterpret_cast<uint32_t *>(t + nc * (cells_b + pv_b)) + k * HB_NPAIRS;
+            J.out = reinterpret_cast<uint32_t *>(base + tot_o) + 2 * j;
+        }
+        e += (size_t)cap * nc;
     }
     memcpy(pin + o_desc, out->desc.data(), n * sizeof(hb_group_desc));
     auto upload_fill = [&](bool count) {
         return hipMemcpyAsync(in, pin, in_b, hipMemcpyHostToDevice, st) == hipSuccess &&
-               (!count || hb_launch_lut(d_jobs, (int)n, out->d_mat, p.threshold, false, st) ==
+               (!count || hb_launch_lut(d_jobs, (int)nj, out->d_mat, p.threshold, false, st) ==
                               hipSuccess) &&
-               hb_launch_lut(d_jobs, (int)n, out->d_mat, p.threshold, true, st) == hipSuccess &&
+               hb_launch_lut(d_jobs, (int)nj, out->d_mat, p.threshold, true, st) == hipSuccess &&
                hipMemcpyAsync(totals, base + tot_o, tot_b, hipMemcpyDeviceToHost, st) ==
                    hipSuccess &&
                hipStreamSynchronize(st) == hipSuccess;
     };
     if (!upload_fill(true)) return done(HB_ERR_DEVICE);
-    out->n_entries.resize(n);
+    out->n_entries.assign(n, 0);
     out->n_cells_used.resize(n);
     bool fits = true;
     size_t need = 0;
+    j = 0;
     for (size_t g = 0; g < n; ++g) {
-        out->n_entries[g] = totals[2 * g];
-        out->n_cells_used[g] = totals[2 * g + 1];
-        fits &= totals[2 * g] <= jobs[g].cap;
-        need += totals[2 * g];
+        out->n_cells_used[g] = totals[2 * j + 1];
+        for (size_t k = 0; k < (size_t)1 << shift[g]; ++k, ++j) {
+            out->n_entries[g] += totals[2 * j];
+            fits &= totals[2 * j] <= jobs[j].cap;
+        }
+        need += out->n_entries[g];
     }
     if (!fits) {
         hb_pool_put(c, out->d_entries, out->entries_bytes);
         out->entries_bytes = need * sizeof(uint32_t);
         out->d_entries = static_cast<uint32_t *>(hb_pool_get(c, out->entries_bytes));
         if (!out->d_entries) return done(HB_ERR_NOMEM);
-        e = 0;
+        e = j = 0;
         for (size_t g = 0; g < n; ++g) {
-            out->desc[g].entries = jobs[g].entries = out->d_entries + e;
-            jobs[g].cap = out->n_entries[g];
-            e += out->n_entries[g];
+            out->desc[g].entries = out->d_entries + e;
+            uint32_t first = 0;
+            for (size_t k = 0; k < (size_t)1 << shift[g]; ++k, ++j) {
+                jobs[j].entries = out->d_entries + e;
+                jobs[j].first = first;
+                jobs[j].cap = totals[2 * j];
+                first += totals[2 * j];
+            }
+            e += first;
         }
         memcpy(pin + o_desc, out->desc.data(), n * sizeof(hb_group_desc));
         if (!upload_fill(false)) return done(HB_ERR_DEVICE);
@@ -333,7 +365,7 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
 // more wavefronts per workgroup (they share the query tables).  The batched
 // form stages at most 2048 residues per wave: its largest class of C3
 // queries lost a workgroup per CU to larger staging.
-int hb_scan_config(hb_ctx *c, bool multi, int32_t qlen_pad_max, int32_t ctx_pad_max,
+int hb_scan_config(hb_ctx *c, bool multi, bool split, int32_t qlen_pad_max, int32_t ctx_pad_max,
                    int32_t diag_len_max, uint32_t work_items, hb_launch_cfg *cfg, int place,
                    int32_t ring_cap, int32_t force_waves)
 {
@@ -343,13 +375,14 @@ int hb_scan_config(hb_ctx *c, bool multi, int32_t qlen_pad_max, int32_t ctx_pad_
     int32_t ring_top = multi ? std::min(HB_RING_MAX, 2048) : HB_RING_MAX;
     if (ring_cap > 0) ring_top = std::min(ring_top, ring_cap & ~63);
     int best_wpc = 0;
-    for (int waves : {4, 2, 1}) {
+    for (int waves : {16, 8, 4, 2, 1}) {
         if (force_waves > 0 && waves != force_waves) continue;
+        if (waves * HB_WAVE > hb_block_max(multi, split, gstate)) continue;
         for (int32_t ring = ring_top; ring >= 256; ring -= 64) {
             const size_t lds = fixed + waves * hb_scan_wave_lds(diag_len_max, ring, sb);
             if (lds > c->max_lds) continue;
             int per_cu = 0;
-            HB_CHECK(hb_scan_occupancy(multi, gstate, lds, waves * HB_WAVE, &per_cu));
+            HB_CHECK(hb_scan_occupancy(multi, gstate, split, lds, waves * HB_WAVE, &per_cu));
             const int wpc = std::min(per_cu * waves, 16);
             if (wpc > best_wpc || (wpc == best_wpc && ring > cfg->ring)) {
                 best_wpc = wpc;
@@ -393,6 +426,29 @@ int hb_state_choose(const hb_ctx *c, int32_t D, size_t fixed, uint64_t max_len, 
     if (hb_state_lds_ok(max_len, window) && lds_waves(c, D, fixed, 4) >= kGstateMinWaves)
         return HB_PLACE_LDS;
     return HB_PLACE_GLOBAL;
+}
+
+// The fewest classes with which 16 wavefronts per CU (workgroups of 4, or one
+// of 16 for a plain scan of several classes) have LDS for their diagonals and
+// a ring of kSplitRing residues.  A class scans the windows of every subject
+// again, so more classes than that cost: G hits/s of a plain scan with 1, 2,
+// 4, .. classes, 1,500 residues 130, 122, 89; 2,000 89, 135, 104; 3,000 101,
+// 145, 122; 6,000 55, 101, 138, 121; 8,001 56, 95, 76, 135, 103; 12,000 (one
+// class: state in global memory) 45, ., 100, 132, 120; 24,000 41, .., 100, 89,
+// 117.  Queries whose diagonals no LDS layout holds at once keep one class in
+// global memory.
+static constexpr int32_t kSplitRing = 512;
+int32_t hb_diag_shift(const hb_ctx *c, bool multi, int32_t qlen, int32_t n_ctx, int32_t window)
+{
+    const size_t fixed = hb_scan_fixed_lds((qlen + 15) & ~15, hb_ctx_pad(n_ctx));
+    if (fixed + hb_scan_wave_lds(hb_diag_len(qlen, window, 0), 256, 4) > c->max_lds) return 0;
+    int32_t shift = 0;
+    while (shift < HB_SHIFT_MAX &&
+           (shift && !multi ? 1 : 4) * fixed +
+                   16 * hb_scan_wave_lds(hb_diag_len(qlen, window, shift), kSplitRing, 4) >
+               c->max_lds)
+        ++shift;
+    return shift;
 }
 
 bool hb_query_lds_ok(const hb_ctx *c, int32_t qlen, int32_t n_ctx)
@@ -972,7 +1028,7 @@ int hb_query_prepare_masked(hb_ctx *c, const uint8_t *seq, int32_t len, int32_t 
         delete q;
         return HB_ERR_DEVICE;
     }
-    rc = hb_group_set_build(c, qs, std::vector<int32_t>(1, 0), q->p, c->stream, &q->gs);
+    rc = hb_group_set_build(c, qs, std::vector<int32_t>(1, 0), q->p, false, c->stream, &q->gs);
     if (rc) {
         delete q;
         return rc;
@@ -1038,15 +1094,25 @@ int hb_query_lut_fetch(const hb_query *q, uint32_t *cell_start, uint32_t *entrie
     if (!entries && ne) return HB_ERR_ARG;
     if (cap < ne) return HB_ERR_CAPACITY;
     HB_CHECK(hipSetDevice(q->ctx->device));
-    std::vector<uint2> cells(HB_NCELLS);
-    HB_CHECK(hipMemcpy(cells.data(), q->gs.desc[0].cells, HB_NCELLS * sizeof(uint2),
+    const int32_t nc = 1 << q->gs.desc[0].shift;
+    std::vector<uint2> cells((size_t)HB_NCELLS * nc);
+    std::vector<uint32_t> ent(q->gs.entries_bytes / sizeof(uint32_t));
+    HB_CHECK(hipMemcpy(cells.data(), q->gs.desc[0].cells, cells.size() * sizeof(uint2),
                        hipMemcpyDeviceToHost));
-    // every cell holds its exclusive start, empty ones included (CSR)
-    for (int i = 0; i < HB_NCELLS; ++i) cell_start[i] = cells[i].x;
-    cell_start[HB_NCELLS] = ne;
     if (ne)
-        HB_CHECK(hipMemcpy(entries, q->gs.desc[0].entries, (size_t)ne * sizeof(uint32_t),
+        HB_CHECK(hipMemcpy(ent.data(), q->gs.desc[0].entries, q->gs.entries_bytes,
                            hipMemcpyDeviceToHost));
+    // a cell's entries are those of its classes, ascending
+    uint32_t k = 0;
+    for (int i = 0; i < HB_NCELLS; ++i) {
+        cell_start[i] = k;
+        for (int32_t j = 0; j < nc; ++j) {
+            const uint2 x = cells[(size_t)i * nc + j];
+            for (uint32_t e = 0; e < x.y; ++e) entries[k++] = ent[x.x + e];
+        }
+        if (nc > 1) std::sort(entries + cell_start[i], entries + k);
+    }
+    cell_start[HB_NCELLS] = k;
     return HB_OK;
 }
 
@@ -1068,6 +1134,7 @@ static int plain_scan_args(const hb_db *db, const hb_query *q, int place,
     a->qlen_pad_max = q->gs.qlen_pad_max;
     a->ctx_pad_max = q->gs.ctx_pad_max;
     a->diag_len_max = q->gs.diag_len_max;
+    a->split = q->gs.split;
     a->wave_lds = (uint32_t)hb_scan_wave_lds(q->gs.diag_len_max, cfg.ring, hb_state_bytes(place));
     a->ring = (uint32_t)cfg.ring;
     a->state_limit = hb_state_limit(place, db->max_len);
@@ -1091,8 +1158,8 @@ static int launch_scan(hb_scan *s)
     const int place = state_place(q, db);
     if (place < 0) return HB_ERR_UNSUPPORTED;   // LDS state asked for, subjects too long
     s->place = place;
-    int rc = hb_scan_config(c, false, q->gs.qlen_pad_max, q->gs.ctx_pad_max, q->gs.diag_len_max,
-                            db->n_qtiles, &cfg, place);
+    int rc = hb_scan_config(c, false, q->gs.split != 0, q->gs.qlen_pad_max, q->gs.ctx_pad_max,
+                            q->gs.diag_len_max, db->n_qtiles << q->gs.desc[0].shift, &cfg, place);
     if (rc) return rc;
     if (place == HB_PLACE_GLOBAL && !s->d_gstate) {
         s->gstate_bytes =
@@ -1111,6 +1178,7 @@ static int launch_scan(hb_scan *s)
     a.stats = s->d_stats;
     a.group_totals = nullptr;
     HB_CHECK(hb_launch_fill_u32(s->d_misc, 0u, HB_SCAN_MISC_WORDS, c->stream));
+    if (a.split) HB_CHECK(hb_launch_fill_u32(s->d_stats, 0u, 3 * db->n, c->stream));
     HB_CHECK(hipEventRecord(s->ev0, c->stream));
     if (db->n_qtiles) HB_CHECK(hb_launch_scan(a, false, cfg.blocks, cfg.waves * HB_WAVE, cfg.lds, c->stream));
     HB_CHECK(hipEventRecord(s->ev1, c->stream));
@@ -1282,8 +1350,8 @@ int hb_scan_noalloc(hb_ctx *c, hb_db *db, hb_query *q, hb_hsp *d_hsps, uint32_t 
     const int place = state_place(q, db);
     if (place < 0) return HB_ERR_UNSUPPORTED;
     hb_launch_cfg cfg;
-    int rc = hb_scan_config(c, false, q->gs.qlen_pad_max, q->gs.ctx_pad_max, q->gs.diag_len_max,
-                            db->n_qtiles, &cfg, place);
+    int rc = hb_scan_config(c, false, q->gs.split != 0, q->gs.qlen_pad_max, q->gs.ctx_pad_max,
+                            q->gs.diag_len_max, db->n_qtiles << q->gs.desc[0].shift, &cfg, place);
     if (rc) return rc;
     hb_scan_args a;
     rc = plain_scan_args(db, q, place, cfg, &a);
@@ -1306,6 +1374,7 @@ int hb_scan_noalloc(hb_ctx *c, hb_db *db, hb_query *q, hb_hsp *d_hsps, uint32_t 
     a.group_totals = nullptr;
     // the previous call's counters stay in the scratch: cleared by a kernel
     HB_CHECK(hb_launch_fill_u32(ctr, 0u, HB_SCAN_MISC_WORDS, st));
+    if (a.split && d_counts) HB_CHECK(hb_launch_fill_u32(d_counts, 0u, 3 * db->n, st));
     if (db->n_qtiles)
         HB_CHECK(hb_launch_scan(a, false, blocks, cfg.waves * HB_WAVE, cfg.lds, st));
     HB_CHECK(hipMemcpyAsync(d_n_hsp, ctr, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));

@@ -97,11 +97,12 @@ static void estimate(const hb_server *s, Request *r)
 {
     const double cells = (double)r->residues * (double)s->db->total;
     r->est_hsps = (uint64_t)(s->o.hsp_per_cell * cells) + 256;
-    const size_t group_fixed = HB_NCELLS * (sizeof(uint2) + sizeof(uint32_t)) + 8192 +
-                               HB_PV_WORDS * sizeof(uint32_t);
+    const int32_t shift = hb_diag_shift(s->ctx, true, (int32_t)r->residues, 8, s->window);
+    const size_t group_fixed = ((HB_NCELLS * sizeof(uint2) + HB_PV_WORDS * sizeof(uint32_t) +
+                                 HB_NPAIRS * sizeof(uint32_t)) << shift) + 8192;
     r->est_bytes = r->est_hsps * sizeof(hb_hsp) + group_fixed +
                    64 * sizeof(uint32_t) * (size_t)r->residues;
-    const int32_t D = (int32_t)((r->residues + s->window + 63) & ~63);
+    const int32_t D = hb_diag_len((int32_t)r->residues, s->window, shift);
     if (hb_state_choose(s->ctx, D, hb_scan_fixed_lds((int32_t)((r->residues + 15) & ~15), 8),
                         s->db->max_len, s->window) == HB_PLACE_GLOBAL)
         r->est_bytes += hb_gstate_bytes_max(s->ctx, D);
