@@ -6,7 +6,7 @@
 #include <chrono>
 #include <cstring>
 #include <numeric>
-#include <thread>
+#include <tuple>
 #include <vector>
 
 #include "hb_runtime.h"
@@ -54,7 +54,12 @@ struct hb_batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float kernel_ms = 0;
     uint64_t tot[3] = {0, 0, 0};
-    std::vector<hb_hsp> results;               // ordered by (query, oid, s_off, q_off)
+    // the last pass's records, ordered by (query, oid, s_off, q_off): in a
+    // page-locked buffer, or in the vector when there are many
+    std::vector<hb_hsp> many;
+    const hb_hsp *results = nullptr;
+    void *pin = nullptr;
+    size_t pin_bytes = 0;
     std::vector<uint64_t> q_first, q_count;
 };
 
@@ -469,63 +474,123 @@ static int autotune(hb_batch *b, int32_t *best)
     return HB_OK;
 }
 
-// Fetches the n records and per-group counters of the last pass, maps
-// records back to their queries (local context and offsets) and orders each
-// query's records by (oid, s_off, q_off).
-static int collect(hb_batch *b, uint32_t n)
+static int bits_of(uint64_t v)
 {
-    b->results.resize(n);
+    int b = 0;
+    for (; v; v >>= 1) ++b;
+    return b;
+}
+
+static void drop_results(hb_batch *b)
+{
+    hb_pin_put(b->ctx, b->pin, b->pin_bytes);
+    b->pin = nullptr;
+    b->results = nullptr;
+}
+
+// The same without device memory: the records are mapped and ordered here.
+static int collect_host(hb_batch *b, uint32_t n)
+{
+    hipGetLastError();   // the allocation that failed
     std::vector<unsigned long long> tot(3 * b->gs.desc.size());
     HB_CHECK(hipMemcpyAsync(tot.data(), b->d_totals, tot.size() * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, b->st));
-    HB_CHECK(hipStreamSynchronize(b->st));
-    if (n) {
-        const int rc = hb_copy_out(b->ctx, b->results.data(), b->d_out, (size_t)n * sizeof(hb_hsp), b->st);
-        if (rc) return rc;
-    }
+    b->many.resize(n);
+    const int rc = hb_copy_out(b->ctx, b->many.data(), b->d_out, (size_t)n * sizeof(hb_hsp), b->st);
+    if (rc) return rc;
     b->tot[0] = b->tot[1] = b->tot[2] = 0;
-    for (size_t g = 0; g < b->gs.desc.size(); ++g)
-        for (int k = 0; k < 3; ++k) b->tot[k] += tot[3 * g + k];
-    // partition by query (counting), then order each query's records on
-    // host threads
-    const size_t nq = b->queries.size();
-    std::vector<int32_t> qid(n);
+    for (size_t i = 0; i < tot.size(); ++i) b->tot[i % 3] += tot[i];
+    std::sort(b->many.begin(), b->many.end(), [&](const hb_hsp &x, const hb_hsp &y) {
+        const int32_t qx = b->ctx_query[x.context], qy = b->ctx_query[y.context];
+        return std::tie(qx, x.oid, x.s_off, x.q_off) < std::tie(qy, y.oid, y.s_off, y.q_off);
+    });
+    for (hb_hsp &h : b->many) {
+        const int32_t q = b->ctx_query[h.context];
+        h.context = b->ctx_local[h.context];
+        h.q_start -= b->q_base[q];
+        h.q_off -= b->q_base[q];
+        b->q_count[q]++;
+    }
+    for (size_t q = 0; q < b->q_count.size(); ++q) b->q_first[q + 1] = b->q_first[q] + b->q_count[q];
+    b->results = b->many.data();
+    return HB_OK;
+}
+
+// Orders the n records of the last pass on the device, mapped to their
+// queries' contexts and offsets, and fetches them with the per-group counters.
+static int collect(hb_batch *b, uint32_t n)
+{
+    hb_ctx *c = b->ctx;
+    const size_t nq = b->queries.size(), ng = b->gs.desc.size(), nc = b->ctx_query.size();
+    drop_results(b);
     b->q_first.assign(nq + 1, 0);
     b->q_count.assign(nq, 0);
-    for (uint32_t i = 0; i < n; ++i) {
-        hb_hsp &h = b->results[i];
-        const int32_t qi = b->ctx_query[h.context];
-        qid[i] = qi;
-        h.context = b->ctx_local[h.context];
-        h.q_start -= b->q_base[qi];
-        h.q_off -= b->q_base[qi];
-        b->q_count[qi]++;
+    // one page-locked buffer: context map (up), totals, first records (down),
+    // then the records unless they are many
+    constexpr size_t kPinMax = (size_t)12 << 20;
+    const size_t map_b = nc * sizeof(int4), tot_b = 3 * ng * sizeof(unsigned long long);
+    const size_t first_b = (nq + 1) * sizeof(uint32_t), rec_b = (size_t)n * sizeof(hb_hsp);
+    auto up16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
+    const size_t o_tot = up16(map_b), o_first = o_tot + up16(tot_b), o_rec = o_first + up16(first_b);
+    const bool pinned = rec_b <= kPinMax;
+    b->pin_bytes = o_rec + (pinned ? rec_b : 0);
+    b->pin = hb_pin_get(c, &b->pin_bytes);
+    if (!b->pin) return HB_ERR_NOMEM;
+    char *pin = static_cast<char *>(b->pin);
+    int4 *map = reinterpret_cast<int4 *>(pin);
+    int32_t longest = 0;
+    for (const hb_concat &q : b->queries) longest = std::max(longest, (int32_t)q.seq.size());
+    for (size_t k = 0; k < nc; ++k)
+        map[k] = make_int4(b->ctx_query[k], b->ctx_local[k], b->q_base[b->ctx_query[k]], 0);
+    const size_t scr_b = n ? hb_order_scratch(n) : 0, dev_b = up16(map_b) + up16(first_b) + rec_b + scr_b;
+    char *dev = n ? static_cast<char *>(hb_pool_get(c, dev_b)) : nullptr;
+    if (n && !dev) return collect_host(b, n);
+    hipError_t e = hipMemcpyAsync(pin + o_tot, b->d_totals, tot_b, hipMemcpyDeviceToHost, b->st);
+    hb_order_args a{};
+    if (n) {
+        a.in = b->d_out;
+        a.n = n;
+        a.ctx_map = reinterpret_cast<const int4 *>(dev);
+        a.n_queries = (int32_t)nq;
+        a.s_bits = bits_of(b->db->max_len);
+        a.q_bits = bits_of((uint64_t)longest);
+        a.query_bits = bits_of(nq - 1);
+        a.oid_bits = bits_of(b->db->n - 1);
+        a.q_first = reinterpret_cast<uint32_t *>(dev + up16(map_b));
+        a.out = reinterpret_cast<hb_hsp *>(dev + up16(map_b) + up16(first_b));
+        if (e == hipSuccess) e = hipMemcpyAsync(dev, map, map_b, hipMemcpyHostToDevice, b->st);
+        if (e == hipSuccess) e = hb_launch_order(a, dev + up16(map_b) + up16(first_b) + rec_b, b->st);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(pin + o_first, a.q_first, first_b, hipMemcpyDeviceToHost, b->st);
+        if (e == hipSuccess && pinned)
+            e = hipMemcpyAsync(pin + o_rec, a.out, rec_b, hipMemcpyDeviceToHost, b->st);
     }
-    for (size_t q = 0; q < nq; ++q) b->q_first[q + 1] = b->q_first[q] + b->q_count[q];
-    std::vector<hb_hsp> sorted(n);
-    {
-        std::vector<uint64_t> cur(b->q_first.begin(), b->q_first.end() - 1);
-        for (uint32_t i = 0; i < n; ++i) sorted[cur[qid[i]]++] = b->results[i];
+    if (e == hipSuccess) e = hipStreamSynchronize(b->st);
+    int rc = HB_OK;
+    if (e != hipSuccess) {
+        hb_note_hip_error(e, "collect", __LINE__);
+        rc = HB_ERR_DEVICE;
     }
-    const unsigned nt = std::max(1u, std::min<unsigned>({16u, std::thread::hardware_concurrency(),
-                                                         (unsigned)std::max<size_t>(1, nq)}));
-    auto order = [&](size_t t) {
-        for (size_t q = t; q < nq; q += nt)
-            std::sort(sorted.begin() + (long)b->q_first[q], sorted.begin() + (long)b->q_first[q + 1],
-                      [](const hb_hsp &x, const hb_hsp &y) {
-                          if (x.oid != y.oid) return x.oid < y.oid;
-                          if (x.s_off != y.s_off) return x.s_off < y.s_off;
-                          return x.q_off < y.q_off;
-                      });
-    };
-    if (nt == 1 || n < 65536) {
-        for (size_t t = 0; t < nt; ++t) order(t);
+    b->results = reinterpret_cast<const hb_hsp *>(pin + o_rec);
+    if (!rc && !pinned) {
+        b->many.resize(n);
+        b->results = b->many.data();
+        rc = hb_copy_out(c, b->many.data(), a.out, rec_b, b->st);
     } else {
-        std::vector<std::thread> th;
-        for (unsigned t = 0; t < nt; ++t) th.emplace_back(order, (size_t)t);
-        for (auto &x : th) x.join();
+        std::vector<hb_hsp>().swap(b->many);
     }
-    b->results.swap(sorted);
+    hb_pool_put(c, dev, dev_b);
+    if (rc) return rc;
+    b->tot[0] = b->tot[1] = b->tot[2] = 0;
+    const auto *tot = reinterpret_cast<const unsigned long long *>(pin + o_tot);
+    for (size_t g = 0; g < ng; ++g)
+        for (int k = 0; k < 3; ++k) b->tot[k] += tot[3 * g + k];
+    const auto *first = reinterpret_cast<const uint32_t *>(pin + o_first);
+    for (size_t q = 0; n && q < nq; ++q) {
+        b->q_first[q] = first[q];
+        b->q_count[q] = first[q + 1] - first[q];
+    }
+    b->q_first[nq] = n;
     return HB_OK;
 }
 
@@ -752,6 +817,7 @@ int hb_batch_free(hb_batch *b)
     hipSetDevice(b->ctx->device);
     hipStreamSynchronize(b->st);
     free_groups(b);
+    drop_results(b);
     hb_pool_put(b->ctx, b->d_out, (size_t)b->cap * sizeof(hb_hsp));
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);

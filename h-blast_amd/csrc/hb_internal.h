@@ -194,6 +194,24 @@ hipError_t hb_launch_finalize_compact(const uint32_t *st3, uint32_t ns, const hb
 hipError_t hb_launch_first_index(const uint32_t *st3, uint32_t ns, uint32_t *first,
                                  uint32_t *scratch, hipStream_t st);
 
+// Batched results (hb_order.hip): the pass's records in the order (query, oid,
+// s_off, q_off) with their query's contexts and offsets.
+struct hb_order_args {
+    const hb_hsp *in;
+    uint32_t n;
+    const int4 *ctx_map;         // per context of the pass {query, context in it, its base, 0}
+    int32_t n_queries;
+    // bits that the fields can set: s_off and q_off, query and oid (each pair
+    // 64 at most)
+    int s_bits, q_bits, query_bits, oid_bits;
+    hb_hsp *out;
+    uint32_t *q_first;           // n_queries + 1: each query's first record, then n
+    uint64_t *key[2];            // set by hb_launch_order
+    uint32_t *idx[2];
+};
+size_t hb_order_scratch(uint32_t n);   // bytes
+hipError_t hb_launch_order(hb_order_args a, void *scratch, hipStream_t st);
+
 // ---------------------------------------------------------------- gapped stage
 // Kernel arguments of the preliminary gapped extension (hb_gapped.hip).
 #define HB_GAP_RING 256       // DP columns per wavefront kept in LDS (power of two)
