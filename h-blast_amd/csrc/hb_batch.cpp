@@ -474,13 +474,6 @@ static int autotune(hb_batch *b, int32_t *best)
     return HB_OK;
 }
 
-static int bits_of(uint64_t v)
-{
-    int b = 0;
-    for (; v; v >>= 1) ++b;
-    return b;
-}
-
 static void drop_results(hb_batch *b)
 {
     hb_pin_put(b->ctx, b->pin, b->pin_bytes);
@@ -542,7 +535,7 @@ static int collect(hb_batch *b, uint32_t n)
     for (const hb_concat &q : b->queries) longest = std::max(longest, (int32_t)q.seq.size());
     for (size_t k = 0; k < nc; ++k)
         map[k] = make_int4(b->ctx_query[k], b->ctx_local[k], b->q_base[b->ctx_query[k]], 0);
-    const size_t scr_b = n ? hb_order_scratch(n) : 0, dev_b = up16(map_b) + up16(first_b) + rec_b + scr_b;
+    const size_t scr_b = n ? hb_sort_scratch(n) : 0, dev_b = up16(map_b) + up16(first_b) + rec_b + scr_b;
     char *dev = n ? static_cast<char *>(hb_pool_get(c, dev_b)) : nullptr;
     if (n && !dev) return collect_host(b, n);
     hipError_t e = hipMemcpyAsync(pin + o_tot, b->d_totals, tot_b, hipMemcpyDeviceToHost, b->st);
@@ -552,10 +545,10 @@ static int collect(hb_batch *b, uint32_t n)
         a.n = n;
         a.ctx_map = reinterpret_cast<const int4 *>(dev);
         a.n_queries = (int32_t)nq;
-        a.s_bits = bits_of(b->db->max_len);
-        a.q_bits = bits_of((uint64_t)longest);
-        a.query_bits = bits_of(nq - 1);
-        a.oid_bits = bits_of(b->db->n - 1);
+        a.s_bits = hb_bits_of(b->db->max_len);
+        a.q_bits = hb_bits_of((uint64_t)longest);
+        a.query_bits = hb_bits_of(nq - 1);
+        a.oid_bits = hb_bits_of(b->db->n - 1);
         a.q_first = reinterpret_cast<uint32_t *>(dev + up16(map_b));
         a.out = reinterpret_cast<hb_hsp *>(dev + up16(map_b) + up16(first_b));
         if (e == hipSuccess) e = hipMemcpyAsync(dev, map, map_b, hipMemcpyHostToDevice, b->st);

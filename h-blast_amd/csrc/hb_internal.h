@@ -131,13 +131,6 @@ static inline int hb_block_max(bool multi, bool split, bool gstate)
 }
 
 // Kernel launchers (hb_kernels.hip).
-// Copies every subject's residues (res at offs[oid]) to its processing-order
-// place in out (the record's offset), one workgroup per tile.
-hipError_t hb_launch_gather_subjects(const uint8_t *res, const uint64_t *offs, const uint4 *subj,
-                                     const uint32_t *tiles, uint32_t n_tiles, uint8_t *out,
-                                     hipStream_t st);
-hipError_t hb_launch_check_residues(const uint8_t *res, uint64_t n, uint32_t *flag,
-                                    hipStream_t st);
 // Lookup tables of n groups (grid.y = group).
 struct hb_lut_job {
     // for the offsets q = i << shift | cls, i ascending: letters q | q+1 << 5 |
@@ -194,6 +187,44 @@ hipError_t hb_launch_finalize_compact(const uint32_t *st3, uint32_t ns, const hb
 hipError_t hb_launch_first_index(const uint32_t *st3, uint32_t ns, uint32_t *first,
                                  uint32_t *scratch, hipStream_t st);
 
+// Stable LSD radix sort of n 64-bit keys with their indices (hb_order.hip),
+// 8 bits a pass over the lowest `bits` bits; the result is in key[src], idx[src].
+struct hb_sort {
+    uint64_t *key[2];
+    uint32_t *idx[2];
+    uint32_t *counts, *totals;
+    uint32_t n;
+    int src;
+};
+static inline int hb_bits_of(uint64_t v)   // bits that values up to v can set
+{
+    int b = 0;
+    for (; v; v >>= 1) ++b;
+    return b;
+}
+size_t hb_sort_scratch(uint32_t n);   // bytes
+void hb_sort_init(hb_sort *s, uint32_t n, void *scratch);
+void hb_launch_sort(hb_sort *s, int bits, hipStream_t st);
+
+// Loading a database (hb_load.hip): records {oid, length, place low, high} in
+// processing order (length-descending, then oid), and the residues copied
+// to those places (16-byte aligned, ends padded with 0), checked on the way.
+struct hb_load_args {
+    const uint8_t *res;          // packed residues and 64 spare bytes
+    const uint64_t *offs;        // n + 1
+    uint32_t n;
+    uint64_t max_len;
+    uint4 *subj;                 // records (n)
+    uint8_t *out;                // copy
+    uint32_t *flag;              // |= 1 when a residue is >= HB_ALPHA
+    hb_sort sort;                // set by hb_launch_load_records
+    uint64_t *part;
+};
+size_t hb_load_scratch(uint32_t n);   // bytes
+hipError_t hb_launch_load_records(hb_load_args a, void *scratch, hipStream_t st);
+// bytes: the copy's (the last record's place and padded length)
+hipError_t hb_launch_load_copy(const hb_load_args &a, uint64_t bytes, hipStream_t st);
+
 // Batched results (hb_order.hip): the pass's records in the order (query, oid,
 // s_off, q_off) with their query's contexts and offsets.
 struct hb_order_args {
@@ -206,10 +237,9 @@ struct hb_order_args {
     int s_bits, q_bits, query_bits, oid_bits;
     hb_hsp *out;
     uint32_t *q_first;           // n_queries + 1: each query's first record, then n
-    uint64_t *key[2];            // set by hb_launch_order
-    uint32_t *idx[2];
+    hb_sort sort;                // set by hb_launch_order
 };
-size_t hb_order_scratch(uint32_t n);   // bytes
+// scratch: hb_sort_scratch(n) bytes
 hipError_t hb_launch_order(hb_order_args a, void *scratch, hipStream_t st);
 
 // ---------------------------------------------------------------- gapped stage

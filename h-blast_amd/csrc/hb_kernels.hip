@@ -80,23 +80,6 @@ __device__ __forceinline__ uint32_t lane63(uint32_t v)
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 __device__ __forceinline__ bool lane_bit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// ---------------------------------------------------------------- residues
-__global__ void check_residues_kernel(const uint8_t *res, uint64_t n, uint32_t *flag)
-{
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    uint32_t bad = 0;
-    const uint64_t n4 = n / 4;
-    const uint32_t *r4 = reinterpret_cast<const uint32_t *>(res);
-    for (uint64_t k = i; k < n4; k += stride) {
-        const uint32_t w = r4[k];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) bad |= (((w >> (8 * b)) & 0xffu) >= HB_ALPHA);
-    }
-    for (uint64_t k = n4 * 4 + i; k < n; k += stride) bad |= (res[k] >= HB_ALPHA);
-    if (bad) atomicOr(flag, 1u);
-}
-
 // ---------------------------------------------------------------- lookup table
 // Cell w = (a<<10)|(b<<5)|c holds query offset q (a word inside one context)
 // when M[q0][a]+M[q1][b]+M[q2][c] >= T, or when w is the query word itself
@@ -1739,40 +1722,6 @@ hipError_t hb_launch_fill_u32(uint32_t *dst, uint32_t value, uint32_t n, hipStre
     const uint32_t blocks = n ? (n + 255) / 256 : 1;
     hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, st, dst,
                        value, n);
-    return hipGetLastError();
-}
-
-__global__ void gather_subjects_kernel(const uint8_t *res, const uint64_t *offs, const uint4 *subj,
-                                       const uint32_t *tiles, uint8_t *out)
-{
-    const uint32_t t = blockIdx.x;
-    for (uint32_t i = tiles[t]; i < tiles[t + 1]; ++i) {
-        const uint4 m = subj[i];
-        const uint8_t *src = res + offs[m.x];
-        uint8_t *dst = out + ((uint64_t)m.z | ((uint64_t)m.w << 32));
-        for (uint32_t j = threadIdx.x; j < m.y; j += blockDim.x) dst[j] = src[j];
-    }
-}
-
-hipError_t hb_launch_gather_subjects(const uint8_t *res, const uint64_t *offs, const uint4 *subj,
-                                     const uint32_t *tiles, uint32_t n_tiles, uint8_t *out,
-                                     hipStream_t st)
-{
-    if (n_tiles == 0) return hipSuccess;
-    hipLaunchKernelGGL(gather_subjects_kernel, dim3(n_tiles), dim3(256), 0, st, res, offs, subj,
-                       tiles, out);
-    return hipGetLastError();
-}
-
-hipError_t hb_launch_check_residues(const uint8_t *res, uint64_t n, uint32_t *flag,
-                                    hipStream_t st)
-{
-    if (n == 0) return hipSuccess;
-    uint64_t blocks = (n / 4 + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(check_residues_kernel, dim3((unsigned)blocks), dim3(256), 0, st, res, n,
-                       flag);
     return hipGetLastError();
 }
 

@@ -33,18 +33,18 @@ __global__ __launch_bounds__(kThreads) void order_lo_kernel(hb_order_args a)
 {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= a.n) return;
-    a.key[0][i] = key_of(a, i, false);
-    a.idx[0][i] = i;
+    a.sort.key[0][i] = key_of(a, i, false);
+    a.sort.idx[0][i] = i;
 }
 
-__global__ __launch_bounds__(kThreads) void order_hi_kernel(hb_order_args a, int src)
+__global__ __launch_bounds__(kThreads) void order_hi_kernel(hb_order_args a)
 {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < a.n) a.key[src][i] = key_of(a, a.idx[src][i], true);
+    if (i < a.n) a.sort.key[a.sort.src][i] = key_of(a, a.sort.idx[a.sort.src][i], true);
 }
 
 // Keys of each digit in each block: counts[digit * blocks + block].
-__global__ __launch_bounds__(kThreads) void order_count_kernel(const uint64_t *key, uint32_t n,
+__global__ __launch_bounds__(kThreads) void sort_count_kernel(const uint64_t *key, uint32_t n,
                                                                int shift, uint32_t *counts)
 {
     __shared__ uint32_t h[kDigits];
@@ -75,7 +75,7 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t *sm, uint32_
 
 // One block per digit: its blocks' counts become exclusive sums, their total
 // goes to totals[digit].
-__global__ __launch_bounds__(kThreads) void order_scan_kernel(uint32_t *counts, uint32_t blocks,
+__global__ __launch_bounds__(kThreads) void sort_scan_kernel(uint32_t *counts, uint32_t blocks,
                                                               uint32_t *totals)
 {
     __shared__ uint32_t sm[kThreads];
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void order_scan_kernel(uint32_t *counts, 
 // Moves keys and indices to their digit's place, in order: a wavefront takes
 // kWaveKeys consecutive keys, 64 a round, and a key's rank among its digit's
 // keys of the round is the number of lower lanes with the same digit.
-__global__ __launch_bounds__(kThreads) void order_move_kernel(const uint64_t *key,
+__global__ __launch_bounds__(kThreads) void sort_move_kernel(const uint64_t *key,
                                                               const uint32_t *idx, uint32_t n,
                                                               int shift, const uint32_t *counts,
                                                               const uint32_t *totals,
@@ -149,14 +149,15 @@ __global__ __launch_bounds__(kThreads) void order_move_kernel(const uint64_t *ke
 
 // The records in order, with their query's contexts and offsets, and each
 // query's first record (q_first[n_queries] = n).
-__global__ __launch_bounds__(kThreads) void order_emit_kernel(hb_order_args a, int src)
+__global__ __launch_bounds__(kThreads) void order_emit_kernel(hb_order_args a)
 {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= a.n) return;
-    hb_hsp h = a.in[a.idx[src][i]];
+    const uint32_t *idx = a.sort.idx[a.sort.src];
+    hb_hsp h = a.in[idx[i]];
     const int4 m = a.ctx_map[h.context];
     int32_t prev = -1;
-    if (i > 0) prev = a.ctx_map[a.in[a.idx[src][i - 1]].context].x;
+    if (i > 0) prev = a.ctx_map[a.in[idx[i - 1]].context].x;
     for (int32_t q = prev + 1; q <= m.x; ++q) a.q_first[q] = i;
     if (i == a.n - 1)
         for (int32_t q = m.x + 1; q <= a.n_queries; ++q) a.q_first[q] = a.n;
@@ -168,38 +169,50 @@ __global__ __launch_bounds__(kThreads) void order_emit_kernel(hb_order_args a, i
 
 }  // namespace
 
-size_t hb_order_scratch(uint32_t n)
+size_t hb_sort_scratch(uint32_t n)
 {
     const size_t blocks = (n + kBlockKeys - 1) / kBlockKeys;
-    return (size_t)n * 2 * (sizeof(uint64_t) + sizeof(uint32_t)) +
-           (blocks + 1) * kDigits * sizeof(uint32_t) + 64;
+    const size_t b = (size_t)n * 2 * (sizeof(uint64_t) + sizeof(uint32_t)) +
+                     (blocks + 1) * kDigits * sizeof(uint32_t);
+    return (b + 15) & ~(size_t)15;
+}
+
+void hb_sort_init(hb_sort *s, uint32_t n, void *scratch)
+{
+    const uint32_t blocks = (n + kBlockKeys - 1) / kBlockKeys;
+    s->n = n;
+    s->src = 0;
+    s->key[0] = static_cast<uint64_t *>(scratch);
+    s->key[1] = s->key[0] + n;
+    s->idx[0] = reinterpret_cast<uint32_t *>(s->key[1] + n);
+    s->idx[1] = s->idx[0] + n;
+    s->counts = s->idx[1] + n;
+    s->totals = s->counts + (size_t)blocks * kDigits;
+}
+
+void hb_launch_sort(hb_sort *s, int bits, hipStream_t st)
+{
+    const uint32_t blocks = (s->n + kBlockKeys - 1) / kBlockKeys;
+    for (int shift = 0; shift < bits; shift += 8, s->src ^= 1) {
+        const int i = s->src, o = i ^ 1;
+        hipLaunchKernelGGL(sort_count_kernel, dim3(blocks), dim3(kThreads), 0, st, s->key[i], s->n,
+                           shift, s->counts);
+        hipLaunchKernelGGL(sort_scan_kernel, dim3(kDigits), dim3(kThreads), 0, st, s->counts,
+                           blocks, s->totals);
+        hipLaunchKernelGGL(sort_move_kernel, dim3(blocks), dim3(kThreads), 0, st, s->key[i],
+                           s->idx[i], s->n, shift, s->counts, s->totals, s->key[o], s->idx[o]);
+    }
 }
 
 hipError_t hb_launch_order(hb_order_args a, void *scratch, hipStream_t st)
 {
     if (a.n == 0) return hipSuccess;
-    const uint32_t blocks = (a.n + kBlockKeys - 1) / kBlockKeys, grid = (a.n + kThreads - 1) / kThreads;
-    a.key[0] = static_cast<uint64_t *>(scratch);
-    a.key[1] = a.key[0] + a.n;
-    a.idx[0] = reinterpret_cast<uint32_t *>(a.key[1] + a.n);
-    a.idx[1] = a.idx[0] + a.n;
-    uint32_t *counts = a.idx[1] + a.n, *totals = counts + (size_t)blocks * kDigits;
-    int src = 0;
-    auto sort = [&](int bits) {
-        for (int shift = 0; shift < bits; shift += 8, src ^= 1) {
-            hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(kThreads), 0, st, a.key[src],
-                               a.n, shift, counts);
-            hipLaunchKernelGGL(order_scan_kernel, dim3(kDigits), dim3(kThreads), 0, st, counts,
-                               blocks, totals);
-            hipLaunchKernelGGL(order_move_kernel, dim3(blocks), dim3(kThreads), 0, st, a.key[src],
-                               a.idx[src], a.n, shift, counts, totals, a.key[src ^ 1],
-                               a.idx[src ^ 1]);
-        }
-    };
+    const uint32_t grid = (a.n + kThreads - 1) / kThreads;
+    hb_sort_init(&a.sort, a.n, scratch);
     hipLaunchKernelGGL(order_lo_kernel, dim3(grid), dim3(kThreads), 0, st, a);
-    sort(a.s_bits + a.q_bits);
-    hipLaunchKernelGGL(order_hi_kernel, dim3(grid), dim3(kThreads), 0, st, a, src);
-    sort(a.query_bits + a.oid_bits);
-    hipLaunchKernelGGL(order_emit_kernel, dim3(grid), dim3(kThreads), 0, st, a, src);
+    hb_launch_sort(&a.sort, a.s_bits + a.q_bits, st);
+    hipLaunchKernelGGL(order_hi_kernel, dim3(grid), dim3(kThreads), 0, st, a);
+    hb_launch_sort(&a.sort, a.query_bits + a.oid_bits, st);
+    hipLaunchKernelGGL(order_emit_kernel, dim3(grid), dim3(kThreads), 0, st, a);
     return hipGetLastError();
 }

@@ -64,10 +64,13 @@ struct hb_db {
     uint4 *d_subj = nullptr;     // {oid, length, offset into d_scan_res} in processing order
     uint8_t *d_scan_res = nullptr;  // residues in processing order: the scan's copy (each
                                     // subject 16-byte aligned, spans padded to 16 bytes)
+    uint8_t *d_scan_alloc = nullptr;   // the allocation that holds it
     uint64_t scan_bytes = 0;        // bytes of that copy's subject spans
     uint32_t *d_tiles = nullptr;   // n_tiles + 1 boundaries (batched scans), then the
     uint32_t n_tiles = 0;          // n_qtiles + 1 of the plain scan's queue tiles
     uint32_t n_qtiles = 0;
+    void *load_scratch = nullptr;  // while it is loaded
+    size_t load_bytes = 0;
     std::vector<uint64_t> h_offs;
     uint64_t max_len = 0;   // longest subject
     float hdb_len_ms = 0.f, hdb_copy_ms = 0.f;   // hb_db_upload_hdb's kernels

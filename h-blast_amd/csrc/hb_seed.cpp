@@ -643,10 +643,14 @@ int hb_db_free(hb_db *db)
 {
     if (!db) return HB_ERR_ARG;
     hipSetDevice(db->ctx->device);
+    if (db->load_scratch) {   // loading failed: its work may be under way
+        hipStreamSynchronize(db->ctx->stream);
+        hb_pool_put(db->ctx, db->load_scratch, db->load_bytes);
+    }
     hipFree(db->d_res);
     hipFree(db->d_offs);
     hipFree(db->d_subj);
-    hipFree(db->d_scan_res);
+    hipFree(db->d_scan_alloc);
     hipFree(db->d_tiles);
     delete db;
     return HB_OK;
@@ -668,121 +672,134 @@ int hb_db_free(hb_db *db)
 // at one subject a tile made 200,000 subjects slower than 16K tiles did.
 static constexpr uint64_t kTileMax = 16384, kQueueTileMin = 256;
 
-// Processing order and tiles of a database whose host offsets are set, and
-// the device copies of offsets, per-subject records in processing order and
-// tiles.
+// The database's lengths, longest first, as runs of equal ones.
+static std::vector<std::pair<uint64_t, uint32_t>> length_runs(const hb_db *db)
+{
+    constexpr uint64_t kCounted = 1 << 16;   // longer subjects are few: sorted
+    std::vector<uint32_t> cnt(kCounted, 0);
+    std::vector<uint64_t> longer;
+    for (uint32_t i = 0; i < db->n; ++i) {
+        const uint64_t len = db->h_offs[i + 1] - db->h_offs[i];
+        if (len < kCounted) ++cnt[len];
+        else longer.push_back(len);
+    }
+    std::sort(longer.begin(), longer.end(), std::greater<uint64_t>());
+    std::vector<std::pair<uint64_t, uint32_t>> runs;
+    for (uint64_t len : longer) {
+        if (!runs.empty() && runs.back().first == len) ++runs.back().second;
+        else runs.emplace_back(len, 1u);
+    }
+    for (uint64_t len = kCounted; len-- > 0;)
+        if (cnt[len]) runs.emplace_back(len, cnt[len]);
+    return runs;
+}
+
+// Appends tile boundaries (0 first) of subjects with these lengths: a tile ends
+// at 64 subjects or at `want` residues (shrink: at a quarter of a wavefront's
+// share of the residues after the tile before, between want_min and kTileMax).
+static uint32_t cut_tiles(const std::vector<std::pair<uint64_t, uint32_t>> &runs, uint64_t total,
+                          uint64_t waves, bool shrink, uint64_t want_min,
+                          std::vector<uint32_t> *tiles)
+{
+    const size_t t0 = tiles->size();
+    tiles->push_back(0);
+    auto share = [&](uint64_t left) { return std::min(kTileMax, left / (4 * waves)); };
+    uint64_t acc = 0, left = total, w = share(left);
+    uint32_t at = 0, cnt = 0;
+    for (const auto &r : runs)
+        for (uint32_t m = r.second; m > 0;) {
+            uint64_t k = 64 - cnt;
+            if (r.first) k = std::min(k, w > acc ? (w - acc + r.first - 1) / r.first : 1);
+            else if (acc >= w) k = 1;
+            const uint32_t take = (uint32_t)std::min<uint64_t>(k, m);
+            m -= take;
+            at += take;
+            cnt += take;
+            acc += take * r.first;
+            left -= take * r.first;
+            if (cnt >= 64 || acc >= w) {
+                tiles->push_back(at);
+                acc = 0;
+                cnt = 0;
+                if (shrink) w = std::max(want_min, share(left));
+            }
+        }
+    if (tiles->back() != at) tiles->push_back(at);
+    return (uint32_t)(tiles->size() - t0) - 1;
+}
+
+// Tiles of a database whose host offsets are set, and the device copies of
+// offsets and tiles; then, enqueued on the context's stream, the records in
+// processing order (length-descending: the longest subjects start first).
+// The scan reads each subject's oid, length and offset from one 16-byte
+// record in processing order (sequential), not offs[oid] (one scattered
+// cache line per subject); the offset points into the scan's copy of the
+// residues, laid out in the same order, so consecutive subjects share no cache
+// line with subjects read at other times.
 static int db_meta(hb_db *db)
 {
+    hb_ctx *c = db->ctx;
     const uint32_t n = db->n;
-    // Length-descending processing order: the longest subjects start first.
-    // (stable LSD radix sort on the length, 11 bits a pass: a comparison
-    // sort reading scattered offsets took ~0.2 s for 2M subjects)
-    std::vector<uint32_t> order(n), tmp(n), key(n), key2(n);
-    uint32_t kmax = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        order[i] = i;
-        key[i] = (uint32_t)(db->h_offs[i + 1] - db->h_offs[i]);
-        kmax = std::max(kmax, key[i]);
-    }
-    db->max_len = kmax;
-    for (uint32_t i = 0; i < n; ++i) key[i] = kmax - key[i];   // ascending key = descending length
-    for (int shift = 0; shift < 32 && (kmax >> shift) != 0; shift += 11) {
-        uint32_t cnt[2049] = {0};
-        for (uint32_t i = 0; i < n; ++i) ++cnt[((key[i] >> shift) & 2047u) + 1];
-        for (int b = 0; b < 2048; ++b) cnt[b + 1] += cnt[b];
-        for (uint32_t i = 0; i < n; ++i) {
-            const uint32_t d = cnt[(key[i] >> shift) & 2047u]++;
-            tmp[d] = order[i];
-            key2[d] = key[i];
-        }
-        order.swap(tmp);
-        key.swap(key2);
-    }
-    // the scan reads each subject's oid, length and offset from one 16-byte
-    // record in processing order (sequential), not offs[oid] (one scattered
-    // cache line per subject); the offset points into the scan's copy of
-    // the residues, laid out in the same order, so consecutive subjects share
-    // no cache line with subjects read at other times
-    std::vector<uint4> subj(n);
-    std::vector<uint32_t> tiles(1, 0), qtiles(1, 0);
-    uint64_t acc = 0, qacc = 0, dst = 0, left = db->total;
-    uint32_t cnt = 0, qcnt = 0;
-    const uint64_t waves = db->ctx->n_cu * 16ull;
-    const uint64_t want = std::min(kTileMax, db->total / (4 * waves));
-    const uint64_t qmin = std::min(kQueueTileMin, db->total / (16 * waves));
-    uint64_t qwant = want;
-    for (uint32_t i = 0; i < n; ++i) {
-        const uint64_t len = db->h_offs[order[i] + 1] - db->h_offs[order[i]];
-        subj[i] = make_uint4(order[i], (uint32_t)len, (uint32_t)dst, (uint32_t)(dst >> 32));
-        dst += (len + 15) & ~15ull;   // the scan stages subjects with 16-byte loads
-        acc += len;
-        qacc += len;
-        left -= len;
-        ++cnt;
-        ++qcnt;
-        if (cnt >= 64 || acc >= want) {
-            tiles.push_back(i + 1);
-            acc = 0;
-            cnt = 0;
-        }
-        if (qcnt >= 64 || qacc >= qwant) {
-            qtiles.push_back(i + 1);
-            qacc = 0;
-            qcnt = 0;
-            qwant = std::min(kTileMax, std::max(qmin, left / (4 * waves)));
-        }
-    }
-    if (tiles.back() != n) tiles.push_back(n);
-    if (qtiles.back() != n) qtiles.push_back(n);
-    db->n_tiles = (uint32_t)tiles.size() - 1;
-    db->n_qtiles = (uint32_t)qtiles.size() - 1;
-    tiles.insert(tiles.end(), qtiles.begin(), qtiles.end());
-    db->scan_bytes = dst;
+    const auto runs = length_runs(db);
+    db->max_len = runs.empty() ? 0 : runs.front().first;
+    db->scan_bytes = 0;   // the scan stages subjects with 16-byte loads
+    for (const auto &r : runs) db->scan_bytes += ((r.first + 15) & ~15ull) * r.second;
+    const uint64_t waves = c->n_cu * 16ull;
+    const uint64_t want_min = std::min(kQueueTileMin, db->total / (16 * waves));
+    std::vector<uint32_t> tiles;
+    db->n_tiles = cut_tiles(runs, db->total, waves, false, 0, &tiles);
+    db->n_qtiles = cut_tiles(runs, db->total, waves, true, want_min, &tiles);
     if (hipMalloc(&db->d_offs, ((size_t)n + 1) * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc(&db->d_subj, (size_t)std::max<uint32_t>(n, 1) * sizeof(uint4)) != hipSuccess ||
         hipMalloc(&db->d_tiles, tiles.size() * sizeof(uint32_t)) != hipSuccess)
         return HB_ERR_NOMEM;
+    db->load_bytes = hb_load_scratch(n);
+    db->load_scratch = hb_pool_get(c, db->load_bytes);   // until the stream is waited for
+    if (!db->load_scratch) return HB_ERR_NOMEM;
+    hb_load_args a{};
+    a.offs = db->d_offs;
+    a.n = n;
+    a.max_len = db->max_len;
+    a.subj = db->d_subj;
     if (hipMemcpy(db->d_offs, db->h_offs.data(), ((size_t)n + 1) * sizeof(uint64_t),
                   hipMemcpyHostToDevice) != hipSuccess ||
-        (n && hipMemcpy(db->d_subj, subj.data(), (size_t)n * sizeof(uint4),
-                        hipMemcpyHostToDevice) != hipSuccess) ||
         hipMemcpy(db->d_tiles, tiles.data(), tiles.size() * sizeof(uint32_t),
-                  hipMemcpyHostToDevice) != hipSuccess)
+                  hipMemcpyHostToDevice) != hipSuccess ||
+        hb_launch_load_records(a, db->load_scratch, c->stream) != hipSuccess)
         return HB_ERR_DEVICE;
     return HB_OK;
 }
 
 // The scan's copy of the residues in processing order (after d_res holds
-// the database).
+// the database); HB_ERR_RESIDUE when one is not a residue code (< 28).
 static int db_scan_copy(hb_db *db)
 {
     hb_ctx *c = db->ctx;
-    // padding bytes between subject spans read as 0 (the staged copies hold
-    // them past each subject's end)
-    if (hipMalloc(&db->d_scan_res, db->scan_bytes + 64) != hipSuccess) return HB_ERR_NOMEM;
-    if (hipMemsetAsync(db->d_scan_res, 0, db->scan_bytes + 64, c->stream) != hipSuccess ||
-        hb_launch_gather_subjects(db->d_res, db->d_offs, db->d_subj, db->d_tiles, db->n_tiles,
-                                  db->d_scan_res, c->stream) != hipSuccess ||
+    // the flag, then the copy; padding bytes after subjects read as 0 (the
+    // staged copies hold them past each subject's end)
+    constexpr size_t kHead = 256;
+    uint8_t *d = nullptr;
+    if (hipMalloc(&d, kHead + db->scan_bytes + 64) != hipSuccess) return HB_ERR_NOMEM;
+    db->d_scan_alloc = d;
+    db->d_scan_res = d + kHead;
+    hb_load_args a{};
+    a.res = db->d_res;
+    a.offs = db->d_offs;
+    a.n = db->n;
+    a.subj = db->d_subj;
+    a.out = db->d_scan_res;
+    a.flag = reinterpret_cast<uint32_t *>(d);
+    uint32_t flag = 0;
+    if (hb_launch_fill_u32(a.flag, 0u, 1, c->stream) != hipSuccess ||
+        hb_launch_fill_u32(reinterpret_cast<uint32_t *>(db->d_scan_res + db->scan_bytes), 0u, 16,
+                           c->stream) != hipSuccess ||
+        hb_launch_load_copy(a, db->scan_bytes, c->stream) != hipSuccess ||
+        hipMemcpyAsync(&flag, a.flag, sizeof(flag), hipMemcpyDeviceToHost, c->stream) !=
+            hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return HB_ERR_DEVICE;
-    return HB_OK;
-}
-
-// Every residue code of the uploaded database is < 28.
-static int db_check_residues(hb_db *db)
-{
-    hb_ctx *c = db->ctx;
-    uint32_t *d_flag = nullptr;
-    if (hipMalloc(&d_flag, sizeof(uint32_t)) != hipSuccess) return HB_ERR_NOMEM;
-    uint32_t flag = 0;
-    const bool ok = hipMemsetAsync(d_flag, 0, sizeof(uint32_t), c->stream) == hipSuccess &&
-                    hb_launch_check_residues(db->d_res, db->total, d_flag, c->stream) ==
-                        hipSuccess &&
-                    hipMemcpyAsync(&flag, d_flag, sizeof(flag), hipMemcpyDeviceToHost,
-                                   c->stream) == hipSuccess &&
-                    hipStreamSynchronize(c->stream) == hipSuccess;
-    hipFree(d_flag);
-    if (!ok) return HB_ERR_DEVICE;
+    hb_pool_put(c, db->load_scratch, db->load_bytes);
+    db->load_scratch = nullptr;
     return flag ? HB_ERR_RESIDUE : HB_OK;
 }
 
@@ -811,11 +828,12 @@ int hb_db_upload(hb_ctx *c, const uint8_t *residues, const uint64_t *offsets, ui
         return r;
     };
     if (hipMalloc(&db->d_res, db->total + 64) != hipSuccess) return fail(HB_ERR_NOMEM);
-    if (hipMemcpy(db->d_res, residues + first, db->total, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(db->d_res + db->total, 0, 64) != hipSuccess)
-        return fail(HB_ERR_DEVICE);
+    // the records are made while the residues travel
     int rc = db_meta(db);
-    if (rc == HB_OK) rc = db_check_residues(db);
+    if (rc == HB_OK &&
+        (hipMemsetAsync(db->d_res + db->total, 0, 64, c->stream) != hipSuccess ||
+         hipMemcpy(db->d_res, residues + first, db->total, hipMemcpyHostToDevice) != hipSuccess))
+        rc = HB_ERR_DEVICE;
     if (rc == HB_OK) rc = db_scan_copy(db);
     if (rc != HB_OK) return fail(rc);
     *out = db;
@@ -1190,7 +1208,8 @@ static int launch_scan(hb_scan *s)
 // residues (0: bounded by file_bytes), loaded from a .hDb of file_bytes
 // (0: packed arrays), subjects up to max_len residues:
 //   upload:   the file, the residues, lengths (4 B), offsets (8 B) and
-//             processing-order records (16 B) per subject, tiles;
+//             processing-order records (16 B) and their sort (24 B) per
+//             subject, tiles;
 //   resident: the residues, their processing-order copy (spans padded to
 //             16 B) and the metadata;
 //   scan:     the HSP reservation (32 B records), counters (12 B per
@@ -1202,7 +1221,7 @@ static uint64_t scan_need_bytes(const hb_ctx *c, const hb_query *q, uint64_t fil
 {
     const uint64_t R = residues ? residues : file_bytes;
     const uint64_t meta = 8ull * (n + 1) + 16ull * n + 4ull * (n / 16 + std::min(n, 1u << 17) + 4);
-    const uint64_t upload = file_bytes + (R + 64) + 4ull * n + meta;
+    const uint64_t upload = file_bytes + (R + 64) + 4ull * n + hb_load_scratch(n) + meta;
     const uint64_t resident = (R + 64) + (R + 16ull * n + 64) + meta;
     const uint64_t cap = std::max<uint64_t>(1u << 18, n / 4);
     uint64_t scan = 32 * cap + 12ull * n + 64;
