@@ -580,18 +580,19 @@ __global__ __launch_bounds__(kGapWaves * HB_WAVE) void gapped_kernel(hb_gap_args
         W.order16 = L.order;
         W.saved = L.saved;
         W.sbuf = reinterpret_cast<uint8_t *>(L.subj);
-        // one subject per pop, subjects with the most HSPs first
+        // one subject per pop, subjects with the most HSPs first; a wavefront
+        // starts on an item of its own (8,192 pops of the counter that found an
+        // empty list took 90 us)
         const uint32_t n_list = (uint32_t)uniform((int32_t)*A.n_list);
-        for (;;) {
-            uint32_t item = 0;
-            if (lane == 0) item = atomicAdd(A.counter, 1u);
-            item = (uint32_t)lane_read((int32_t)item, 0);
-            if (item >= n_list) break;
+        uint32_t item = (uint32_t)uniform((int32_t)(blockIdx.x * kGapWaves + wave));
+        while (item < n_list) {
             const uint32_t k = (uint32_t)uniform((int32_t)A.list[item]);
             if (!W.subject(k) && lane == 0) {
                 const uint32_t p = atomicAdd(A.wide, 1u);
                 A.wide[1 + p] = k;
             }
+            if (lane == 0) item = gridDim.x * kGapWaves + atomicAdd(A.counter, 1u);
+            item = (uint32_t)lane_read((int32_t)item, 0);
         }
     } else {
         const size_t gw = (size_t)blockIdx.x * kGapWaves + wave;

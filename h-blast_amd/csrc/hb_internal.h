@@ -248,6 +248,7 @@ hipError_t hb_launch_order(hb_order_args a, void *scratch, hipStream_t st);
 #define HB_GAP_ORDER 256      // ungapped HSPs per subject ordered in LDS
 #define HB_GAP_SAVED 32       // saved gapped HSPs per subject kept in LDS
 #define HB_GAP_SUBJ 2048      // subjects up to this length are staged in LDS
+#define HB_GAP_PAIR_HSPS 128  // ungapped HSPs per subject in the pair kernel
 struct hb_gap_args {
     const uint8_t *res;            // database residues
     const uint64_t *offs;          // n + 1 subject offsets
@@ -273,6 +274,11 @@ struct hb_gap_args {
     uint32_t ring_wide;            // power of two > longest subject + 1
     uint32_t n_max;                // most ungapped HSPs of a wide subject
     uint32_t scratch_words;
+    // pair kernel: its queues' counters (HB_QUEUE_WORDS words, zero at launch),
+    // and [0] the count (zero at launch) of the subjects it leaves to the main
+    // pass, then those
+    uint32_t *queues;
+    uint32_t *mid;
 };
 // Work list of the main pass: list[] = subjects with HSPs ordered by
 // descending HSP count (capped at 63), *n_list their number; subjects without
@@ -280,6 +286,10 @@ struct hb_gap_args {
 hipError_t hb_launch_gap_list(const hb_gap_args &a, uint32_t *list, uint32_t *n_list,
                               uint32_t *scratch, hipStream_t st);
 hipError_t hb_launch_gapped(const hb_gap_args &a, bool wide, int n_blocks, hipStream_t st);
+// The pair kernel over the work list (hb_gap_pair.hip), with n_blocks a
+// multiple of HB_QUEUES, and the parameters that it takes.
+hipError_t hb_launch_gap_pair(const hb_gap_args &a, int n_blocks, hipStream_t st);
+bool hb_gap_pair_ok(int32_t gap_open, int32_t gap_extend, int32_t x_dropoff);
 // st3[3 * oid + 2] += 1 for each of the n records (st3 zeroed by the caller).
 hipError_t hb_launch_count_oids(const hb_hsp *rec, uint32_t n, uint32_t *st3, hipStream_t st);
 // Dense layout: stats[k] and out_dense from the sparse output and first[].

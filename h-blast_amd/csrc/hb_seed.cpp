@@ -1727,6 +1727,10 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
     auto *d_gst = static_cast<hb_gapped_stats *>(get((size_t)ns * sizeof(hb_gapped_stats)));
     auto *d_gdense = static_cast<hb_gapped_hsp *>(get(nr * sizeof(hb_gapped_hsp)));
     auto *d_list = static_cast<uint32_t *>(get(((size_t)ns + 129) * sizeof(uint32_t)));
+    // the pair kernel's queues and the subjects that it leaves
+    const bool pair = hb_gap_pair_ok(gp->gap_open, gp->gap_extend, gp->x_dropoff);
+    auto *d_mid = static_cast<uint32_t *>(
+        get(pair ? (HB_QUEUE_WORDS + 1 + (size_t)ns) * sizeof(uint32_t) : 0));
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     auto release = [&]() {
         for (auto &h : held) hb_pool_put(c, h.first, h.second);
@@ -1774,8 +1778,17 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
                            hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hb_launch_fill_u32(d_misc, 0u, 2, st);
     if (e == hipSuccess) e = hb_launch_gap_list(a, d_list + 129, d_list + 128, d_list, st);
+    if (e == hipSuccess && pair) e = hb_launch_fill_u32(d_mid, 0u, HB_QUEUE_WORDS + 1, st);
     for (int i = 0; e == hipSuccess && i < 4; ++i) e = hipEventCreate(&ev[i]);
     if (e == hipSuccess) e = hipEventRecord(ev[0], st);
+    if (pair) {
+        a.queues = d_mid;
+        a.mid = d_mid + HB_QUEUE_WORDS;
+        if (e == hipSuccess)
+            e = hb_launch_gap_pair(a, (c->n_cu * 8 + HB_QUEUES - 1) / HB_QUEUES * HB_QUEUES, st);
+        a.list = a.mid + 1;
+        a.n_list = a.mid;
+    }
     if (e == hipSuccess) e = hb_launch_gapped(a, false, c->n_cu * 8, st);
     if (e == hipSuccess) e = hipEventRecord(ev[1], st);
     if (e == hipSuccess) e = hipMemcpyAsync(&n_wide, d_misc + 1, sizeof(n_wide),
