@@ -39,6 +39,7 @@ struct hb_ctx {
     size_t pinned_bytes = 0;
     // small page-locked buffers for uploads and read-backs (kept, bounded)
     std::vector<std::pair<void *, size_t>> pins;
+    hipStream_t up_stream = nullptr;   // copies to the device that overlap the stream's work
     // device address of this GPU's hb_scan_noalloc scratch
     unsigned char *scratch_dev = nullptr;
 };
@@ -52,8 +53,11 @@ int hb_copy_out(hb_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t
 void *hb_pin_get(hb_ctx *c, size_t *bytes);
 void hb_pin_put(hb_ctx *c, void *p, size_t bytes);
 
+// Buffers of the pool; one that nothing on the device uses any more goes back
+// to it.  hb_pool_held: the bytes that it keeps.
 void *hb_pool_get(hb_ctx *c, size_t bytes);
 void hb_pool_put(hb_ctx *c, void *p, size_t bytes);
+size_t hb_pool_held(hb_ctx *c);
 
 struct hb_db {
     hb_ctx *ctx = nullptr;
@@ -71,6 +75,8 @@ struct hb_db {
     uint32_t n_qtiles = 0;
     void *load_scratch = nullptr;  // while it is loaded
     size_t load_bytes = 0;
+    // sizes of the allocations (from the context's pool)
+    size_t res_bytes = 0, offs_bytes = 0, subj_bytes = 0, alloc_bytes = 0, tiles_bytes = 0;
     std::vector<uint64_t> h_offs;
     uint64_t max_len = 0;   // longest subject
     float hdb_len_ms = 0.f, hdb_copy_ms = 0.f;   // hb_db_upload_hdb's kernels
