@@ -366,7 +366,9 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                     const int32_t lo = max(0, min(so - HB_GAP_SUBJ / 2, slen - HB_GAP_SUBJ));
                     stage(lo, lo + HB_GAP_SUBJ);
                 }
-                // both sides' DP: row 0 holds the leading gaps within the drop-off
+                // both sides' DP: row 0 holds the leading gaps within the drop-off.
+                // The sequential DP has no column right of them in row 1 for the
+                // last one's diagonal, so that one's score is not kept.
                 ql = qo + 1;
                 M = rev ? ql : clen - ql;
                 N = rev ? so + 1 : slen - (so + 1);
@@ -381,7 +383,7 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                     const int32_t b = colb + j;
                     const bool in0 = some && b >= 0 && b <= Ns && (b == 0 || goe + (b - 1) * ge <= X);
                     const int32_t v = kBias - (b ? go + b * ge : 0);
-                    ob[j] = in0 ? v : kDead;
+                    ob[j] = in0 && goe + b * ge <= X ? v : kDead;
                     ov[j] = in0 ? v - go : kDead;
                     ob2[j] = ov2[j] = kDead;
                 }

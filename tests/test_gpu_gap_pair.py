@@ -72,6 +72,28 @@ def test_subjects_around_the_staged_length(ctx, slen):  # noqa: F811
     assert len(g)
 
 
+@pytest.mark.parametrize("mirrored", [False, True])
+def test_leading_gaps_of_the_drop_off(ctx, mirrored):  # noqa: F811
+    """A short piece of the query next to a copy of it 20 to 32 diagonals away:
+    the extension of the piece starts with a gap that costs about the drop-off
+    (27 residues: all of it)."""
+    q = hbseed.random_protein(1260, 90)
+    parts = []
+    for d in range(20, 33):
+        for m in range(4, 10):
+            for i in range(0, 40, 3):
+                j = max(0, i + m - d)
+                gap = j + d - i - m
+                parts.append(np.concatenate([hbseed.random_protein(4 * i + m, 4), q[i:i + m],
+                                             hbseed.random_protein(100 * d + i, gap), q[j:]]))
+    if mirrored:
+        q = q[::-1].copy()
+        parts = [p[::-1].copy() for p in parts]
+    res, offs = pack(parts)
+    _, g, _, _ = run_both(ctx, hbseed.blastp_query(q), res, offs, [20])
+    assert len(g) > len(parts)
+
+
 @pytest.mark.parametrize("n", [32, 33, 64, 128, 129, 300])
 def test_many_hsps_and_many_saved(ctx, n):  # noqa: F811
     q = hbseed.random_protein(1300, 300)
