@@ -623,23 +623,28 @@ __global__ __launch_bounds__(256) void gap_count_kernel(hb_gap_args A, uint32_t 
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < A.n_subjects) {
         const uint32_t n = A.ust[k].n_hsp;
-        if (n == 0) {
-            A.st3[3 * (size_t)k] = 0;
-            A.st3[3 * (size_t)k + 1] = 0;
-            A.st3[3 * (size_t)k + 2] = 0;
-        } else {
-            atomicAdd(&h[gap_bucket_of(n)], 1u);
-        }
+        // (also what a subject left to the wide pass counts until then)
+        A.st3[3 * (size_t)k] = 0;
+        A.st3[3 * (size_t)k + 1] = 0;
+        A.st3[3 * (size_t)k + 2] = 0;
+        if (n) atomicAdd(&h[gap_bucket_of(n)], 1u);
     }
     __syncthreads();
     if (threadIdx.x < 64 && h[threadIdx.x]) atomicAdd(&bucket[threadIdx.x], h[threadIdx.x]);
 }
 
 // One wavefront: exclusive prefix of the 64 bucket counts into the cursors
-// (bucket[64 ..]) and the total.
-__global__ void gap_bucket_kernel(uint32_t *bucket, uint32_t *n_list)
+// (bucket[64 ..]) and the total, and the next kernels' counters.
+__global__ void gap_bucket_kernel(hb_gap_args A, uint32_t *bucket, uint32_t *n_list)
 {
     const uint32_t lane = threadIdx.x;
+    if (A.queues)
+        for (uint32_t i = lane; i < HB_QUEUE_WORDS; i += 64) A.queues[i] = 0;
+    if (lane == 0) {
+        *A.counter = 0;
+        A.wide[0] = 0;
+        if (A.mid) A.mid[0] = 0;
+    }
     const uint32_t v = bucket[lane];
     uint32_t incl = v;
     for (uint32_t d = 1; d < 64; d <<= 1) {
@@ -681,10 +686,11 @@ __global__ void count_oids_kernel(const hb_hsp *rec, uint32_t n, uint32_t *st3)
 }
 
 // One thread per subject: dense layout of the gapped HSPs and the stats.
-__global__ void gap_compact_kernel(hb_gap_args A, const uint32_t *first, hb_gapped_stats *stats,
-                                   hb_gapped_hsp *dense)
+__global__ void gap_compact_kernel(hb_gap_args A, const uint32_t *first, const uint32_t *total,
+                                   hb_gapped_stats *stats, hb_gapped_hsp *dense, uint2 *small)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k == 0) *small = make_uint2(*total, A.wide[0]);
     if (k >= A.n_subjects) return;
     const uint32_t n = A.st3[3 * (size_t)k + 2];
     hb_gapped_stats o;
@@ -703,11 +709,10 @@ __global__ void gap_compact_kernel(hb_gap_args A, const uint32_t *first, hb_gapp
 hipError_t hb_launch_gap_list(const hb_gap_args &a, uint32_t *list, uint32_t *n_list,
                               uint32_t *scratch, hipStream_t st)
 {
-    hipError_t e = hb_launch_fill_u32(scratch, 0u, 128, st);
-    if (e != hipSuccess || a.n_subjects == 0) return e;
+    if (a.n_subjects == 0) return hipSuccess;
     const dim3 grid((a.n_subjects + 255) / 256);
     hipLaunchKernelGGL(gap_count_kernel, grid, dim3(256), 0, st, a, scratch);
-    hipLaunchKernelGGL(gap_bucket_kernel, dim3(1), dim3(64), 0, st, scratch, n_list);
+    hipLaunchKernelGGL(gap_bucket_kernel, dim3(1), dim3(64), 0, st, a, scratch, n_list);
     hipLaunchKernelGGL(gap_place_kernel, grid, dim3(256), 0, st, a, scratch, list);
     return hipGetLastError();
 }
@@ -731,12 +736,12 @@ hipError_t hb_launch_gapped(const hb_gap_args &a, bool wide, int n_blocks, hipSt
     return hipGetLastError();
 }
 
-hipError_t hb_launch_gap_compact(const hb_gap_args &a, const uint32_t *first,
+hipError_t hb_launch_gap_compact(const hb_gap_args &a, const uint32_t *first, const uint32_t *total,
                                  hb_gapped_stats *stats, hb_gapped_hsp *out_dense,
-                                 hipStream_t st)
+                                 uint2 *small, hipStream_t st)
 {
     if (a.n_subjects == 0) return hipSuccess;
     hipLaunchKernelGGL(gap_compact_kernel, dim3((a.n_subjects + 255) / 256), dim3(256), 0, st, a,
-                       first, stats, out_dense);
+                       first, total, stats, out_dense, small);
     return hipGetLastError();
 }

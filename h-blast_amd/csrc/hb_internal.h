@@ -169,23 +169,29 @@ struct hb_fin_big {
     uint32_t oid, n;
     uint64_t first;
 };
-// scratch: ns + ns / 4096 + 1 uint32
+// scratch: ns + ns / 4096 + 1 uint32.  Clears n_big[0 .. n_zero - 1] (n_zero >=
+// 1) before anything is listed.
 hipError_t hb_launch_finalize(const uint32_t *st3, uint32_t ns, const hb_hsp *recs, uint32_t n,
                               hb_subject_stats *stats_out, hb_hsp *recs_out, uint32_t *scratch,
-                              hb_fin_big *big, uint32_t big_cap, uint32_t *n_big, hipStream_t st);
+                              hb_fin_big *big, uint32_t big_cap, uint32_t *n_big, uint32_t n_zero,
+                              hipStream_t st);
 // The compact layout: entries of the subjects with HSPs in oid order
-// (subj_out, at most min(ns, n)), the records grouped and ordered as above,
-// tot[0..1] += the lookup hits and extensions of all subjects (tot cleared
-// by the caller).  With nb = (ns + 4095) / 4096, scratch holds 2 nb + 1 + ns
-// uint32, and the number of subjects with HSPs ends up in scratch[2 nb].
+// (subj_out, at most min(ns, n)), the records grouped and ordered as above, and
+// the totals in *small.  With nb = (ns + 4095) / 4096, scratch holds 2 nb + ns
+// uint32 and tot 2 nb 64-bit words.
+struct hb_fin_small {
+    unsigned long long lookup_hits, extensions;
+    uint32_t n_subj, n_big;   // subjects with HSPs; subjects listed in big[]
+};
 hipError_t hb_launch_finalize_compact(const uint32_t *st3, uint32_t ns, const hb_hsp *recs,
                                       uint32_t n, hb_subject_hits *subj_out, hb_hsp *recs_out,
                                       uint32_t *scratch, unsigned long long *tot, hb_fin_big *big,
-                                      uint32_t big_cap, uint32_t *n_big, hipStream_t st);
+                                      uint32_t big_cap, hb_fin_small *small, hipStream_t st);
 // First-record indices of per-subject counts st3[3i + 2] (hb_kernels.hip):
-// first[i] = sum of the counts of subjects < i.  scratch: ns / 4096 + 1.
+// first[i] = sum of the counts of subjects < i, *total the sum of all.
+// scratch: ns / 4096 + 1.
 hipError_t hb_launch_first_index(const uint32_t *st3, uint32_t ns, uint32_t *first,
-                                 uint32_t *scratch, hipStream_t st);
+                                 uint32_t *scratch, uint32_t *total, hipStream_t st);
 
 // Stable LSD radix sort of n 64-bit keys with their indices (hb_order.hip),
 // 8 bits a pass over the lowest `bits` bits; the result is in key[src], idx[src].
@@ -274,15 +280,17 @@ struct hb_gap_args {
     uint32_t ring_wide;            // power of two > longest subject + 1
     uint32_t n_max;                // most ungapped HSPs of a wide subject
     uint32_t scratch_words;
-    // pair kernel: its queues' counters (HB_QUEUE_WORDS words, zero at launch),
-    // and [0] the count (zero at launch) of the subjects it leaves to the main
-    // pass, then those
+    // pair kernel (or null): its queues' counters (HB_QUEUE_WORDS words, zero at
+    // launch), and [0] the count (zero at launch) of the subjects it leaves to
+    // the main pass, then those
     uint32_t *queues;
     uint32_t *mid;
 };
 // Work list of the main pass: list[] = subjects with HSPs ordered by
 // descending HSP count (capped at 63), *n_list their number; subjects without
-// HSPs get zero stats.  scratch: 128 uint32 (zeroed here).
+// HSPs get zero stats.  scratch: 128 uint32 (zero).  Also clears the counters of
+// the passes that follow: *counter, wide[0] and, where they are set, the queues
+// and mid[0].
 hipError_t hb_launch_gap_list(const hb_gap_args &a, uint32_t *list, uint32_t *n_list,
                               uint32_t *scratch, hipStream_t st);
 hipError_t hb_launch_gapped(const hb_gap_args &a, bool wide, int n_blocks, hipStream_t st);
@@ -292,10 +300,11 @@ hipError_t hb_launch_gap_pair(const hb_gap_args &a, int n_blocks, hipStream_t st
 bool hb_gap_pair_ok(int32_t gap_open, int32_t gap_extend, int32_t x_dropoff);
 // st3[3 * oid + 2] += 1 for each of the n records (st3 zeroed by the caller).
 hipError_t hb_launch_count_oids(const hb_hsp *rec, uint32_t n, uint32_t *st3, hipStream_t st);
-// Dense layout: stats[k] and out_dense from the sparse output and first[].
-hipError_t hb_launch_gap_compact(const hb_gap_args &a, const uint32_t *first,
+// Dense layout: stats[k] and out_dense from the sparse output and first[];
+// small = {*total, wide[0]}.
+hipError_t hb_launch_gap_compact(const hb_gap_args &a, const uint32_t *first, const uint32_t *total,
                                  hb_gapped_stats *stats, hb_gapped_hsp *out_dense,
-                                 hipStream_t st);
+                                 uint2 *small, hipStream_t st);
 
 // Unpacking of a .hDb volume on the device (hb_hdb.hip).  Sequence c sits
 // in block B = c / threadsx (global over the volume), group g = B / blocksx;

@@ -34,10 +34,11 @@ struct hb_ctx {
     std::vector<std::pair<void *, size_t>> pool;
     size_t pool_bytes = 0;
     // pinned host staging for result copies (grown on demand, kept)
-    std::mutex pin_mu;
+    std::mutex pinned_mu;
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
     // small page-locked buffers for uploads and read-backs (kept, bounded)
+    std::mutex pin_mu;
     std::vector<std::pair<void *, size_t>> pins;
     hipStream_t up_stream = nullptr;   // copies to the device that overlap the stream's work
     // device address of this GPU's hb_scan_noalloc scratch

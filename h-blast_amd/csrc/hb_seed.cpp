@@ -236,35 +236,83 @@ class Upload {
 };
 }  // namespace
 
-int hb_copy_out(hb_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t st)
+// Copies between host buffers, 1 MiB or more a thread: a search with 4.8 MB of
+// counters and a gapped stage with 8 MB took 1,159 and 1,520 us with one thread,
+// 1,090 and 1,468 with two, 1,089 and 1,437 with four, and the same with eight.
+static void host_copy(void *dst, const void *src, size_t bytes)
 {
-    if (bytes == 0) return HB_OK;
-    std::lock_guard<std::mutex> lk(c->pin_mu);
-    if (c->pinned_bytes < bytes) {
+    constexpr size_t kPart = (size_t)1 << 20;
+    const size_t nt = std::min<size_t>(4, std::max<size_t>(1, bytes / kPart));
+    const size_t per = (bytes + nt - 1) / nt;
+    auto part = [&](size_t t) {
+        const size_t b = t * per, e = std::min(bytes, b + per);
+        if (b < e) memcpy(static_cast<char *>(dst) + b, static_cast<const char *>(src) + b, e - b);
+    };
+    std::vector<std::thread> th;
+    size_t t = 1;
+    try {
+        th.reserve(nt);
+        for (; t < nt; ++t) th.emplace_back(part, t);
+    } catch (...) {   // the rest is done here
+    }
+    part(0);
+    for (; t < nt; ++t) part(t);
+    for (auto &x : th) x.join();
+}
+
+// Copies of device memory to pageable host memory through the context's pinned
+// buffer (held while this lives, and of at least kKeep and room(bytes)): add()
+// enqueues one, wait() waits for all, store() moves one on.
+namespace {
+class CopyOut {
+  public:
+    CopyOut(hb_ctx *c, size_t bytes, hipStream_t st) : c_(c), st_(st), lk_(c->pinned_mu)
+    {
+        bytes = std::max(room(bytes), kKeep);
+        if (c->pinned_bytes >= bytes) return;
         if (c->pinned) hipHostFree(c->pinned);
         c->pinned = nullptr;
         c->pinned_bytes = 0;
-        const size_t want = std::max(bytes, (size_t)64 << 20);
-        HB_CHECK(hipHostMalloc(&c->pinned, want, hipHostMallocDefault));
-        c->pinned_bytes = want;
+        e_ = hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault);
+        if (e_ == hipSuccess) c->pinned_bytes = bytes;
+        else c->pinned = nullptr;
     }
-    HB_CHECK(hipMemcpyAsync(c->pinned, src, bytes, hipMemcpyDeviceToHost, st));
-    HB_CHECK(hipStreamSynchronize(st));
-    const unsigned nt = bytes < ((size_t)4 << 20)
-                            ? 1u
-                            : std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-    const size_t per = (bytes + nt - 1) / nt;
-    auto part = [&](unsigned t) {
-        const size_t b = (size_t)t * per, e = std::min(bytes, b + per);
-        if (b < e) memcpy(static_cast<char *>(dst) + b, static_cast<const char *>(c->pinned) + b, e - b);
-    };
-    if (nt == 1) {
-        part(0);
-    } else {
-        std::vector<std::thread> th;
-        for (unsigned t = 0; t < nt; ++t) th.emplace_back(part, t);
-        for (auto &x : th) x.join();
+    static constexpr size_t kKeep = (size_t)64 << 20;
+    static size_t room(size_t bytes) { return (bytes + 63) & ~(size_t)63; }
+    size_t add(const void *src, size_t bytes)
+    {
+        const size_t at = at_;
+        at_ += room(bytes);
+        if (e_ == hipSuccess && at_ > c_->pinned_bytes) e_ = hipErrorInvalidValue;
+        if (e_ == hipSuccess && bytes)
+            e_ = hipMemcpyAsync(ptr(at), src, bytes, hipMemcpyDeviceToHost, st_);
+        return at;
     }
+    void rewind() { at_ = 0; }   // after a wait: what was copied is no longer needed
+    hipError_t wait()
+    {
+        if (e_ == hipSuccess) e_ = hipStreamSynchronize(st_);
+        return e_;
+    }
+    char *ptr(size_t at) const { return static_cast<char *>(c_->pinned) + at; }
+    void store(void *dst, size_t at, size_t bytes) const { host_copy(dst, ptr(at), bytes); }
+
+  private:
+    hb_ctx *c_;
+    hipStream_t st_;
+    std::unique_lock<std::mutex> lk_;
+    hipError_t e_ = hipSuccess;
+    size_t at_ = 0;
+};
+}  // namespace
+
+int hb_copy_out(hb_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    if (bytes == 0) return HB_OK;
+    CopyOut out(c, bytes, st);
+    out.add(src, bytes);
+    HB_CHECK(out.wait());
+    out.store(dst, 0, bytes);
     return HB_OK;
 }
 
@@ -514,6 +562,10 @@ int hb_scan_config(hb_ctx *c, bool multi, bool split, int32_t qlen_pad_max, int3
         for (int32_t ring = ring_top; ring >= 256; ring -= 64) {
             const size_t lds = fixed + waves * hb_scan_wave_lds(diag_len_max, ring, sb);
             if (lds > c->max_lds) continue;
+            // no better than the best so far, as many as its LDS would let in (up
+            // to 180 questions to the runtime for each scan otherwise)
+            const int most = (int)std::min<size_t>(c->max_lds / lds * waves, 16);
+            if (most < best_wpc || (most == best_wpc && ring <= cfg->ring)) continue;
             int per_cu = 0;
             HB_CHECK(hb_scan_occupancy(multi, gstate, split, lds, waves * HB_WAVE, &per_cu));
             const int wpc = std::min(per_cu * waves, 16);
@@ -1673,17 +1725,28 @@ int hb_scan_results(hb_scan *s, hb_subject_stats *stats, hb_hsp *hsps, uint64_t 
     uint32_t *d_nbig = d_scr + ns + nb;
     hipStream_t st = c->stream;
     uint32_t nbig = 0;
-    hipError_t e = hb_launch_fill_u32(d_nbig, 0u, 1, st);
-    if (e == hipSuccess)
-        e = hb_launch_finalize(s->d_stats, ns, s->d_out, (uint32_t)n, d_st, d_rec, d_scr, d_big,
-                               kBig, d_nbig, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(&nbig, d_nbig, sizeof(nbig), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess && stats && hb_copy_out(c, stats, d_st, b_st, st) != HB_OK)
-        e = hipErrorUnknown;
-    if (e == hipSuccess && hsps && n &&
-        hb_copy_out(c, hsps, d_rec, (size_t)n * sizeof(hb_hsp), st) != HB_OK)
-        e = hipErrorUnknown;
+    hipError_t e = hb_launch_finalize(s->d_stats, ns, s->d_out, (uint32_t)n, d_st, d_rec, d_scr, d_big,
+                                      kBig, d_nbig, 1, st);
+    if (e == hipSuccess) {
+        // all of it behind the kernels and one wait, unless the buffer would grow
+        // for that
+        const size_t w_st = stats ? b_st : 0, w_rec = hsps ? (size_t)n * sizeof(hb_hsp) : 0;
+        const bool at_once = 64 + CopyOut::room(w_st) + CopyOut::room(w_rec) <= CopyOut::kKeep;
+        CopyOut out(c, 64 + CopyOut::room(std::max(w_st, w_rec)), st);
+        const size_t o_big = out.add(d_nbig, sizeof(nbig)), o_st = out.add(d_st, w_st);
+        size_t o_rec = at_once ? out.add(d_rec, w_rec) : 0;
+        e = out.wait();
+        if (e == hipSuccess) {
+            memcpy(&nbig, out.ptr(o_big), sizeof(nbig));
+            if (w_st) out.store(stats, o_st, w_st);
+            if (!at_once && w_rec) {
+                out.rewind();
+                o_rec = out.add(d_rec, w_rec);
+                e = out.wait();
+            }
+            if (e == hipSuccess && w_rec) out.store(hsps, o_rec, w_rec);
+        }
+    }
     // subjects with many records are ordered here
     std::vector<hb_fin_big> big;
     if (e == hipSuccess && hsps && nbig) {
@@ -1736,14 +1799,14 @@ int hb_scan_results_compact(hb_scan *s, hb_subject_hits *subj, uint64_t subj_cap
     const uint64_t max_subj = std::min<uint64_t>(ns, n);
     const size_t b_sub = (size_t)std::max<uint64_t>(max_subj, 1) * sizeof(hb_subject_hits);
     const size_t b_rec = (size_t)std::max<uint64_t>(n, 1) * sizeof(hb_hsp);
-    const size_t b_scr = (2 * (size_t)nb + 1 + ns) * sizeof(uint32_t);
+    const size_t b_scr = (2 * (size_t)nb + ns) * sizeof(uint32_t);
     const size_t b_big = kBig * sizeof(hb_fin_big);
-    const size_t b_small = 32;   // two 64-bit totals, the big-subject count
+    const size_t b_small = 64 + 2 * (size_t)nb * sizeof(unsigned long long);   // totals, blocks' sums
     auto *d_sub = static_cast<hb_subject_hits *>(hb_pool_get(c, b_sub));
     auto *d_rec = static_cast<hb_hsp *>(hb_pool_get(c, b_rec));
     auto *d_scr = static_cast<uint32_t *>(hb_pool_get(c, b_scr));
     auto *d_big = static_cast<hb_fin_big *>(hb_pool_get(c, b_big));
-    auto *d_small = static_cast<unsigned long long *>(hb_pool_get(c, b_small));
+    auto *d_small = static_cast<hb_fin_small *>(hb_pool_get(c, b_small));
     auto release = [&]() {
         hb_pool_put(c, d_sub, b_sub);
         hb_pool_put(c, d_rec, b_rec);
@@ -1755,38 +1818,56 @@ int hb_scan_results_compact(hb_scan *s, hb_subject_hits *subj, uint64_t subj_cap
         release();
         return HB_ERR_NOMEM;
     }
-    uint32_t *d_nbig = reinterpret_cast<uint32_t *>(d_small + 2);
     hipStream_t st = c->stream;
-    unsigned long long small[3] = {0, 0, 0};
-    uint32_t n_subj = 0;
-    hipError_t e = hb_launch_fill_u32(reinterpret_cast<uint32_t *>(d_small), 0u, 6, st);
-    if (e == hipSuccess)
-        e = hb_launch_finalize_compact(s->d_stats, ns, s->d_out, (uint32_t)n, d_sub, d_rec, d_scr,
-                                       d_small, d_big, kBig, d_nbig, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(small, d_small, sizeof(small), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(&n_subj, d_scr + 2 * nb, sizeof(n_subj), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    const uint32_t nbig = (uint32_t)small[2];
-    if (e == hipSuccess) {
-        totals->lookup_hits = small[0];
-        totals->extensions = small[1];
-        totals->n_subjects = n_subj;
-        if ((subj && subj_cap < n_subj) || (hsps && hsp_cap < n)) {
-            release();
-            return HB_ERR_CAPACITY;
-        }
-    }
+    hb_fin_small small{};
+    hipError_t e = hb_launch_finalize_compact(
+        s->d_stats, ns, s->d_out, (uint32_t)n, d_sub, d_rec, d_scr,
+        reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(d_small) + 64), d_big, kBig,
+        d_small, st);
     std::vector<hb_subject_hits> host_sub;
     hb_subject_hits *sp = subj;
-    if (e == hipSuccess && !sp && hsps && nbig > kBig) {   // the host needs the entries below
-        host_sub.resize(n_subj);
-        sp = host_sub.data();
+    uint32_t nbig = 0;
+    bool done = false;   // the results are copied
+    if (e == hipSuccess) {
+        // The records' number is known and bounds that of the entries: up to
+        // kAtOnce of both are copied behind the kernels with one wait (the
+        // entries too many cost less than another wait); else when the totals
+        // are known.
+        constexpr size_t kAtOnce = (size_t)32 << 20;
+        const size_t w_sub = subj ? (size_t)max_subj * sizeof(hb_subject_hits) : 0;
+        const size_t w_rec = hsps ? (size_t)n * sizeof(hb_hsp) : 0;
+        const bool at_once = w_sub + w_rec <= kAtOnce;
+        CopyOut out(c, 0, st);
+        const size_t o_small = out.add(d_small, sizeof(small));
+        const size_t o_sub = at_once ? out.add(d_sub, w_sub) : 0;
+        const size_t o_rec = at_once ? out.add(d_rec, w_rec) : 0;
+        e = out.wait();
+        if (e == hipSuccess) {
+            memcpy(&small, out.ptr(o_small), sizeof(small));
+            nbig = small.n_big;
+            totals->lookup_hits = small.lookup_hits;
+            totals->extensions = small.extensions;
+            totals->n_subjects = small.n_subj;
+            if ((subj && subj_cap < small.n_subj) || (hsps && hsp_cap < n)) {
+                release();
+                return HB_ERR_CAPACITY;
+            }
+            if (at_once) {
+                if (w_sub) out.store(subj, o_sub, (size_t)small.n_subj * sizeof(hb_subject_hits));
+                if (w_rec) out.store(hsps, o_rec, w_rec);
+            }
+        }
+        if (e == hipSuccess && !sp && hsps && nbig > kBig) {   // the host needs the entries below
+            host_sub.resize(small.n_subj);
+            sp = host_sub.data();
+        }
+        done = at_once;
     }
-    if (e == hipSuccess && sp && n_subj &&
+    const uint32_t n_subj = small.n_subj;
+    if (e == hipSuccess && sp && n_subj && !(done && sp == subj) &&
         hb_copy_out(c, sp, d_sub, (size_t)n_subj * sizeof(hb_subject_hits), st) != HB_OK)
         e = hipErrorUnknown;
-    if (e == hipSuccess && hsps && n &&
+    if (e == hipSuccess && hsps && n && !done &&
         hb_copy_out(c, hsps, d_rec, (size_t)n * sizeof(hb_hsp), st) != HB_OK)
         e = hipErrorUnknown;
     // subjects with many records are ordered here
@@ -1858,16 +1939,19 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
     const uint64_t nr = std::max<uint64_t>(n, 1);
     auto *d_ust = static_cast<hb_subject_stats *>(get((size_t)ns * sizeof(hb_subject_stats)));
     auto *d_urec = static_cast<hb_hsp *>(get(nr * sizeof(hb_hsp)));
-    auto *d_scr = static_cast<uint32_t *>(get(((size_t)ns + nb + 1) * sizeof(uint32_t)));
+    // (layout's scratch; its big-subject count; the list's 128 buckets, cleared
+    // with that count)
+    auto *d_scr = static_cast<uint32_t *>(get(((size_t)ns + nb + 1 + 128) * sizeof(uint32_t)));
     auto *d_big = static_cast<hb_fin_big *>(get(kBig * sizeof(hb_fin_big)));
     auto *d_st3 = static_cast<uint32_t *>(get((size_t)ns * 3 * sizeof(uint32_t)));
     auto *d_gout = static_cast<hb_gapped_hsp *>(get(nr * sizeof(hb_gapped_hsp)));
     auto *d_misc = static_cast<uint32_t *>(get(((size_t)ns + 2) * sizeof(uint32_t)));
     auto *d_ctx = static_cast<int32_t *>(get((size_t)3 * n_ctx * sizeof(int32_t)));
-    auto *d_first = static_cast<uint32_t *>(get(((size_t)ns + nb + 1) * sizeof(uint32_t)));
+    auto *d_first = static_cast<uint32_t *>(get(((size_t)ns + nb + 4) * sizeof(uint32_t)));
     auto *d_gst = static_cast<hb_gapped_stats *>(get((size_t)ns * sizeof(hb_gapped_stats)));
     auto *d_gdense = static_cast<hb_gapped_hsp *>(get(nr * sizeof(hb_gapped_hsp)));
-    auto *d_list = static_cast<uint32_t *>(get(((size_t)ns + 129) * sizeof(uint32_t)));
+    auto *d_list = static_cast<uint32_t *>(get(((size_t)ns + 1) * sizeof(uint32_t)));
+    auto *d_small = static_cast<uint2 *>(get(sizeof(uint2)));
     // the pair kernel's queues and the subjects that it leaves
     const bool pair = hb_gap_pair_ok(gp->gap_open, gp->gap_extend, gp->x_dropoff);
     auto *d_mid = static_cast<uint32_t *>(
@@ -1906,35 +1990,56 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
     a.out = d_gout;
     a.st3 = d_st3;
     a.wide = d_misc + 1;
-    a.list = d_list + 129;
-    a.n_list = d_list + 128;
-    uint32_t n_wide = 0;
-    uint32_t *d_nbig = d_scr + ns + nb;
-    hipError_t e = hb_launch_fill_u32(d_nbig, 0u, 1, st);
-    if (e == hipSuccess)
-        e = hb_launch_finalize(st3_in, ns, rec_in, (uint32_t)n, d_ust, d_urec, d_scr, d_big,
-                               kBig, d_nbig, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(d_ctx, hctx.data(), hctx.size() * sizeof(int32_t),
-                           hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hb_launch_fill_u32(d_misc, 0u, 2, st);
-    if (e == hipSuccess) e = hb_launch_gap_list(a, d_list + 129, d_list + 128, d_list, st);
-    if (e == hipSuccess && pair) e = hb_launch_fill_u32(d_mid, 0u, HB_QUEUE_WORDS + 1, st);
-    for (int i = 0; e == hipSuccess && i < 4; ++i) e = hipEventCreate(&ev[i]);
-    if (e == hipSuccess) e = hipEventRecord(ev[0], st);
+    a.list = d_list + 1;
+    a.n_list = d_list;
     if (pair) {
         a.queues = d_mid;
         a.mid = d_mid + HB_QUEUE_WORDS;
+    }
+    uint32_t n_wide = 0;
+    uint32_t *d_nbig = d_scr + ns + nb;
+    hipError_t e = hb_launch_finalize(st3_in, ns, rec_in, (uint32_t)n, d_ust, d_urec, d_scr, d_big,
+                                      kBig, d_nbig, 1 + 128, st);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(d_ctx, hctx.data(), hctx.size() * sizeof(int32_t),
+                           hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hb_launch_gap_list(a, d_list + 1, d_list, d_nbig + 1, st);
+    for (int i = 0; ms_out && e == hipSuccess && i < 4; ++i) e = hipEventCreate(&ev[i]);
+    if (e == hipSuccess && ms_out) e = hipEventRecord(ev[0], st);
+    if (pair) {
         if (e == hipSuccess)
             e = hb_launch_gap_pair(a, (c->n_cu * 8 + HB_QUEUES - 1) / HB_QUEUES * HB_QUEUES, st);
         a.list = a.mid + 1;
         a.n_list = a.mid;
     }
     if (e == hipSuccess) e = hb_launch_gapped(a, false, c->n_cu * 8, st);
-    if (e == hipSuccess) e = hipEventRecord(ev[1], st);
-    if (e == hipSuccess) e = hipMemcpyAsync(&n_wide, d_misc + 1, sizeof(n_wide),
-                                            hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess && ms_out) e = hipEventRecord(ev[1], st);
+    // The dense layout and the copies out go behind the kernels with one wait
+    // for all; up to kAtOnce of records are copied before their number is known.
+    constexpr size_t kAtOnce = (size_t)1 << 20;
+    const size_t w_st = stats ? (size_t)ns * sizeof(hb_gapped_stats) : 0;
+    const size_t w_max = hsps ? (size_t)n * sizeof(hb_gapped_hsp) : 0;
+    const bool at_once = w_max <= kAtOnce && w_st <= CopyOut::kKeep / 2;
+    uint32_t *d_total = d_first + ns + nb + 1;
+    CopyOut out(c, 64 + CopyOut::room(std::max(w_st, w_max)), st);
+    size_t o_small = 0, o_st = 0, o_rec = 0;
+    uint64_t total = 0;
+    auto layout = [&]() {
+        if (e == hipSuccess) e = hb_launch_first_index(d_st3, ns, d_first, d_first + ns, d_total, st);
+        if (e == hipSuccess)
+            e = hb_launch_gap_compact(a, d_first, d_total, d_gst, d_gdense, d_small, st);
+        if (e != hipSuccess) return;
+        out.rewind();
+        o_small = out.add(d_small, sizeof(uint2));
+        o_st = out.add(d_gst, w_st);
+        if (at_once) o_rec = out.add(d_gdense, w_max);
+        e = out.wait();
+        uint2 v = make_uint2(0, 0);
+        if (e == hipSuccess) memcpy(&v, out.ptr(o_small), sizeof(v));
+        total = v.x;
+        n_wide = v.y;
+    };
+    layout();
     if (e == hipSuccess && n_wide) {
         // subjects that outgrew the LDS capacities: same code, global scratch
         std::vector<uint32_t> wl(n_wide);
@@ -1962,38 +2067,32 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
         a.n_wide = n_wide;
         if (oom) e = hipErrorOutOfMemory;
         if (e == hipSuccess) e = hb_launch_fill_u32(d_misc, 0u, 1, st);
-        if (e == hipSuccess) e = hipEventRecord(ev[2], st);
+        if (e == hipSuccess && ms_out) e = hipEventRecord(ev[2], st);
         if (e == hipSuccess) e = hb_launch_gapped(a, true, blocks, st);
-        if (e == hipSuccess) e = hipEventRecord(ev[3], st);
+        if (e == hipSuccess && ms_out) e = hipEventRecord(ev[3], st);
+        layout();
     }
     if (wide_out) *wide_out = n_wide;
-    if (e == hipSuccess) e = hb_launch_first_index(d_st3, ns, d_first, d_first + ns, st);
-    if (e == hipSuccess) e = hb_launch_gap_compact(a, d_first, d_gst, d_gdense, st);
-    uint32_t tail[2] = {0, 0};
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(&tail[0], d_first + ns - 1, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(&tail[1], d_st3 + 3 * (size_t)(ns - 1) + 2, sizeof(uint32_t),
-                           hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
     float ms = 0.f, ms2 = 0.f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
-    if (e == hipSuccess && n_wide) e = hipEventElapsedTime(&ms2, ev[2], ev[3]);
+    if (e == hipSuccess && ms_out) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
+    if (e == hipSuccess && ms_out && n_wide) e = hipEventElapsedTime(&ms2, ev[2], ev[3]);
     if (ms_out) *ms_out = ms + ms2;
-    const uint64_t total = (uint64_t)tail[0] + tail[1];
     if (e == hipSuccess) {
         if (n_hsp) *n_hsp = total;
         if (hsps && cap < total) {
             release();
             return HB_ERR_CAPACITY;
         }
-        if (stats && hb_copy_out(c, stats, d_gst, (size_t)ns * sizeof(hb_gapped_stats), st) !=
-                         HB_OK)
-            e = hipErrorUnknown;
-        if (e == hipSuccess && hsps && total &&
-            hb_copy_out(c, hsps, d_gdense, total * sizeof(hb_gapped_hsp), st) != HB_OK)
-            e = hipErrorUnknown;
+        const size_t w_rec = hsps ? (size_t)total * sizeof(hb_gapped_hsp) : 0;
+        const bool room = o_st + CopyOut::room(w_st) + w_rec <= CopyOut::kKeep;
+        if (!at_once && room) o_rec = out.add(d_gdense, w_rec);   // while the stats move on
+        if (w_st) out.store(stats, o_st, w_st);
+        if (!at_once && !room) {
+            out.rewind();
+            o_rec = out.add(d_gdense, w_rec);
+        }
+        if (!at_once) e = out.wait();
+        if (e == hipSuccess && w_rec) out.store(hsps, o_rec, w_rec);
     }
     release();
     if (e != hipSuccess) {
@@ -2054,31 +2153,44 @@ int hb_gapped_search(hb_ctx *c, hb_db *db, const uint8_t *seq, int32_t len, int3
     HB_CHECK(hipSetDevice(c->device));
     if (db->n == 0) return HB_OK;
     const uint32_t ns = db->n;
-    const size_t b_q = (size_t)len + 64, b_rec = std::max<size_t>(n_in, 1) * sizeof(hb_hsp);
+    // matrix, query (and spare bytes), records
+    const size_t o_rec = align256(1024 + (size_t)len + 64);
+    const size_t b_in = o_rec + std::max<size_t>(n_in, 1) * sizeof(hb_hsp);
     const size_t b_st3 = (size_t)ns * 3 * sizeof(uint32_t);
-    auto *d_q = static_cast<uint8_t *>(hb_pool_get(c, b_q));
-    auto *d_mat = static_cast<int8_t *>(hb_pool_get(c, 1024));
-    auto *d_rec = static_cast<hb_hsp *>(hb_pool_get(c, b_rec));
+    auto *d_in = static_cast<uint8_t *>(hb_pool_get(c, b_in));
     auto *d_st3 = static_cast<uint32_t *>(hb_pool_get(c, b_st3));
     auto release = [&]() {
-        hb_pool_put(c, d_q, b_q);
-        hb_pool_put(c, d_mat, 1024);
-        hb_pool_put(c, d_rec, b_rec);
+        hb_pool_put(c, d_in, b_in);
         hb_pool_put(c, d_st3, b_st3);
     };
-    if (!d_q || !d_mat || !d_rec || !d_st3) {
+    if (!d_in || !d_st3) {
         release();
         return HB_ERR_NOMEM;
     }
+    auto *d_mat = reinterpret_cast<int8_t *>(d_in);
+    uint8_t *d_q = d_in + 1024;
+    auto *d_rec = reinterpret_cast<hb_hsp *>(d_in + o_rec);
     hipStream_t st = c->stream;
-    hipError_t e = hipMemcpyAsync(d_q, seq, (size_t)len, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(d_mat, rp.mat32, 1024, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess && n_in)
-        e = hipMemcpyAsync(d_rec, in, n_in * sizeof(hb_hsp), hipMemcpyHostToDevice, st);
+    // matrix, query and (up to kStage bytes of) records in one copy
+    constexpr size_t kStage = (size_t)4 << 20;
+    const size_t w_rec = n_in * sizeof(hb_hsp);
+    const bool staged = w_rec <= kStage;
+    size_t pin_b = o_rec + (staged ? w_rec : 0);
+    auto *pin = static_cast<uint8_t *>(hb_pin_get(c, &pin_b));
+    hipError_t e = pin ? hipSuccess : hipErrorOutOfMemory;
+    if (e == hipSuccess) {
+        memcpy(pin, rp.mat32, 1024);
+        memcpy(pin + 1024, seq, (size_t)len);
+        if (staged && n_in) memcpy(pin + o_rec, in, w_rec);
+        e = hipMemcpyAsync(d_in, pin, o_rec + (staged ? w_rec : 0), hipMemcpyHostToDevice, st);
+    }
+    if (e == hipSuccess && !staged)
+        e = hipMemcpyAsync(d_rec, in, w_rec, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hb_launch_fill_u32(d_st3, 0u, 3 * ns, st);
     if (e == hipSuccess) e = hb_launch_count_oids(d_rec, (uint32_t)n_in, d_st3, st);
     if (e != hipSuccess) {
+        hipStreamSynchronize(st);
+        if (pin) hb_pin_put(c, pin, pin_b);
         release();
         hb_note_hip_error(e, "hb_gapped_search", __LINE__);
         return HB_ERR_DEVICE;
@@ -2086,6 +2198,8 @@ int hb_gapped_search(hb_ctx *c, hb_db *db, const uint8_t *seq, int32_t len, int3
     std::vector<int32_t> co(ctx_off, ctx_off + n_ctx), cl(ctx_len, ctx_len + n_ctx);
     rc = gapped_core(c, db, d_q, d_mat, co, cl, gap_cutoff, gp, d_st3, d_rec, n_in, stats, hsps,
                      cap, n_hsp, nullptr, nullptr);
+    if (rc) hipStreamSynchronize(st);   // (a call that succeeds has waited)
+    hb_pin_put(c, pin, pin_b);
     release();
     return rc;
 }
