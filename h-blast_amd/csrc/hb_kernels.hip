@@ -610,12 +610,13 @@ struct WaveScan {
             if (active) old = w_max(d, (word_t)mk << W::kMS);
             sync();
             const word_t wv = w_ld(d);
-            mwin = ballot((uint32_t)(wv >> W::kMS) == mk) & am;
+            // (the word holds a marker only: the max cleared the state)
+            mwin = ballot(wv == (word_t)mk << W::kMS) & am;
             // the first hit to reach the word found no marker and holds the
             // state (the max cleared the state bits for the hits after it); a
             // winner that came later gets it from that hit through the word
-            const uint64_t mfirst = ballot((uint32_t)(old >> W::kMS) == 0) & am;
-            st = (uint32_t)old & W::kSM;
+            const uint64_t mfirst = ballot(old < (word_t)1 << W::kMS) & am;
+            st = (uint32_t)old;   // (of the winners that came first, which it has no marker for)
             if (mwin & ~mfirst) {
                 if (lane_bit(mfirst & ~mwin)) w_or(d, old);
                 sync();
@@ -653,7 +654,7 @@ struct WaveScan {
         } else {
             if (win) w_st(d, (word_t)nst);
             sync();
-            st2 = (uint32_t)w_ld(d) & W::kSM;
+            st2 = (uint32_t)w_ld(d);   // (the winner's store cleared the marker)
         }
         const int32_t diff2 = (int32_t)((uint32_t)sb - st2);
         const uint64_t mlose = am & ~mwin;
@@ -961,6 +962,13 @@ struct WaveScan {
     // of the next round (ahead of every newer hit, so each diagonal still
     // sees its hits in subject order), and a round makes a single decision
     // pass.  Returns the subject's lookup hits.
+    // A round is bound by its instructions, vector ones above all: 17 fewer of
+    // about 190 (remainders as min(x, x - D) on unsigned values, the carried
+    // segment folded into the scan's operand, the tag count kept scalar, entry
+    // indices from one lane move, words compared unshifted) took 718.8 M residues
+    // against 1,000 from 10.58 to 10.17 ms.  Taking the staged hits in their own
+    // lanes instead of moving them behind the carried ones saved three LDS moves
+    // a round, cost instructions for the order of the carried and was 3% slower.
     template <bool SL, typename SP>
     __device__ __forceinline__ uint32_t subject(SP S, int32_t slen, uint32_t sl, int32_t sbase)
     {
@@ -985,6 +993,7 @@ struct WaveScan {
         // flight), position, position mod D
         uint32_t n_st = 0, n_a = 0, eq = 0;
         int32_t eso = 0, esm = 0;
+        uint32_t gen = (uint32_t)__builtin_amdgcn_readfirstlane((int)rgen);
         auto stage = [&]() {
             // A: a window with hits left, unless the subject has no more
             while (r == A.H && (hasB || nxt + 3 <= slen)) {
@@ -1018,40 +1027,35 @@ struct WaveScan {
             if (n_st == 0) return;
             // A's hits r .. r + t1 - 1 to lanes 0 .. t1 - 1, then B's 0 ..
             // t2 - 1; segment starts are tagged with their source position
-            // + 1 (B's positions count from 64)
-            if (++rgen == (1u << 24)) {
+            // + 1 (B's positions count from 64), older ones have lower tags
+            if (++gen == (1u << 24)) {
                 seg[lane] = 0;
-                rgen = 1;
+                gen = 1;
             }
-            const uint32_t tag = rgen << 8;
+            const uint32_t tag = gen << 8;
             const uint32_t ea = A.excl - r;
             if (ea < t1) seg[ea] = tag | ((uint32_t)lane + 1);
             if (t2 && B.excl < t2) seg[B.excl + t1] = tag | ((uint32_t)lane + 65);
             sync();
-            const uint32_t sv = seg[lane] - tag;
             // lanes before the first segment start continue the last taken
             // hit's segment (carry); the source of each lane is the largest
             // start at or before it
-            uint32_t v = sv < 256u ? sv : 0u;
-            if (lane == 0 && v == 0) v = carry + 1;
-            v = wave_incl_max(v);
-            const uint32_t p = v - 1;
-            const int p4 = (int)((p & 63u) << 2);
-            int32_t eb = __builtin_amdgcn_ds_bpermute(p4, A.eb);
+            const uint32_t p = wave_incl_max(max(seg[lane], tag + carry + 1)) - (tag + 1);
+            const int p4 = (int)(p << 2);   // (a lane move takes it modulo 64 lanes)
+            int32_t at = __builtin_amdgcn_ds_bpermute(p4, A.eb + (int32_t)r);
             if (t2) {   // B's position p - 64 (its lane p - 64)
-                const int32_t ebb = __builtin_amdgcn_ds_bpermute(p4, B.eb);
-                eb = p >= 64 ? ebb : eb;
+                const int32_t b = __builtin_amdgcn_ds_bpermute(p4, B.eb - (int32_t)t1);
+                at = p >= 64 ? b : at;
             }
             // (s0 + p) mod D, p < 128 <= 2 D (SPLIT: of the diagonal's position
             // in its class, (s0 + p + cls) >> shift)
-            int32_t smp = A.s0m + (int32_t)(SPLIT ? (p + cls) >> shift : p);
-            if (smp >= D) smp -= D;
-            if (smp >= D) smp -= D;
-            const uint32_t flat = (uint32_t)lane >= t1 ? (uint32_t)lane - t1 : (uint32_t)lane + r;
+            uint32_t smp = (uint32_t)A.s0m + (SPLIT ? (p + cls) >> shift : p);
+            smp = min(smp, smp - (uint32_t)D);
+            smp = min(smp, smp - (uint32_t)D);
             eq = 0;
-            if ((uint32_t)lane < n_st) eq = entries[(uint32_t)((int32_t)flat + eb)];
+            if ((uint32_t)lane < n_st) eq = entries[(uint32_t)lane + (uint32_t)at];
             eso = A.s0 + (int32_t)p;
-            esm = smp;
+            esm = (int32_t)smp;
             sync();
         };
         stage();
@@ -1060,7 +1064,7 @@ struct WaveScan {
             drain_some<SL>(S);
             // this round takes the first m staged hits into lanes c .. c + m - 1
             const uint32_t m = min(n_st, (uint32_t)HB_WAVE - c);
-            const int src4 = (int)((((uint32_t)lane - c) & 63u) << 2);
+            const int src4 = (int)(((uint32_t)lane - c) << 2);   // (modulo 64 lanes)
             const uint32_t qn = (uint32_t)__builtin_amdgcn_ds_bpermute(src4, (int)eq);
             const int32_t son = __builtin_amdgcn_ds_bpermute(src4, eso);
             const int32_t smp = __builtin_amdgcn_ds_bpermute(src4, esm);
@@ -1078,16 +1082,17 @@ struct WaveScan {
                 }
             }
             stage();
-            int32_t dn = (int32_t)(SPLIT ? qn >> shift : qn) - smp;
-            if (dn < 0) dn += D;
+            uint32_t dn = (SPLIT ? qn >> shift : qn) - (uint32_t)smp;
+            dn = min(dn, dn + (uint32_t)D);   // a negative one wraps
             const bool isc = (uint32_t)lane < c;
             const uint32_t q = isc ? cq : qn;
             const int32_t so = isc ? cs_ : son;
-            const uint32_t d = isc ? cd : (uint32_t)dn;
+            const uint32_t d = isc ? cd : dn;
             // the carried hits and the new ones: lanes 0 .. c + m - 1
-            const uint64_t am = c + m >= (uint32_t)HB_WAVE ? ~0ull : (1ull << (c + m)) - 1;
+            const uint64_t am = ballot((uint32_t)lane < c + m);
             c = carry_losers(decide_pass(am, q, so, d, sbase, sl), q, so, d, cq, cs_, cd);
         }
+        rgen = gen;
         return hits;
     }
 
