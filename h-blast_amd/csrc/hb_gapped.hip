@@ -17,8 +17,10 @@
 //     AdjustSubjectRange, :3608-3637); the HSP is saved when the two scores
 //     sum to the context's cutoff.
 //
-// Layout on CDNA4: one wavefront owns one subject (subjects are popped 64 at
-// a time from a counter).  The DP runs row by row (one query residue per
+// hb_gap_pair.hip takes the usual subjects with two of them per wavefront; what
+// it leaves, and other parameters, run here.
+// Layout on CDNA4: one wavefront owns one subject (a pop of a counter each).
+// The DP runs row by row (one query residue per
 // row) with the band's columns spread over the 64 lanes, so a row costs a
 // few VALU instructions per 64 cells instead of a sequential walk:
 //   T(b) = max(diagonal, gap-in-subject score carried down the column)

@@ -963,7 +963,7 @@ struct WaveScan {
     // sees its hits in subject order), and a round makes a single decision
     // pass.  Returns the subject's lookup hits.
     // A round is bound by its instructions, vector ones above all: 17 fewer of
-    // about 190 (remainders as min(x, x - D) on unsigned values, the carried
+    // about 200 (remainders as min(x, x - D) on unsigned values, the carried
     // segment folded into the scan's operand, the tag count kept scalar, entry
     // indices from one lane move, words compared unshifted) took 718.8 M residues
     // against 1,000 from 10.58 to 10.17 ms.  Taking the staged hits in their own
