@@ -260,49 +260,75 @@ static void host_copy(void *dst, const void *src, size_t bytes)
     for (auto &x : th) x.join();
 }
 
-// Copies of device memory to pageable host memory through the context's pinned
-// buffer (held while this lives, and of at least kKeep and room(bytes)): add()
-// enqueues one, wait() waits for all, store() moves one on.
+// Copies of device memory to pageable host memory through page-locked memory:
+// add() enqueues one, wait() waits for all, store() moves one on.  Up to kOwn
+// bytes go through a buffer of their own, so that a call whose kernels are still
+// running holds up no other thread's results; more through the context's (of at
+// least kKeep), which is held while this lives.
 namespace {
 class CopyOut {
   public:
-    CopyOut(hb_ctx *c, size_t bytes, hipStream_t st) : c_(c), st_(st), lk_(c->pinned_mu)
+    CopyOut(hb_ctx *c, size_t bytes, hipStream_t st) : c_(c), st_(st)
     {
-        bytes = std::max(room(bytes), kKeep);
-        if (c->pinned_bytes >= bytes) return;
-        if (c->pinned) hipHostFree(c->pinned);
-        c->pinned = nullptr;
-        c->pinned_bytes = 0;
-        e_ = hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault);
-        if (e_ == hipSuccess) c->pinned_bytes = bytes;
-        else c->pinned = nullptr;
+        bytes = std::max(room(bytes), (size_t)64);
+        if (bytes <= kOwn) {
+            cap_ = bytes;
+            base_ = own_ = static_cast<char *>(hb_pin_get(c, &cap_));
+            if (!own_) e_ = hipErrorOutOfMemory;
+            return;
+        }
+        lk_ = std::unique_lock<std::mutex>(c->pinned_mu);
+        bytes = std::max(bytes, kKeep);
+        if (c->pinned_bytes < bytes) {
+            if (c->pinned) hipHostFree(c->pinned);
+            c->pinned = nullptr;
+            c->pinned_bytes = 0;
+            e_ = hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault);
+            if (e_ == hipSuccess) c->pinned_bytes = bytes;
+            else c->pinned = nullptr;
+        }
+        base_ = static_cast<char *>(c->pinned);
+        cap_ = c->pinned_bytes;
     }
-    static constexpr size_t kKeep = (size_t)64 << 20;
+    ~CopyOut()
+    {
+        if (pending_) hipStreamSynchronize(st_);
+        hb_pin_put(c_, own_, cap_);
+    }
+    CopyOut(const CopyOut &) = delete;
+    CopyOut &operator=(const CopyOut &) = delete;
+    static constexpr size_t kKeep = (size_t)64 << 20, kOwn = (size_t)16 << 20;
     static size_t room(size_t bytes) { return (bytes + 63) & ~(size_t)63; }
+    bool fits(size_t bytes) const { return at_ + room(bytes) <= cap_; }
     size_t add(const void *src, size_t bytes)
     {
         const size_t at = at_;
+        if (e_ == hipSuccess && !fits(bytes)) e_ = hipErrorInvalidValue;
         at_ += room(bytes);
-        if (e_ == hipSuccess && at_ > c_->pinned_bytes) e_ = hipErrorInvalidValue;
-        if (e_ == hipSuccess && bytes)
+        if (e_ == hipSuccess && bytes) {
             e_ = hipMemcpyAsync(ptr(at), src, bytes, hipMemcpyDeviceToHost, st_);
+            pending_ = true;
+        }
         return at;
     }
     void rewind() { at_ = 0; }   // after a wait: what was copied is no longer needed
     hipError_t wait()
     {
         if (e_ == hipSuccess) e_ = hipStreamSynchronize(st_);
+        if (e_ == hipSuccess) pending_ = false;
         return e_;
     }
-    char *ptr(size_t at) const { return static_cast<char *>(c_->pinned) + at; }
+    char *ptr(size_t at) const { return base_ + at; }
     void store(void *dst, size_t at, size_t bytes) const { host_copy(dst, ptr(at), bytes); }
 
   private:
     hb_ctx *c_;
     hipStream_t st_;
     std::unique_lock<std::mutex> lk_;
+    char *own_ = nullptr, *base_ = nullptr;
+    size_t cap_ = 0, at_ = 0;
+    bool pending_ = false;
     hipError_t e_ = hipSuccess;
-    size_t at_ = 0;
 };
 }  // namespace
 
@@ -1732,7 +1758,7 @@ int hb_scan_results(hb_scan *s, hb_subject_stats *stats, hb_hsp *hsps, uint64_t 
         // for that
         const size_t w_st = stats ? b_st : 0, w_rec = hsps ? (size_t)n * sizeof(hb_hsp) : 0;
         const bool at_once = 64 + CopyOut::room(w_st) + CopyOut::room(w_rec) <= CopyOut::kKeep;
-        CopyOut out(c, 64 + CopyOut::room(std::max(w_st, w_rec)), st);
+        CopyOut out(c, 64 + (at_once ? CopyOut::room(w_st) + w_rec : std::max(w_st, w_rec)), st);
         const size_t o_big = out.add(d_nbig, sizeof(nbig)), o_st = out.add(d_st, w_st);
         size_t o_rec = at_once ? out.add(d_rec, w_rec) : 0;
         e = out.wait();
@@ -1837,7 +1863,7 @@ int hb_scan_results_compact(hb_scan *s, hb_subject_hits *subj, uint64_t subj_cap
         const size_t w_sub = subj ? (size_t)max_subj * sizeof(hb_subject_hits) : 0;
         const size_t w_rec = hsps ? (size_t)n * sizeof(hb_hsp) : 0;
         const bool at_once = w_sub + w_rec <= kAtOnce;
-        CopyOut out(c, 0, st);
+        CopyOut out(c, 64 + (at_once ? CopyOut::room(w_sub) + w_rec : 0), st);
         const size_t o_small = out.add(d_small, sizeof(small));
         const size_t o_sub = at_once ? out.add(d_sub, w_sub) : 0;
         const size_t o_rec = at_once ? out.add(d_rec, w_rec) : 0;
@@ -2019,9 +2045,10 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
     constexpr size_t kAtOnce = (size_t)1 << 20;
     const size_t w_st = stats ? (size_t)ns * sizeof(hb_gapped_stats) : 0;
     const size_t w_max = hsps ? (size_t)n * sizeof(hb_gapped_hsp) : 0;
-    const bool at_once = w_max <= kAtOnce && w_st <= CopyOut::kKeep / 2;
+    const size_t w_all = 64 + CopyOut::room(w_st) + w_max;
+    const bool at_once = w_max <= kAtOnce && w_all <= CopyOut::kKeep;
     uint32_t *d_total = d_first + ns + nb + 1;
-    CopyOut out(c, 64 + CopyOut::room(std::max(w_st, w_max)), st);
+    CopyOut out(c, w_all <= CopyOut::kKeep ? w_all : 64 + std::max(w_st, w_max), st);
     size_t o_small = 0, o_st = 0, o_rec = 0;
     uint64_t total = 0;
     auto layout = [&]() {
@@ -2084,7 +2111,7 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
             return HB_ERR_CAPACITY;
         }
         const size_t w_rec = hsps ? (size_t)total * sizeof(hb_gapped_hsp) : 0;
-        const bool room = o_st + CopyOut::room(w_st) + w_rec <= CopyOut::kKeep;
+        const bool room = out.fits(w_rec);
         if (!at_once && room) o_rec = out.add(d_gdense, w_rec);   // while the stats move on
         if (w_st) out.store(stats, o_st, w_st);
         if (!at_once && !room) {
