@@ -29,11 +29,12 @@
 // column state's decrement (all compares of a row are between cells of that
 // row), and the bias makes 0, which lane moves fill in, lower than any live cell.
 //
-// Bound by vector instruction issue: 121 of them per row of four sides (30 a
+// Bound by vector instruction issue: 118 of them per row of four sides (30 a
 // side; hb_gapped.hip spends 53 and as many scalar ones on a row of one side),
 // which fill 3/4 of the kernel's time.  The 73,052 HSPs of a 1,000-residue query
-// against 500,000 subjects take 950 us here and 1,507 us there, the 5,191 of 350
-// residues against 50,000 long-tailed subjects 195 and 340 us.  One set of 6
+// against 500,000 subjects take 920 us here and 1,507 us there, the 5,191 of 350
+// residues against 50,000 long-tailed subjects 186 and 340 us (950 and 195 us with
+// two tests a row for the letters at hand and the last row instead of one).  One set of 6
 // columns a lane took 1,000 us and left more subjects to the other kernel (373
 // us of it, its longest chain of rows), 5 columns 901 and 509 us.
 #include <hip/hip_runtime.h>
@@ -148,7 +149,9 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
     int32_t ob[kC], ov[kC], ob2[kC], ov2[kC], sv[kC];
     int32_t colb = 0, Xl = -1;             // first column; X (-1 past the staged letters)
     uint32_t l1 = 0, l2 = 0, ln = 0;       // letters * 2 of the columns; those right of the window
-    uint32_t qrow = 0, qnext = 0;          // letters of the rows to come, one per lane
+    uint32_t qrow = 0, qnext = 0;          // letters * 64 of the rows to come, one per lane; letters
+                                           // of the 16 rows after those
+    int32_t event = 0;                     // the row after which they run out, or the last row
 #pragma unroll
     for (int j = 0; j < kC; ++j) {
         ob[j] = ov[j] = ob2[j] = ov2[j] = kDead;
@@ -396,8 +399,9 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                 a = abest = 0;
                 top = kBias;
                 stop = INT32_MAX;
-                qrow = 0;
-                qnext = row_letters(1);
+                qrow = row_letters(1) << 6;
+                qnext = row_letters(17);
+                event = min(16, M);
                 ovf = false;
                 ran = true;
                 break;
@@ -461,15 +465,9 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
         do {
             ++a;
             top += ge;
-            if (ballot((a & 15) == 1)) {
-                if ((a & 15) == 1) {
-                    qrow = qnext;
-                    qnext = row_letters(a + 16);
-                }
-            }
             const int32_t row = dpp<kBcast>((int32_t)qrow);
             qrow = (uint32_t)dpp<kShl1>((int32_t)qrow);
-            const char *mrow = mat_b + 64 * row;
+            const char *mrow = mat_b + row;
             const int32_t last_ob = ob[kC - 1];
             const Row w = eval(mrow, l1, dpp<kShr1>(last_ob), lane_ge, Xl, 0, top, ob, ov);
             live = w.any;
@@ -505,9 +503,9 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                     for (int j = 0; j < kC; ++j) sv[j] = w.S[j];
                 }
             }
-            // the rows are used up
-            const uint64_t end = ballot(a == M);
-            if (end) {
+            // the rows, or the letters at hand, are used up
+            if (ballot(a == event)) {
+                const uint64_t end = ballot(a == event && a == M);
                 live &= ~end;
                 live0 &= ~end;
 #pragma unroll
@@ -516,6 +514,11 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                     ov[j] = lane_bit(end) ? kDead : ov[j];
                     ob2[j] = lane_bit(end) ? kDead : ob2[j];
                     ov2[j] = lane_bit(end) ? kDead : ov2[j];
+                }
+                if (a == event) {
+                    event = min(a + 16, M);
+                    qrow = qnext << 6;
+                    qnext = row_letters(a + 17);
                 }
             }
             // the band may leave the window, or the staged letters
