@@ -474,11 +474,14 @@ static int autotune(hb_batch *b, int32_t *best)
     return HB_OK;
 }
 
+// After this and until a pass is collected the batch has no results.
 static void drop_results(hb_batch *b)
 {
     hb_pin_put(b->ctx, b->pin, b->pin_bytes);
     b->pin = nullptr;
     b->results = nullptr;
+    b->q_first.clear();
+    b->q_count.clear();
 }
 
 // The same without device memory: the records are mapped and ordered here.
@@ -497,6 +500,9 @@ static int collect_host(hb_batch *b, uint32_t n)
         const int32_t qx = b->ctx_query[x.context], qy = b->ctx_query[y.context];
         return std::tie(qx, x.oid, x.s_off, x.q_off) < std::tie(qy, y.oid, y.s_off, y.q_off);
     });
+    const size_t nq = b->queries.size();
+    b->q_first.assign(nq + 1, 0);
+    b->q_count.assign(nq, 0);
     for (hb_hsp &h : b->many) {
         const int32_t q = b->ctx_query[h.context];
         h.context = b->ctx_local[h.context];
@@ -504,7 +510,7 @@ static int collect_host(hb_batch *b, uint32_t n)
         h.q_off -= b->q_base[q];
         b->q_count[q]++;
     }
-    for (size_t q = 0; q < b->q_count.size(); ++q) b->q_first[q + 1] = b->q_first[q] + b->q_count[q];
+    for (size_t q = 0; q < nq; ++q) b->q_first[q + 1] = b->q_first[q] + b->q_count[q];
     b->results = b->many.data();
     return HB_OK;
 }
@@ -516,8 +522,6 @@ static int collect(hb_batch *b, uint32_t n)
     hb_ctx *c = b->ctx;
     const size_t nq = b->queries.size(), ng = b->gs.desc.size(), nc = b->ctx_query.size();
     drop_results(b);
-    b->q_first.assign(nq + 1, 0);
-    b->q_count.assign(nq, 0);
     // one page-locked buffer: context map (up), totals, first records (down),
     // then the records unless they are many
     constexpr size_t kPinMax = (size_t)12 << 20;
@@ -579,6 +583,8 @@ static int collect(hb_batch *b, uint32_t n)
     for (size_t g = 0; g < ng; ++g)
         for (int k = 0; k < 3; ++k) b->tot[k] += tot[3 * g + k];
     const auto *first = reinterpret_cast<const uint32_t *>(pin + o_first);
+    b->q_first.assign(nq + 1, 0);
+    b->q_count.assign(nq, 0);
     for (size_t q = 0; n && q < nq; ++q) {
         b->q_first[q] = first[q];
         b->q_count[q] = first[q + 1] - first[q];

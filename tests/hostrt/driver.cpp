@@ -1,0 +1,119 @@
+// driver.cpp -- the host runtime over the stand-in of fake_hip.h (test
+// infrastructure): `driver NAME` runs one scenario; exit status 0 = its
+// checks hold.
+#include "fake_hip.h"
+
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "hb_runtime.h"
+
+static int fails = 0;
+#define CHECK(c)                                                               \
+    do {                                                                       \
+        if (!(c)) {                                                            \
+            std::fprintf(stderr, "check failed: %s (line %d)\n", #c, __LINE__); \
+            ++fails;                                                           \
+        }                                                                      \
+    } while (0)
+
+namespace {
+
+struct Fixture {
+    hb_ctx *c = nullptr;
+    Fixture() { CHECK(hb_create(0, &c) == HB_OK); }
+    ~Fixture()
+    {
+        if (c) CHECK(hb_destroy(c) == HB_OK);
+    }
+    // n subjects of `len` residues
+    hb_db *database(uint32_t n, uint32_t len = 16, int rc = HB_OK)
+    {
+        std::vector<uint8_t> res((size_t)n * len + 1, 1);
+        std::vector<uint64_t> offs(n + 1);
+        for (uint32_t i = 0; i <= n; ++i) offs[i] = (uint64_t)i * len;
+        hb_db *db = nullptr;
+        CHECK(hb_db_upload(c, res.data(), offs.data(), n, &db) == rc);
+        return db;
+    }
+    hb_batch *batch(hb_db *db, int queries, hipStream_t st = nullptr)
+    {
+        hb_batch_opts o;
+        hb_batch_opts_default(&o);
+        o.group_residues = 768;
+        o.use_graph = 0;
+        hb_batch *b = nullptr;
+        CHECK(hb_batch_create_on(c, db, nullptr, &o, st, &b) == HB_OK);
+        const std::vector<uint8_t> seq(100, 1);
+        const int32_t off = 0, len = 100, x = 16, cut = 41;
+        for (int i = 0; i < queries; ++i)
+            CHECK(hb_batch_add(b, seq.data(), len, 1, &off, &len, &x, &cut, nullptr) == HB_OK);
+        return b;
+    }
+    hb_query *query(int32_t len = 100)
+    {
+        const std::vector<uint8_t> seq(len, 1);
+        const int32_t off = 0, x = 16, cut = 41;
+        hb_query *q = nullptr;
+        CHECK(hb_query_prepare(c, seq.data(), len, 1, &off, &len, &x, &cut, nullptr, &q) == HB_OK);
+        return q;
+    }
+};
+
+// Every scan finds n HSPs of query 0.
+void found(uint32_t n)
+{
+    g_fake.scan = [n](const hb_scan_args &a) {
+        for (uint32_t i = 0; i < n && i < a.out_cap; ++i) {
+            memset(&a.out[i], 0, sizeof(hb_hsp));
+            a.out[i].oid = i;
+        }
+        *a.out_count = n;
+    };
+}
+
+// A pass whose results could not be collected leaves none.
+void failed_collect()
+{
+    Fixture f;
+    hb_db *db = f.database(10);
+    found(7);
+    hb_batch *b = f.batch(db, 2);
+    uint64_t n = 99;
+    g_fake.fail_order = 1;
+    CHECK(hb_batch_run(b) == HB_ERR_DEVICE);
+    CHECK(hb_batch_results(b, 0, nullptr, 0, &n) == HB_ERR_STATE);
+    CHECK(hb_batch_run(b) == HB_OK);
+    CHECK(hb_batch_results(b, 0, nullptr, 0, &n) == HB_OK && n == 7);
+    g_fake.fail_order = 1;
+    CHECK(hb_batch_run(b) == HB_ERR_DEVICE);
+    CHECK(hb_batch_results(b, 1, nullptr, 0, &n) == HB_ERR_STATE);
+    CHECK(hb_batch_run(b) == HB_OK);
+    std::vector<hb_hsp> got(7);
+    CHECK(hb_batch_results(b, 0, got.data(), 7, &n) == HB_OK && n == 7 && got[6].oid == 6);
+    CHECK(hb_batch_results(b, 1, nullptr, 0, &n) == HB_OK && n == 0);
+    hb_batch_free(b);
+    hb_db_free(db);
+}
+
+const struct {
+    const char *name;
+    void (*run)();
+} kScenarios[] = {
+    {"failed_collect", failed_collect},
+};
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    for (const auto &s : kScenarios)
+        if (argc > 1 && std::string(argv[1]) == s.name) {
+            s.run();
+            return fails ? 1 : 0;
+        }
+    std::fprintf(stderr, "no such scenario\n");
+    return 2;
+}
