@@ -493,7 +493,10 @@ static int collect_host(hb_batch *b, uint32_t n)
                             hipMemcpyDeviceToHost, b->st));
     b->many.resize(n);
     const int rc = hb_copy_out(b->ctx, b->many.data(), b->d_out, (size_t)n * sizeof(hb_hsp), b->st);
-    if (rc) return rc;
+    if (rc) {
+        hipStreamSynchronize(b->st);   // the counters' copy
+        return rc;
+    }
     b->tot[0] = b->tot[1] = b->tot[2] = 0;
     for (size_t i = 0; i < tot.size(); ++i) b->tot[i % 3] += tot[i];
     std::sort(b->many.begin(), b->many.end(), [&](const hb_hsp &x, const hb_hsp &y) {
@@ -576,6 +579,7 @@ static int collect(hb_batch *b, uint32_t n)
     } else {
         std::vector<hb_hsp>().swap(b->many);
     }
+    if (rc) hipStreamSynchronize(b->st);   // what was enqueued
     hb_pool_put(c, dev, dev_b);
     if (rc) return rc;
     b->tot[0] = b->tot[1] = b->tot[2] = 0;

@@ -1792,6 +1792,7 @@ int hb_scan_results(hb_scan *s, hb_subject_stats *stats, hb_hsp *hsps, uint64_t 
                     big.push_back(hb_fin_big{i, sp[i].n_hsp, (uint64_t)sp[i].first});
         }
     }
+    if (e != hipSuccess) hipStreamSynchronize(st);   // the kernels that were launched
     release();
     if (e != hipSuccess) {
         hb_note_hip_error(e, "hb_scan_results", __LINE__);
@@ -1908,6 +1909,7 @@ int hb_scan_results_compact(hb_scan *s, hb_subject_hits *subj, uint64_t subj_cap
                     big.push_back(hb_fin_big{sp[i].oid, sp[i].n_hsp, sp[i].first});
         }
     }
+    if (e != hipSuccess) hipStreamSynchronize(st);   // the kernels that were launched
     release();
     if (e != hipSuccess) {
         hb_note_hip_error(e, "hb_scan_results_compact", __LINE__);
@@ -2121,6 +2123,7 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
         if (!at_once) e = out.wait();
         if (e == hipSuccess && w_rec) out.store(hsps, o_rec, w_rec);
     }
+    if (e != hipSuccess) hipStreamSynchronize(st);   // the kernels that were launched
     release();
     if (e != hipSuccess) {
         hb_note_hip_error(e, "gapped stage", __LINE__);

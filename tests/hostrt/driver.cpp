@@ -98,11 +98,60 @@ void failed_collect()
     hb_db_free(db);
 }
 
+// A call that fails has waited for what it enqueued: its buffers go back to
+// the pool, and the next load fills them on other streams.
+void failed_calls_wait()
+{
+    Fixture f;
+    hb_db *db = f.database(20000);
+    hb_query *q = f.query();
+    found(20000);
+    hb_scan *s = nullptr;
+    CHECK(hb_scan_start(f.c, db, q, &s) == HB_OK && hb_scan_wait(s) == HB_OK);
+    std::vector<hb_subject_stats> st(20000);
+    std::vector<hb_subject_hits> sub(20000);
+    std::vector<hb_hsp> hsps(20000);
+    std::vector<hb_gapped_stats> gst(20000);
+    std::vector<hb_gapped_hsp> g(20000);
+    hb_scan_totals tot;
+    hb_gap_params gp;
+    hb_gap_params_default(&gp);
+    const int32_t cut = 30;
+    uint64_t n = 0;
+    for (int how = 0; how < 2; ++how) {
+        // no page-locked memory, or a kernel that cannot be launched
+        std::atomic<int> &fail = how ? g_fake.fail_finalize : g_fake.fail_host_malloc;
+        fail = 1;
+        CHECK(hb_scan_results(s, st.data(), hsps.data(), hsps.size(), &n) == HB_ERR_DEVICE);
+        CHECK(fake_pending(f.c->stream) == 0);
+        fail = 1;
+        CHECK(hb_scan_results_compact(s, sub.data(), sub.size(), hsps.data(), hsps.size(), &tot) ==
+              HB_ERR_DEVICE);
+        CHECK(fake_pending(f.c->stream) == 0);
+        fail = 1;
+        CHECK(hb_scan_gapped(s, &gp, &cut, gst.data(), g.data(), g.size(), &n) < 0);
+        CHECK(fake_pending(f.c->stream) == 0);
+        CHECK(fail == 0);
+    }
+    found(3);
+    hipStream_t own = nullptr;
+    CHECK(hipStreamCreateWithFlags(&own, hipStreamNonBlocking) == hipSuccess);
+    hb_batch *b = f.batch(db, 1, own);
+    g_fake.fail_order = 1;
+    CHECK(hb_batch_run(b) == HB_ERR_DEVICE);
+    CHECK(fake_pending(own) == 0);
+    hb_batch_free(b);
+    hb_scan_free(s);
+    hb_query_free(q);
+    hb_db_free(db);
+}
+
 const struct {
     const char *name;
     void (*run)();
 } kScenarios[] = {
     {"failed_collect", failed_collect},
+    {"failed_calls_wait", failed_calls_wait},
 };
 
 }  // namespace

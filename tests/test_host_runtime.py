@@ -49,3 +49,7 @@ def run(driver, name):
 
 def test_failed_pass_leaves_no_results(driver):
     run(driver, "failed_collect")
+
+
+def test_failed_call_waits_for_its_work(driver):
+    run(driver, "failed_calls_wait")
