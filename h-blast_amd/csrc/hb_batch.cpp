@@ -487,7 +487,6 @@ static void drop_results(hb_batch *b)
 // The same without device memory: the records are mapped and ordered here.
 static int collect_host(hb_batch *b, uint32_t n)
 {
-    hipGetLastError();   // the allocation that failed
     std::vector<unsigned long long> tot(3 * b->gs.desc.size());
     HB_CHECK(hipMemcpyAsync(tot.data(), b->d_totals, tot.size() * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, b->st));

@@ -36,6 +36,8 @@ const int8_t kHbBlosum62[HB_ALPHA][HB_ALPHA] = {
 #include "hb_blosum62.inc"
 };
 
+// (An allocation that fails and is handled must not leave its error: the next
+// launcher would return it.)
 void *hb_pool_get(hb_ctx *c, size_t bytes)
 {
     {
@@ -62,7 +64,10 @@ void *hb_pool_get(hb_ctx *c, size_t bytes)
         c->pool.clear();
         c->pool_bytes = 0;
     }
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     return p;
 }
 
@@ -118,7 +123,10 @@ void *hb_pin_get(hb_ctx *c, size_t *bytes)
     }
     *bytes = (*bytes + 0x3ffff) & ~(size_t)0x3ffff;
     void *p = nullptr;
-    if (hipHostMalloc(&p, *bytes, hipHostMallocDefault) != hipSuccess) return nullptr;
+    if (hipHostMalloc(&p, *bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     return p;
 }
 
@@ -162,6 +170,7 @@ class Upload {
         else if (at.type == hipMemoryTypeHost) return;
         if (!c->up_stream &&
             hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
             c->up_stream = nullptr;
             return;
         }
@@ -284,8 +293,12 @@ class CopyOut {
             c->pinned = nullptr;
             c->pinned_bytes = 0;
             e_ = hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault);
-            if (e_ == hipSuccess) c->pinned_bytes = bytes;
-            else c->pinned = nullptr;
+            if (e_ == hipSuccess) {
+                c->pinned_bytes = bytes;
+            } else {
+                (void)hipGetLastError();
+                c->pinned = nullptr;
+            }
         }
         base_ = static_cast<char *>(c->pinned);
         cap_ = c->pinned_bytes;
@@ -827,6 +840,7 @@ int hb_host_alloc(hb_ctx *c, uint64_t bytes, void **out)
     *out = nullptr;
     HB_CHECK(hipSetDevice(c->device));
     if (hipHostMalloc(out, std::max<uint64_t>(bytes, 1), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         *out = nullptr;
         return HB_ERR_NOMEM;
     }
@@ -2269,6 +2283,7 @@ int hb_diag_copy(hb_ctx *c, uint64_t bytes, int reps, float *ms_per_copy)
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = HB_OK;
     if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) {
+        (void)hipGetLastError();
         rc = HB_ERR_NOMEM;
     } else if (hipMemsetAsync(a, 1, bytes, c->stream) != hipSuccess ||
                hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess ||

@@ -146,12 +146,80 @@ void failed_calls_wait()
     hb_db_free(db);
 }
 
+// An allocation that fails and is handled leaves no error for the launches
+// after it: the load takes the plain copy, and the next call works.
+void handled_errors()
+{
+    const uint32_t n = 20000, len = 300;   // 6 MB: through page-locked chunks
+    for (std::atomic<int> *fail : {&g_fake.fail_host_malloc, &g_fake.fail_stream_create}) {
+        Fixture g;
+        *fail = 1;
+        const int copies = g_fake.host_to_device;
+        hb_db *db = g.database(n, len);
+        CHECK(*fail == 0 && g_fake.host_to_device == copies + 3);   // residues, offsets, tiles
+        hb_db_free(db);
+    }
+    Fixture f;
+    hb_db *db = f.database(n);
+    hb_query *q = f.query();
+    found(5);
+    hb_scan *s = nullptr;
+    g_fake.fail_malloc = 2;
+    CHECK(hb_scan_start(f.c, db, q, &s) == HB_ERR_NOMEM);
+    g_fake.fail_malloc = 0;
+    CHECK(hb_scan_start(f.c, db, q, &s) == HB_OK);
+    CHECK(hb_scan_wait(s) == HB_OK);
+    std::vector<hb_subject_stats> st(n);
+    std::vector<hb_hsp> hsps(5);
+    uint64_t found_n = 0;
+    g_fake.fail_host_malloc = 1;
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_ERR_DEVICE);
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK && found_n == 5);
+    // results past 16 MiB: the context's own buffer
+    hb_scan_free(s);
+    hb_db_free(db);
+    const uint32_t many = 1 << 20;
+    db = f.database(many, 1);
+    CHECK(hb_scan_start(f.c, db, q, &s) == HB_OK);
+    st.resize(many);
+    g_fake.fail_host_malloc = 1;
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_ERR_DEVICE);
+    CHECK(g_fake.fail_host_malloc == 0);
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
+    void *p = nullptr;
+    g_fake.fail_host_malloc = 1;
+    CHECK(hb_host_alloc(f.c, 64, &p) == HB_ERR_NOMEM);
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
+    float ms = 0;
+    g_fake.fail_malloc = 1;
+    CHECK(hb_diag_copy(f.c, 4096, 1, &ms) == HB_ERR_NOMEM);
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
+    // a batch whose order finds no memory orders on the host
+    hb_batch *b = f.batch(db, 1);
+    CHECK(hb_batch_run(b) == HB_OK);
+    f.c->pool_mu.lock();
+    for (auto &x : f.c->pool) (void)hipFree(x.first);
+    f.c->pool.clear();
+    f.c->pool_bytes = 0;
+    f.c->pool_mu.unlock();
+    g_fake.fail_malloc = 2;
+    CHECK(hb_batch_run(b) == HB_OK);
+    g_fake.fail_malloc = 0;
+    CHECK(hb_batch_results(b, 0, nullptr, 0, &found_n) == HB_OK && found_n == 5);
+    CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
+    hb_batch_free(b);
+    hb_scan_free(s);
+    hb_query_free(q);
+    hb_db_free(db);
+}
+
 const struct {
     const char *name;
     void (*run)();
 } kScenarios[] = {
     {"failed_collect", failed_collect},
     {"failed_calls_wait", failed_calls_wait},
+    {"handled_errors", handled_errors},
 };
 
 }  // namespace

@@ -53,3 +53,7 @@ def test_failed_pass_leaves_no_results(driver):
 
 def test_failed_call_waits_for_its_work(driver):
     run(driver, "failed_calls_wait")
+
+
+def test_handled_errors_are_cleared(driver):
+    run(driver, "handled_errors")
