@@ -20,7 +20,6 @@ struct Class {
     uint32_t tiles_per_item = 1;
     int place = HB_PLACE_LDS;          // where the diagonal state goes
     uint32_t *d_gstate = nullptr;   // diag_len_max words per wavefront of the grid
-    size_t gstate_bytes = 0;
 };
 
 }  // namespace
@@ -80,10 +79,10 @@ static void free_groups(hb_batch *b)
 {
     free_graph(b);
     hb_group_set_free(&b->gs);
-    hb_pool_put(b->ctx, b->d_misc, misc_words(b) * sizeof(uint32_t));
-    hb_pool_put(b->ctx, b->d_totals, 3 * b->gs.desc.size() * sizeof(unsigned long long));
+    hb_pool_put(b->ctx, b->d_misc);
+    hb_pool_put(b->ctx, b->d_totals);
     for (Class &c : b->classes)
-        if (c.d_gstate) hb_pool_put(b->ctx, c.d_gstate, c.gstate_bytes);
+        if (c.d_gstate) hb_pool_put(b->ctx, c.d_gstate);
     b->d_misc = nullptr;
     b->d_totals = nullptr;
     b->classes.clear();
@@ -254,9 +253,9 @@ static int build(hb_batch *b, int32_t target)
                             &c.cfg, c.place, b->g_ring, b->g_waves);
         if (rc) return rc;
         if (c.place == HB_PLACE_GLOBAL) {
-            c.gstate_bytes =
-                (size_t)c.cfg.blocks * c.cfg.waves * (size_t)c.diag_len_max * HB_GSTATE_WORD;
-            c.d_gstate = static_cast<uint32_t *>(hb_pool_get(b->ctx, c.gstate_bytes));
+            c.d_gstate = static_cast<uint32_t *>(hb_pool_get(
+                b->ctx,
+                (size_t)c.cfg.blocks * c.cfg.waves * (size_t)c.diag_len_max * HB_GSTATE_WORD));
             if (!c.d_gstate) return HB_ERR_NOMEM;
         }
     }
@@ -331,7 +330,7 @@ static int ensure_out(hb_batch *b, uint32_t cap)
 {
     if (b->d_out && b->cap >= cap) return HB_OK;
     free_graph(b);   // the captured launches hold the old buffer
-    hb_pool_put(b->ctx, b->d_out, (size_t)b->cap * sizeof(hb_hsp));
+    hb_pool_put(b->ctx, b->d_out);
     b->cap = 0;
     b->d_out = static_cast<hb_hsp *>(hb_pool_get(b->ctx, (size_t)cap * sizeof(hb_hsp)));
     if (!b->d_out) return HB_ERR_NOMEM;
@@ -579,7 +578,7 @@ static int collect(hb_batch *b, uint32_t n)
         std::vector<hb_hsp>().swap(b->many);
     }
     if (rc) hipStreamSynchronize(b->st);   // what was enqueued
-    hb_pool_put(c, dev, dev_b);
+    hb_pool_put(c, dev);
     if (rc) return rc;
     b->tot[0] = b->tot[1] = b->tot[2] = 0;
     const auto *tot = reinterpret_cast<const unsigned long long *>(pin + o_tot);
@@ -820,7 +819,7 @@ int hb_batch_free(hb_batch *b)
     hipStreamSynchronize(b->st);
     free_groups(b);
     drop_results(b);
-    hb_pool_put(b->ctx, b->d_out, (size_t)b->cap * sizeof(hb_hsp));
+    hb_pool_put(b->ctx, b->d_out);
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);
     delete b;

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <unordered_map>
 #include <vector>
 
 #include "hb_internal.h"
@@ -31,8 +32,9 @@ struct hb_ctx {
     // Device buffers of finished scans, reused by later scans so that a
     // per-query loop does not pay hipMalloc/hipFree per call.
     std::mutex pool_mu;
-    std::vector<std::pair<void *, size_t>> pool;
+    std::vector<std::pair<void *, size_t>> pool;   // kept buffers and their sizes
     size_t pool_bytes = 0;
+    std::unordered_map<void *, size_t> lent;       // ... those handed out
     // pinned host staging for result copies (grown on demand, kept)
     std::mutex pinned_mu;
     void *pinned = nullptr;
@@ -57,7 +59,7 @@ void hb_pin_put(hb_ctx *c, void *p, size_t bytes);
 // Buffers of the pool; one that nothing on the device uses any more goes back
 // to it.  hb_pool_held: the bytes that it keeps.
 void *hb_pool_get(hb_ctx *c, size_t bytes);
-void hb_pool_put(hb_ctx *c, void *p, size_t bytes);
+void hb_pool_put(hb_ctx *c, void *p, size_t keep = (size_t)-1);
 size_t hb_pool_held(hb_ctx *c);
 
 struct hb_db {
@@ -75,9 +77,6 @@ struct hb_db {
     uint32_t n_tiles = 0;          // n_qtiles + 1 of the plain scan's queue tiles
     uint32_t n_qtiles = 0;
     void *load_scratch = nullptr;  // while it is loaded
-    size_t load_bytes = 0;
-    // sizes of the allocations (from the context's pool)
-    size_t res_bytes = 0, offs_bytes = 0, subj_bytes = 0, alloc_bytes = 0, tiles_bytes = 0;
     std::vector<uint64_t> h_offs;
     uint64_t max_len = 0;   // longest subject
     float hdb_len_ms = 0.f, hdb_copy_ms = 0.f;   // hb_db_upload_hdb's kernels

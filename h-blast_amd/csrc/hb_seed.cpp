@@ -36,38 +36,42 @@ const int8_t kHbBlosum62[HB_ALPHA][HB_ALPHA] = {
 #include "hb_blosum62.inc"
 };
 
+// A buffer of at least `bytes` and at most twice that and 4 KB.  The pool keeps
+// the sizes that its buffers have, also while they are handed out: one that
+// served something smaller is as large as before when it comes back.
 // (An allocation that fails and is handled must not leave its error: the next
 // launcher would return it.)
 void *hb_pool_get(hb_ctx *c, size_t bytes)
 {
-    {
-        std::lock_guard<std::mutex> lk(c->pool_mu);
-        size_t best = (size_t)-1;
-        for (size_t i = 0; i < c->pool.size(); ++i)
-            if (c->pool[i].second >= bytes && c->pool[i].second <= 2 * bytes + 4096 &&
-                (best == (size_t)-1 || c->pool[i].second < c->pool[best].second))
-                best = i;
-        if (best != (size_t)-1) {
-            void *p = c->pool[best].first;
-            c->pool_bytes -= c->pool[best].second;
-            c->pool.erase(c->pool.begin() + (long)best);
-            return p;
-        }
+    std::unique_lock<std::mutex> lk(c->pool_mu);
+    size_t best = (size_t)-1;
+    for (size_t i = 0; i < c->pool.size(); ++i)
+        if (c->pool[i].second >= bytes && c->pool[i].second <= 2 * bytes + 4096 &&
+            (best == (size_t)-1 || c->pool[i].second < c->pool[best].second))
+            best = i;
+    if (best != (size_t)-1) {
+        const std::pair<void *, size_t> b = c->pool[best];
+        c->pool_bytes -= b.second;
+        c->pool.erase(c->pool.begin() + (long)best);
+        c->lent.insert(b);
+        return b.first;
     }
+    lk.unlock();
     void *p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError();
-    {   // what the pool keeps may be what is missing
-        std::lock_guard<std::mutex> lk(c->pool_mu);
-        if (c->pool.empty()) return nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {   // what the pool keeps may be what is missing
+        (void)hipGetLastError();
+        lk.lock();
         for (auto &b : c->pool) hipFree(b.first);
         c->pool.clear();
         c->pool_bytes = 0;
+        lk.unlock();
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
     }
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    lk.lock();
+    c->lent.emplace(p, bytes);
     return p;
 }
 
@@ -77,14 +81,22 @@ size_t hb_pool_held(hb_ctx *c)
     return c->pool_bytes;
 }
 
-// Returns a buffer to the pool.  hipFree waits for the whole device, so the
-// pool frees (oldest first) only past 64 buffers or 16 GiB.
-void hb_pool_put(hb_ctx *c, void *p, size_t bytes)
+// Returns a buffer to the pool; one larger than `keep` goes back to the device.
+// hipFree waits for the whole device, so the pool frees (oldest first) only past
+// 64 buffers or 16 GiB.
+void hb_pool_put(hb_ctx *c, void *p, size_t keep)
 {
     if (!p) return;
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    c->pool.emplace_back(p, bytes);
-    c->pool_bytes += bytes;
+    const auto b = c->lent.find(p);
+    if (b == c->lent.end() || b->second > keep) {
+        if (b != c->lent.end()) c->lent.erase(b);
+        hipFree(p);
+        return;
+    }
+    c->pool.push_back(*b);
+    c->pool_bytes += b->second;
+    c->lent.erase(b);
     while (c->pool.size() > 64 || c->pool_bytes > ((size_t)16 << 30)) {
         hipFree(c->pool.front().first);
         c->pool_bytes -= c->pool.front().second;
@@ -97,17 +109,12 @@ void hb_pool_put(hb_ctx *c, void *p, size_t bytes)
 // MB.  Large ones go back to the device.
 static constexpr size_t kDbKeep = (size_t)1 << 30;
 template <class T>
-static bool db_get(hb_ctx *c, T **p, size_t *held, size_t bytes)
+static bool db_get(hb_ctx *c, T **p, size_t bytes)
 {
     *p = static_cast<T *>(hb_pool_get(c, bytes));
-    *held = bytes;
     return *p != nullptr;
 }
-static void db_put(hb_ctx *c, void *p, size_t bytes)
-{
-    if (bytes > kDbKeep) hipFree(p);
-    else hb_pool_put(c, p, bytes);
-}
+static void db_put(hb_ctx *c, void *p) { hb_pool_put(c, p, kDbKeep); }
 
 void *hb_pin_get(hb_ctx *c, size_t *bytes)
 {
@@ -398,8 +405,8 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 void hb_group_set_free(hb_group_set *g)
 {
     if (!g || !g->ctx) return;
-    hb_pool_put(g->ctx, g->d_fixed, g->fixed_bytes);
-    hb_pool_put(g->ctx, g->d_entries, g->entries_bytes);
+    hb_pool_put(g->ctx, g->d_fixed);
+    hb_pool_put(g->ctx, g->d_entries);
     g->d_desc = nullptr;
     g->d_fixed = nullptr;
     g->d_entries = nullptr;
@@ -554,7 +561,7 @@ int hb_group_set_build(hb_ctx *c, const std::vector<hb_concat> &qs,
         need += out->n_entries[g];
     }
     if (!fits) {
-        hb_pool_put(c, out->d_entries, out->entries_bytes);
+        hb_pool_put(c, out->d_entries);
         out->entries_bytes = need * sizeof(uint32_t);
         out->d_entries = static_cast<uint32_t *>(hb_pool_get(c, out->entries_bytes));
         if (!out->d_entries) return done(HB_ERR_NOMEM);
@@ -712,7 +719,6 @@ struct hb_scan {
     float gap_ms = 0.f;        // device time of the last gapped stage
     uint32_t gap_wide = 0;     // subjects it ran in the wide pass
     uint32_t *d_gstate = nullptr;   // per-wavefront diagonal words (long queries)
-    size_t gstate_bytes = 0;
     int place = HB_PLACE_LDS;      // where this scan keeps the diagonal state
 };
 
@@ -871,12 +877,12 @@ int hb_db_free(hb_db *db)
     hipSetDevice(db->ctx->device);
     hipDeviceSynchronize();   // work that reads it, on any stream
     hb_ctx *c = db->ctx;
-    hb_pool_put(c, db->load_scratch, db->load_bytes);
-    db_put(c, db->d_res, db->res_bytes);
-    db_put(c, db->d_offs, db->offs_bytes);
-    db_put(c, db->d_subj, db->subj_bytes);
-    db_put(c, db->d_scan_alloc, db->alloc_bytes);
-    db_put(c, db->d_tiles, db->tiles_bytes);
+    hb_pool_put(c, db->load_scratch);
+    db_put(c, db->d_res);
+    db_put(c, db->d_offs);
+    db_put(c, db->d_subj);
+    db_put(c, db->d_scan_alloc);
+    db_put(c, db->d_tiles);
     delete db;
     return HB_OK;
 }
@@ -974,12 +980,11 @@ static int db_meta(hb_db *db)
     std::vector<uint32_t> tiles;
     db->n_tiles = cut_tiles(runs, db->total, waves, false, 0, &tiles);
     db->n_qtiles = cut_tiles(runs, db->total, waves, true, want_min, &tiles);
-    if (!db_get(c, &db->d_offs, &db->offs_bytes, ((size_t)n + 1) * sizeof(uint64_t)) ||
-        !db_get(c, &db->d_subj, &db->subj_bytes, (size_t)std::max<uint32_t>(n, 1) * sizeof(uint4)) ||
-        !db_get(c, &db->d_tiles, &db->tiles_bytes, tiles.size() * sizeof(uint32_t)))
+    if (!db_get(c, &db->d_offs, ((size_t)n + 1) * sizeof(uint64_t)) ||
+        !db_get(c, &db->d_subj, (size_t)std::max<uint32_t>(n, 1) * sizeof(uint4)) ||
+        !db_get(c, &db->d_tiles, tiles.size() * sizeof(uint32_t)))
         return HB_ERR_NOMEM;
-    db->load_bytes = hb_load_scratch(n);
-    db->load_scratch = hb_pool_get(c, db->load_bytes);   // until the stream is waited for
+    db->load_scratch = hb_pool_get(c, hb_load_scratch(n));   // until the stream is waited for
     if (!db->load_scratch) return HB_ERR_NOMEM;
     hb_load_args a{};
     a.offs = db->d_offs;
@@ -1003,7 +1008,7 @@ static int db_scan_copy(hb_db *db)
     // the flag, then the copy; padding bytes after subjects read as 0 (the
     // staged copies hold them past each subject's end)
     constexpr size_t kHead = 256;
-    if (!db_get(c, &db->d_scan_alloc, &db->alloc_bytes, kHead + db->scan_bytes + 64))
+    if (!db_get(c, &db->d_scan_alloc, kHead + db->scan_bytes + 64))
         return HB_ERR_NOMEM;
     uint8_t *d = db->d_scan_alloc;
     db->d_scan_res = d + kHead;
@@ -1023,7 +1028,7 @@ static int db_scan_copy(hb_db *db)
             hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return HB_ERR_DEVICE;
-    hb_pool_put(c, db->load_scratch, db->load_bytes);
+    hb_pool_put(c, db->load_scratch);
     db->load_scratch = nullptr;
     return flag ? HB_ERR_RESIDUE : HB_OK;
 }
@@ -1052,7 +1057,7 @@ int hb_db_upload(hb_ctx *c, const uint8_t *residues, const uint64_t *offsets, ui
         hb_db_free(db);
         return r;
     };
-    if (!db_get(c, &db->d_res, &db->res_bytes, db->total + 64)) return fail(HB_ERR_NOMEM);
+    if (!db_get(c, &db->d_res, db->total + 64)) return fail(HB_ERR_NOMEM);
     // the records are made while the residues travel
     Upload up;
     up.start(c, db->d_res, residues ? residues + first : nullptr, db->total);
@@ -1100,16 +1105,12 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
     int32_t *d_glen = nullptr;
     uint32_t *d_lens = nullptr, *d_bad = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    const size_t ng1 = (size_t)std::max(n_groups, 1);
-    const size_t b_hdb = std::max<uint64_t>(bytes, 4), b_gbase = ng1 * sizeof(uint64_t);
-    const size_t b_glen = ng1 * sizeof(int32_t);
-    const size_t b_lens = (size_t)std::max(n_seqs, 1) * sizeof(uint32_t);
     auto release = [&]() {   // after a wait for the stream
-        db_put(c, d_hdb, b_hdb);
-        db_put(c, d_gbase, b_gbase);
-        db_put(c, d_glen, b_glen);
-        db_put(c, d_lens, b_lens);
-        db_put(c, d_bad, 64);
+        db_put(c, d_hdb);
+        db_put(c, d_gbase);
+        db_put(c, d_glen);
+        db_put(c, d_lens);
+        db_put(c, d_bad);
         for (hipEvent_t &e : ev)
             if (e) hipEventDestroy(e);
     };
@@ -1121,12 +1122,12 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
     };
     for (hipEvent_t &e : ev)
         if (hipEventCreate(&e) != hipSuccess) return fail(HB_ERR_DEVICE);
-    d_hdb = static_cast<uint8_t *>(hb_pool_get(c, b_hdb));
-    d_gbase = static_cast<uint64_t *>(hb_pool_get(c, b_gbase));
-    d_glen = static_cast<int32_t *>(hb_pool_get(c, b_glen));
-    d_lens = static_cast<uint32_t *>(hb_pool_get(c, b_lens));
-    d_bad = static_cast<uint32_t *>(hb_pool_get(c, 64));
-    if (!d_hdb || !d_gbase || !d_glen || !d_lens || !d_bad) return fail(HB_ERR_NOMEM);
+    const size_t ng1 = (size_t)std::max(n_groups, 1);
+    if (!db_get(c, &d_hdb, std::max<uint64_t>(bytes, 4)) ||
+        !db_get(c, &d_gbase, ng1 * sizeof(uint64_t)) || !db_get(c, &d_glen, ng1 * sizeof(int32_t)) ||
+        !db_get(c, &d_lens, (size_t)std::max(n_seqs, 1) * sizeof(uint32_t)) ||
+        !db_get(c, &d_bad, 64))
+        return fail(HB_ERR_NOMEM);
     Upload up;
     up.start(c, d_hdb, hdb, bytes);
     if (up.finish() != HB_OK ||
@@ -1155,7 +1156,7 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
     db->h_offs[0] = 0;
     for (int32_t i = 0; i < n_seqs; ++i) db->h_offs[i + 1] = db->h_offs[i] + lens[i];
     db->total = db->h_offs[n_seqs];
-    if (!db_get(c, &db->d_res, &db->res_bytes, db->total + 64)) return fail(HB_ERR_NOMEM);
+    if (!db_get(c, &db->d_res, db->total + 64)) return fail(HB_ERR_NOMEM);
     int rc = db_meta(db);
     if (rc != HB_OK) return fail(rc);
     a.offs = db->d_offs;
@@ -1412,9 +1413,8 @@ static int launch_scan(hb_scan *s)
                             q->gs.diag_len_max, db->n_qtiles << q->gs.desc[0].shift, &cfg, place);
     if (rc) return rc;
     if (place == HB_PLACE_GLOBAL && !s->d_gstate) {
-        s->gstate_bytes =
-            (size_t)cfg.blocks * cfg.waves * (size_t)q->gs.diag_len_max * HB_GSTATE_WORD;
-        s->d_gstate = static_cast<uint32_t *>(hb_pool_get(c, s->gstate_bytes));
+        s->d_gstate = static_cast<uint32_t *>(hb_pool_get(
+            c, (size_t)cfg.blocks * cfg.waves * (size_t)q->gs.diag_len_max * HB_GSTATE_WORD));
         if (!s->d_gstate) return HB_ERR_NOMEM;
     }
     hb_scan_args a;
@@ -1638,10 +1638,10 @@ int hb_scan_free(hb_scan *s)
     if (!s) return HB_ERR_ARG;
     hipSetDevice(s->ctx->device);
     if (!s->waited) hipStreamSynchronize(s->ctx->stream);
-    hb_pool_put(s->ctx, s->d_out, (size_t)s->cap * sizeof(hb_hsp));
-    hb_pool_put(s->ctx, s->d_misc, HB_SCAN_MISC_WORDS * sizeof(uint32_t));
-    hb_pool_put(s->ctx, s->d_stats, (size_t)std::max<uint32_t>(s->db->n, 1) * 3 * sizeof(uint32_t));
-    if (s->d_gstate) hb_pool_put(s->ctx, s->d_gstate, s->gstate_bytes);
+    hb_pool_put(s->ctx, s->d_out);
+    hb_pool_put(s->ctx, s->d_misc);
+    hb_pool_put(s->ctx, s->d_stats);
+    if (s->d_gstate) hb_pool_put(s->ctx, s->d_gstate);
     if (s->ev0) hipEventDestroy(s->ev0);
     if (s->ev1) hipEventDestroy(s->ev1);
     delete s;
@@ -1703,7 +1703,7 @@ int hb_scan_wait(hb_scan *s)
         }
         // The kernel counted every HSP but stored only cap: rerun with room
         // for all of them (the stage is deterministic).
-        hb_pool_put(c, s->d_out, (size_t)s->cap * sizeof(hb_hsp));
+        hb_pool_put(c, s->d_out);
         s->cap = n + n / 8 + 1024;
         s->d_out = (hb_hsp *)hb_pool_get(c, (size_t)s->cap * sizeof(hb_hsp));
         if (!s->d_out) {
@@ -1753,10 +1753,10 @@ int hb_scan_results(hb_scan *s, hb_subject_stats *stats, hb_hsp *hsps, uint64_t 
     auto *d_scr = static_cast<uint32_t *>(hb_pool_get(c, b_scr));
     auto *d_big = static_cast<hb_fin_big *>(hb_pool_get(c, b_big));
     auto release = [&]() {
-        hb_pool_put(c, d_st, b_st);
-        hb_pool_put(c, d_rec, b_rec);
-        hb_pool_put(c, d_scr, b_scr);
-        hb_pool_put(c, d_big, b_big);
+        hb_pool_put(c, d_st);
+        hb_pool_put(c, d_rec);
+        hb_pool_put(c, d_scr);
+        hb_pool_put(c, d_big);
     };
     if (!d_st || !d_rec || !d_scr || !d_big) {
         release();
@@ -1849,11 +1849,11 @@ int hb_scan_results_compact(hb_scan *s, hb_subject_hits *subj, uint64_t subj_cap
     auto *d_big = static_cast<hb_fin_big *>(hb_pool_get(c, b_big));
     auto *d_small = static_cast<hb_fin_small *>(hb_pool_get(c, b_small));
     auto release = [&]() {
-        hb_pool_put(c, d_sub, b_sub);
-        hb_pool_put(c, d_rec, b_rec);
-        hb_pool_put(c, d_scr, b_scr);
-        hb_pool_put(c, d_big, b_big);
-        hb_pool_put(c, d_small, b_small);
+        hb_pool_put(c, d_sub);
+        hb_pool_put(c, d_rec);
+        hb_pool_put(c, d_scr);
+        hb_pool_put(c, d_big);
+        hb_pool_put(c, d_small);
     };
     if (!d_sub || !d_rec || !d_scr || !d_big || !d_small) {
         release();
@@ -1967,13 +1967,13 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
     const uint32_t ns = db->n;
     const int32_t n_ctx = (int32_t)ctx_off.size();
     // pool buffers, all returned at the end
-    std::vector<std::pair<void *, size_t>> held;
+    std::vector<void *> held;
     bool oom = false;
     auto get = [&](size_t bytes) -> void * {
         bytes = std::max<size_t>(bytes, 64);
         void *p = hb_pool_get(c, bytes);
         if (!p) oom = true;
-        else held.emplace_back(p, bytes);
+        else held.push_back(p);
         return p;
     };
     constexpr uint32_t kBig = 4096;
@@ -2000,7 +2000,7 @@ static int gapped_core(hb_ctx *c, const hb_db *db, const uint8_t *d_query, const
         get(pair ? (HB_QUEUE_WORDS + 1 + (size_t)ns) * sizeof(uint32_t) : 0));
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     auto release = [&]() {
-        for (auto &h : held) hb_pool_put(c, h.first, h.second);
+        for (void *p : held) hb_pool_put(c, p);
         for (hipEvent_t e : ev)
             if (e) hipEventDestroy(e);
     };
@@ -2204,8 +2204,8 @@ int hb_gapped_search(hb_ctx *c, hb_db *db, const uint8_t *seq, int32_t len, int3
     auto *d_in = static_cast<uint8_t *>(hb_pool_get(c, b_in));
     auto *d_st3 = static_cast<uint32_t *>(hb_pool_get(c, b_st3));
     auto release = [&]() {
-        hb_pool_put(c, d_in, b_in);
-        hb_pool_put(c, d_st3, b_st3);
+        hb_pool_put(c, d_in);
+        hb_pool_put(c, d_st3);
     };
     if (!d_in || !d_st3) {
         release();

@@ -213,6 +213,43 @@ void handled_errors()
     hb_db_free(db);
 }
 
+// Buffers keep their sizes in the pool whatever they served: databases of
+// alternating sizes take no more memory after the first round of them, and the
+// pool's bytes are the device's.
+void pool_sizes()
+{
+    Fixture f;
+    // of three buffers asked for in turn the first serves the second
+    void *a = hb_pool_get(f.c, 1000000);
+    hb_pool_put(f.c, a);
+    void *b = hb_pool_get(f.c, 600000);
+    CHECK(a == b && hb_pool_held(f.c) == 0);
+    hb_pool_put(f.c, b);
+    CHECK(hb_pool_held(f.c) == 1000000);
+    b = hb_pool_get(f.c, 1000000);
+    CHECK(a == b);
+    hb_pool_put(f.c, b);
+    // a limit on what is kept applies to the buffer's own size
+    b = hb_pool_get(f.c, 600000);
+    hb_pool_put(f.c, b, 700000);
+    CHECK(hb_pool_held(f.c) == 0 && fake_device_size(a) == 0);
+    int mallocs = 0;
+    for (int round = 0; round < 4; ++round) {
+        for (uint32_t n : {90000u, 50000u, 90000u, 60000u}) hb_db_free(f.database(n, 100));
+        CHECK(hb_pool_held(f.c) == g_fake.device_used);
+        if (round) CHECK(g_fake.mallocs == mallocs);
+        mallocs = g_fake.mallocs;
+    }
+    // past 16 GiB the oldest go, by their own sizes
+    std::vector<void *> p;
+    for (int i = 0; i < 20; ++i) p.push_back(hb_pool_get(f.c, (size_t)1 << 30));
+    for (void *x : p) hb_pool_put(f.c, x);
+    CHECK(hb_pool_held(f.c) <= (size_t)16 << 30 && hb_pool_held(f.c) == g_fake.device_used);
+    for (int i = 0; i < 16; ++i) p[i] = hb_pool_get(f.c, (size_t)6 << 27);
+    for (int i = 0; i < 16; ++i) hb_pool_put(f.c, p[i]);
+    CHECK(hb_pool_held(f.c) <= (size_t)16 << 30 && hb_pool_held(f.c) == g_fake.device_used);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -220,6 +257,7 @@ const struct {
     {"failed_collect", failed_collect},
     {"failed_calls_wait", failed_calls_wait},
     {"handled_errors", handled_errors},
+    {"pool_sizes", pool_sizes},
 };
 
 }  // namespace

@@ -57,3 +57,7 @@ def test_failed_call_waits_for_its_work(driver):
 
 def test_handled_errors_are_cleared(driver):
     run(driver, "handled_errors")
+
+
+def test_pool_keeps_buffer_sizes(driver):
+    run(driver, "pool_sizes")
