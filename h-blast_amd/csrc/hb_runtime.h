@@ -23,6 +23,12 @@ void hb_note_hip_error(hipError_t e, const char *what, int line);
 
 extern const int8_t kHbBlosum62[HB_ALPHA][HB_ALPHA];
 
+struct hb_pool_buf {
+    void *p;
+    size_t bytes;
+    bool db;   // was a database's
+};
+
 struct hb_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -32,9 +38,9 @@ struct hb_ctx {
     // Device buffers of finished scans, reused by later scans so that a
     // per-query loop does not pay hipMalloc/hipFree per call.
     std::mutex pool_mu;
-    std::vector<std::pair<void *, size_t>> pool;   // kept buffers and their sizes
-    size_t pool_bytes = 0;
-    std::unordered_map<void *, size_t> lent;       // ... those handed out
+    std::vector<hb_pool_buf> pool;
+    size_t pool_bytes = 0, pool_db_bytes = 0;   // of all buffers, of databases'
+    std::unordered_map<void *, size_t> lent;    // sizes of the buffers handed out
     // pinned host staging for result copies (grown on demand, kept)
     std::mutex pinned_mu;
     void *pinned = nullptr;
@@ -59,7 +65,7 @@ void hb_pin_put(hb_ctx *c, void *p, size_t bytes);
 // Buffers of the pool; one that nothing on the device uses any more goes back
 // to it.  hb_pool_held: the bytes that it keeps.
 void *hb_pool_get(hb_ctx *c, size_t bytes);
-void hb_pool_put(hb_ctx *c, void *p, size_t keep = (size_t)-1);
+void hb_pool_put(hb_ctx *c, void *p, bool db = false);
 size_t hb_pool_held(hb_ctx *c);
 
 struct hb_db {

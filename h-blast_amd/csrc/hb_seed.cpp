@@ -36,41 +36,65 @@ const int8_t kHbBlosum62[HB_ALPHA][HB_ALPHA] = {
 #include "hb_blosum62.inc"
 };
 
+// The contexts that there are: what one of them keeps is there for the others.
+static std::mutex g_ctx_mu;
+static std::vector<hb_ctx *> g_ctxs;
+
+// Frees buffer i of the pool.
+static void pool_drop(hb_ctx *c, size_t i)
+{
+    const hb_pool_buf b = c->pool[i];
+    c->pool_bytes -= b.bytes;
+    if (b.db) c->pool_db_bytes -= b.bytes;
+    c->pool.erase(c->pool.begin() + (long)i);
+    hipFree(b.p);
+}
+
+// hipMalloc; when it fails, again without what the contexts of the device keep.
+// (A failure that is handled must not leave its error: the next launcher would
+// return it.)
+static void *device_alloc(int device, size_t bytes)
+{
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        for (hb_ctx *c : g_ctxs) {
+            if (c->device != device) continue;
+            std::lock_guard<std::mutex> lk2(c->pool_mu);
+            while (!c->pool.empty()) pool_drop(c, c->pool.size() - 1);
+        }
+    }
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // A buffer of at least `bytes` and at most twice that and 4 KB.  The pool keeps
 // the sizes that its buffers have, also while they are handed out: one that
 // served something smaller is as large as before when it comes back.
-// (An allocation that fails and is handled must not leave its error: the next
-// launcher would return it.)
 void *hb_pool_get(hb_ctx *c, size_t bytes)
 {
-    std::unique_lock<std::mutex> lk(c->pool_mu);
-    size_t best = (size_t)-1;
-    for (size_t i = 0; i < c->pool.size(); ++i)
-        if (c->pool[i].second >= bytes && c->pool[i].second <= 2 * bytes + 4096 &&
-            (best == (size_t)-1 || c->pool[i].second < c->pool[best].second))
-            best = i;
-    if (best != (size_t)-1) {
-        const std::pair<void *, size_t> b = c->pool[best];
-        c->pool_bytes -= b.second;
-        c->pool.erase(c->pool.begin() + (long)best);
-        c->lent.insert(b);
-        return b.first;
-    }
-    lk.unlock();
-    void *p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {   // what the pool keeps may be what is missing
-        (void)hipGetLastError();
-        lk.lock();
-        for (auto &b : c->pool) hipFree(b.first);
-        c->pool.clear();
-        c->pool_bytes = 0;
-        lk.unlock();
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(c->pool_mu);
+        size_t best = (size_t)-1;
+        for (size_t i = 0; i < c->pool.size(); ++i)
+            if (c->pool[i].bytes >= bytes && c->pool[i].bytes <= 2 * bytes + 4096 &&
+                (best == (size_t)-1 || c->pool[i].bytes < c->pool[best].bytes))
+                best = i;
+        if (best != (size_t)-1) {
+            const hb_pool_buf b = c->pool[best];
+            c->pool_bytes -= b.bytes;
+            if (b.db) c->pool_db_bytes -= b.bytes;
+            c->pool.erase(c->pool.begin() + (long)best);
+            c->lent.emplace(b.p, b.bytes);
+            return b.p;
         }
     }
-    lk.lock();
+    void *p = device_alloc(c->device, bytes);
+    if (!p) return nullptr;
+    std::lock_guard<std::mutex> lk(c->pool_mu);
     c->lent.emplace(p, bytes);
     return p;
 }
@@ -81,40 +105,42 @@ size_t hb_pool_held(hb_ctx *c)
     return c->pool_bytes;
 }
 
-// Returns a buffer to the pool; one larger than `keep` goes back to the device.
-// hipFree waits for the whole device, so the pool frees (oldest first) only past
-// 64 buffers or 16 GiB.
-void hb_pool_put(hb_ctx *c, void *p, size_t keep)
+// A program that loads one database or volume after the other gets the last
+// one's buffers again: allocating and freeing them took 1.1 ms of a load of 124
+// MB.  What a database held was free for everyone before, so no more than this is
+// kept of databases, oldest first out: a volume of 340 MB, its residues and
+// their copy.
+static constexpr size_t kDbKeep = (size_t)1 << 30;
+
+// Returns a buffer to the pool (db: of a database).  hipFree waits for the whole
+// device, so the pool frees (oldest first) only past 64 buffers or 16 GiB.
+void hb_pool_put(hb_ctx *c, void *p, bool db)
 {
     if (!p) return;
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    const auto b = c->lent.find(p);
-    if (b == c->lent.end() || b->second > keep) {
-        if (b != c->lent.end()) c->lent.erase(b);
+    const auto it = c->lent.find(p);
+    const size_t bytes = it == c->lent.end() ? 0 : it->second;
+    if (bytes) c->lent.erase(it);
+    if (!bytes || (db && bytes > kDbKeep)) {
         hipFree(p);
         return;
     }
-    c->pool.push_back(*b);
-    c->pool_bytes += b->second;
-    c->lent.erase(b);
-    while (c->pool.size() > 64 || c->pool_bytes > ((size_t)16 << 30)) {
-        hipFree(c->pool.front().first);
-        c->pool_bytes -= c->pool.front().second;
-        c->pool.erase(c->pool.begin());
-    }
+    c->pool.push_back(hb_pool_buf{p, bytes, db});
+    c->pool_bytes += bytes;
+    if (db) c->pool_db_bytes += bytes;
+    for (size_t i = 0; c->pool_db_bytes > kDbKeep;)
+        if (c->pool[i].db) pool_drop(c, i);
+        else ++i;
+    while (c->pool.size() > 64 || c->pool_bytes > ((size_t)16 << 30)) pool_drop(c, 0);
 }
 
-// A program that loads one database or volume after the other gets the last
-// one's buffers again: allocating and freeing them took 1.1 ms of a load of 124
-// MB.  Large ones go back to the device.
-static constexpr size_t kDbKeep = (size_t)1 << 30;
 template <class T>
 static bool db_get(hb_ctx *c, T **p, size_t bytes)
 {
     *p = static_cast<T *>(hb_pool_get(c, bytes));
     return *p != nullptr;
 }
-static void db_put(hb_ctx *c, void *p) { hb_pool_put(c, p, kDbKeep); }
+static void db_put(hb_ctx *c, void *p) { hb_pool_put(c, p, true); }
 
 void *hb_pin_get(hb_ctx *c, size_t *bytes)
 {
@@ -811,6 +837,8 @@ int hb_create(int device, hb_ctx **out)
         delete c;
         return HB_ERR_DEVICE;
     }
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    g_ctxs.push_back(c);
     *out = c;
     return HB_OK;
 }
@@ -819,8 +847,12 @@ int hb_destroy(hb_ctx *c)
 {
     if (!c) return HB_ERR_ARG;
     hipSetDevice(c->device);
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        g_ctxs.erase(std::remove(g_ctxs.begin(), g_ctxs.end(), c), g_ctxs.end());
+    }
     if (c->stream) hipStreamSynchronize(c->stream);
-    for (auto &b : c->pool) hipFree(b.first);
+    for (auto &b : c->pool) hipFree(b.p);
     if (c->pinned) hipHostFree(c->pinned);
     for (auto &b : c->pins) hipHostFree(b.first);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -835,7 +867,7 @@ int hb_mem_info(hb_ctx *c, uint64_t *free_b, uint64_t *total_b)
     size_t f = 0, t = 0;
     HB_CHECK(hipSetDevice(c->device));
     HB_CHECK(hipMemGetInfo(&f, &t));
-    if (free_b) *free_b = f;
+    if (free_b) *free_b = f + hb_pool_held(c);
     if (total_b) *total_b = t;
     return HB_OK;
 }
@@ -877,7 +909,7 @@ int hb_db_free(hb_db *db)
     hipSetDevice(db->ctx->device);
     hipDeviceSynchronize();   // work that reads it, on any stream
     hb_ctx *c = db->ctx;
-    hb_pool_put(c, db->load_scratch);
+    db_put(c, db->load_scratch);
     db_put(c, db->d_res);
     db_put(c, db->d_offs);
     db_put(c, db->d_subj);
@@ -1028,7 +1060,7 @@ static int db_scan_copy(hb_db *db)
             hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return HB_ERR_DEVICE;
-    hb_pool_put(c, db->load_scratch);
+    db_put(c, db->load_scratch);
     db->load_scratch = nullptr;
     return flag ? HB_ERR_RESIDUE : HB_OK;
 }
@@ -1483,7 +1515,6 @@ int hb_check_memory(hb_ctx *c, const hb_query *q, uint64_t file_bytes, uint64_t 
         uint64_t total = 0;
         int rc = hb_mem_info(c, &room, &total);
         if (rc) return rc;
-        room += hb_pool_held(c);
     }
     *fits = *need <= room ? 1 : 0;
     return HB_OK;
@@ -2282,8 +2313,7 @@ int hb_diag_copy(hb_ctx *c, uint64_t bytes, int reps, float *ms_per_copy)
     void *a = nullptr, *b = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = HB_OK;
-    if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) {
-        (void)hipGetLastError();
+    if (!(a = device_alloc(c->device, bytes)) || !(b = device_alloc(c->device, bytes))) {
         rc = HB_ERR_NOMEM;
     } else if (hipMemsetAsync(a, 1, bytes, c->stream) != hipSuccess ||
                hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess ||

@@ -281,8 +281,9 @@ int hb_serve_start(hb_ctx *ctx, hb_db *db, const hb_params *params, const hb_ser
     if (o.group_residues == 0) o.group_residues = 768;
     HB_CHECK(hipSetDevice(ctx->device));
     if (o.mem_budget == 0) {
-        size_t fr = 0, tot = 0;
-        HB_CHECK(hipMemGetInfo(&fr, &tot));
+        uint64_t fr = 0;
+        rc = hb_mem_info(ctx, &fr, nullptr);
+        if (rc) return rc;
         o.mem_budget = (int64_t)(fr / 2);
     }
     hb_server *s = new (std::nothrow) hb_server;

@@ -104,7 +104,10 @@ int hb_create(int device, hb_ctx **out);
 int hb_destroy(hb_ctx *ctx);
 /* Free / total device memory in bytes (the served form's admission and
  * hb_check_memory's default budget use it; hb_check_memory is the
- * counterpart of H_BLAST_check_memory, gpu_cpu_common.h:93-102). */
+ * counterpart of H_BLAST_check_memory, gpu_cpu_common.h:93-102).  The buffers
+ * that the context keeps for its next calls count as free: at most 64 buffers
+ * and 16 GiB, of them 1 GiB of freed databases.  They go back to the device
+ * when an allocation of any context on it needs them, and with hb_destroy. */
 int hb_mem_info(hb_ctx *ctx, uint64_t *free_bytes, uint64_t *total_bytes);
 int hb_synchronize(hb_ctx *ctx);
 /* Page-locked host memory (hipHostMalloc) for the arrays a caller hands to

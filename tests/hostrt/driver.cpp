@@ -191,16 +191,16 @@ void handled_errors()
     CHECK(hb_host_alloc(f.c, 64, &p) == HB_ERR_NOMEM);
     CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
     float ms = 0;
-    g_fake.fail_malloc = 1;
+    g_fake.fail_malloc = 2;
     CHECK(hb_diag_copy(f.c, 4096, 1, &ms) == HB_ERR_NOMEM);
     CHECK(hb_scan_results(s, st.data(), hsps.data(), 5, &found_n) == HB_OK);
     // a batch whose order finds no memory orders on the host
     hb_batch *b = f.batch(db, 1);
     CHECK(hb_batch_run(b) == HB_OK);
     f.c->pool_mu.lock();
-    for (auto &x : f.c->pool) (void)hipFree(x.first);
+    for (auto &x : f.c->pool) (void)hipFree(x.p);
     f.c->pool.clear();
-    f.c->pool_bytes = 0;
+    f.c->pool_bytes = f.c->pool_db_bytes = 0;
     f.c->pool_mu.unlock();
     g_fake.fail_malloc = 2;
     CHECK(hb_batch_run(b) == HB_OK);
@@ -229,10 +229,6 @@ void pool_sizes()
     b = hb_pool_get(f.c, 1000000);
     CHECK(a == b);
     hb_pool_put(f.c, b);
-    // a limit on what is kept applies to the buffer's own size
-    b = hb_pool_get(f.c, 600000);
-    hb_pool_put(f.c, b, 700000);
-    CHECK(hb_pool_held(f.c) == 0 && fake_device_size(a) == 0);
     int mallocs = 0;
     for (int round = 0; round < 4; ++round) {
         for (uint32_t n : {90000u, 50000u, 90000u, 60000u}) hb_db_free(f.database(n, 100));
@@ -250,6 +246,57 @@ void pool_sizes()
     CHECK(hb_pool_held(f.c) <= (size_t)16 << 30 && hb_pool_held(f.c) == g_fake.device_used);
 }
 
+// What a freed database held is free again: for the memory information, for a
+// server's default budget, for another context; and little of it is kept.
+void freed_memory()
+{
+    const size_t total = g_fake.device_total;
+    Fixture f, other;
+    uint64_t before = 0, after = 0;
+    CHECK(hb_mem_info(f.c, &before, nullptr) == HB_OK);
+    for (uint32_t n : {100000u, 400000u, 50000u}) {
+        hb_db_free(f.database(n, 100));
+        CHECK(hb_mem_info(f.c, &after, nullptr) == HB_OK && after == before);
+        CHECK(hb_pool_held(f.c) == g_fake.device_used);
+    }
+    std::vector<void *> p;
+    for (int i = 0; i < 5; ++i) p.push_back(hb_pool_get(f.c, 300000000));
+    for (void *x : p) hb_pool_put(f.c, x, true);
+    CHECK(hb_pool_held(f.c) == 900000000);   // the last three, and no older ones
+    hb_pool_put(f.c, hb_pool_get(f.c, 1200000000), true);
+    CHECK(hb_pool_held(f.c) == 900000000 && g_fake.device_used == 900000000);
+    CHECK(hb_mem_info(f.c, &after, nullptr) == HB_OK && after == before);
+    // a context that needs what another keeps
+    hb_db_free(f.database(1000000, 100));
+    CHECK(hb_pool_held(f.c) > 200000000);
+    g_fake.device_total = 280000000;
+    hb_db *db = other.database(1000000, 100);
+    CHECK(db && hb_pool_held(f.c) == 0);
+    hb_db_free(db);
+    float ms = 0;
+    CHECK(hb_diag_copy(f.c, 100000000, 1, &ms) == HB_OK);
+    // half the free memory, whatever the context keeps of it
+    g_fake.device_total = 120000000;
+    hb_db_free(f.database(400000, 100));
+    CHECK(hb_pool_held(f.c) > 80000000);
+    db = f.database(1000);
+    found(5);
+    hb_serve_opts o;
+    hb_serve_opts_default(&o);
+    o.hsp_per_cell = 30e6 / 32 / (100 * 16000.0);   // about 31 MB for the request
+    hb_server *s = nullptr;
+    CHECK(hb_serve_start(f.c, db, nullptr, &o, &s) == HB_OK);
+    const std::vector<uint8_t> seq(100, 1);
+    const int32_t off = 0, len = 100, x = 16, cut = 41;
+    uint64_t t = 0, n = 0;
+    CHECK(hb_serve_submit(s, seq.data(), len, 1, &off, &len, &x, &cut, &t) == HB_OK);
+    CHECK(hb_serve_wait(s, t, -1) == HB_OK);
+    CHECK(hb_serve_results(s, t, nullptr, 0, &n) == HB_OK && n == 5);
+    hb_serve_stop(s);
+    hb_db_free(db);
+    g_fake.device_total = total;
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -258,6 +305,7 @@ const struct {
     {"failed_calls_wait", failed_calls_wait},
     {"handled_errors", handled_errors},
     {"pool_sizes", pool_sizes},
+    {"freed_memory", freed_memory},
 };
 
 }  // namespace

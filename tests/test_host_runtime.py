@@ -61,3 +61,7 @@ def test_handled_errors_are_cleared(driver):
 
 def test_pool_keeps_buffer_sizes(driver):
     run(driver, "pool_sizes")
+
+
+def test_freed_databases_are_free_memory(driver):
+    run(driver, "freed_memory")
