@@ -142,37 +142,45 @@ static bool db_get(hb_ctx *c, T **p, size_t bytes)
 }
 static void db_put(hb_ctx *c, void *p) { hb_pool_put(c, p, true); }
 
+// The smallest page-locked buffer that holds the request, unless it is more than
+// four times as large as one made for it: a small request must not sit on the
+// buffer of the next load (a batch holds its own as long as it lives).
 void *hb_pin_get(hb_ctx *c, size_t *bytes)
 {
+    const size_t want = (std::max<size_t>(*bytes, 1) + 0x3ffff) & ~(size_t)0x3ffff;
     {
         std::lock_guard<std::mutex> lk(c->pin_mu);
+        size_t best = (size_t)-1;
         for (size_t i = 0; i < c->pins.size(); ++i)
-            if (c->pins[i].second >= *bytes) {
-                void *p = c->pins[i].first;
-                *bytes = c->pins[i].second;
-                c->pins.erase(c->pins.begin() + (long)i);
-                return p;
-            }
+            if (c->pins[i].second >= *bytes && c->pins[i].second <= 4 * want &&
+                (best == (size_t)-1 || c->pins[i].second < c->pins[best].second))
+                best = i;
+        if (best != (size_t)-1) {
+            void *p = c->pins[best].first;
+            *bytes = c->pins[best].second;
+            c->pins.erase(c->pins.begin() + (long)best);
+            return p;
+        }
     }
-    *bytes = (*bytes + 0x3ffff) & ~(size_t)0x3ffff;
     void *p = nullptr;
-    if (hipHostMalloc(&p, *bytes, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
+    *bytes = want;
     return p;
 }
 
-// At most 8 buffers of up to 16 MiB are kept.
+// At most 8 buffers of up to 16 MiB are kept, the last ones put back.
 void hb_pin_put(hb_ctx *c, void *p, size_t bytes)
 {
     if (!p) return;
-    {
+    if (bytes <= ((size_t)16 << 20)) {
         std::lock_guard<std::mutex> lk(c->pin_mu);
-        if (c->pins.size() < 8 && bytes <= ((size_t)16 << 20)) {
-            c->pins.emplace_back(p, bytes);
-            return;
-        }
+        c->pins.emplace_back(p, bytes);
+        if (c->pins.size() <= 8) return;
+        p = c->pins.front().first;
+        c->pins.erase(c->pins.begin());
     }
     hipHostFree(p);
 }

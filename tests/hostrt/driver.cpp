@@ -297,6 +297,47 @@ void freed_memory()
     g_fake.device_total = total;
 }
 
+// Page-locked buffers: a small request leaves a large one alone, the smallest
+// that fits is taken, and the buffers kept stay within their bounds.
+void pinned_buffers()
+{
+    Fixture f;
+    hb_db *db = f.database(20000, 300);   // leaves the upload's 16 MiB
+    found(5);
+    hb_batch *b = f.batch(db, 1);
+    CHECK(hb_batch_run(b) == HB_OK);      // holds a small one
+    int n = g_fake.host_mallocs;
+    hb_db *db2 = f.database(20000, 300);
+    CHECK(g_fake.host_mallocs == n);
+    auto get = [&](size_t bytes) {
+        std::pair<void *, size_t> r(nullptr, bytes);
+        r.first = hb_pin_get(f.c, &r.second);
+        CHECK(r.first && r.second >= bytes && fake_host_size(r.first) == r.second);
+        return r;
+    };
+    const auto big = get(8 << 20), mid = get(1 << 20);
+    hb_pin_put(f.c, big.first, big.second);
+    hb_pin_put(f.c, mid.first, mid.second);
+    n = g_fake.host_mallocs;
+    const auto one = get(900 << 10);
+    CHECK(one.first == mid.first && g_fake.host_mallocs == n);
+    const auto two = get(5 << 20);
+    CHECK(two.first == big.first && g_fake.host_mallocs == n);
+    hb_pin_put(f.c, one.first, one.second);
+    hb_pin_put(f.c, two.first, two.second);
+    std::vector<std::pair<void *, size_t>> all;
+    for (int i = 0; i < 12; ++i) all.push_back(get(16 << 20));
+    for (const auto &x : all) hb_pin_put(f.c, x.first, x.second);
+    CHECK(f.c->pins.size() == 8 && f.c->pins.back().first == all.back().first);
+    const size_t held = g_fake.host_used;
+    const auto large = get((16 << 20) + 1);
+    hb_pin_put(f.c, large.first, large.second);
+    CHECK(g_fake.host_used == held && f.c->pins.size() == 8);
+    hb_batch_free(b);
+    hb_db_free(db);
+    hb_db_free(db2);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -306,6 +347,7 @@ const struct {
     {"handled_errors", handled_errors},
     {"pool_sizes", pool_sizes},
     {"freed_memory", freed_memory},
+    {"pinned_buffers", pinned_buffers},
 };
 
 }  // namespace

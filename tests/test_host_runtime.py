@@ -65,3 +65,7 @@ def test_pool_keeps_buffer_sizes(driver):
 
 def test_freed_databases_are_free_memory(driver):
     run(driver, "freed_memory")
+
+
+def test_small_requests_leave_large_pinned_buffers(driver):
+    run(driver, "pinned_buffers")
