@@ -192,8 +192,8 @@ void hb_pin_put(hb_ctx *c, void *p, size_t bytes)
 // (the copies then go through the DMA engine at 50 GB/s while the context's
 // stream makes the records).  Whole loads of 36, 108 and 216 MB: 2.16, 6.20 and
 // 12.8 ms before, 1.12, 2.86 and 5.47 ms now; chunks of 2 MB 7% slower, of 1 MB
-// 20%; four threads the same as two.  Memory that is page-locked already travels
-// from where it is; below kMin the threads' start costs what they save (3.6 MB:
+// 20%; four threads the same as two.  Memory that the runtime knows (page-locked,
+// managed, a device's) travels from where it is; below kMin the threads' start costs what they save (3.6 MB:
 // 366 us without, 352 us with the rest of it).
 namespace {
 class Upload {
@@ -208,7 +208,7 @@ class Upload {
         if (bytes < kMin) return;
         hipPointerAttribute_t at{};
         if (hipPointerGetAttributes(&at, src) != hipSuccess) (void)hipGetLastError();
-        else if (at.type == hipMemoryTypeHost) return;
+        else if (at.type != hipMemoryTypeUnregistered) return;
         if (!c->up_stream &&
             hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) != hipSuccess) {
             (void)hipGetLastError();

@@ -338,6 +338,28 @@ void pinned_buffers()
     hb_db_free(db2);
 }
 
+// Residues in memory that the runtime knows, page-locked or on the device, are
+// copied by the runtime from where they are and not read by the host.
+void upload_sources()
+{
+    Fixture f;
+    const uint32_t n = 20000, len = 300;
+    std::vector<uint64_t> offs(n + 1);
+    for (uint32_t i = 0; i <= n; ++i) offs[i] = (uint64_t)i * len;
+    void *host = nullptr, *device = nullptr;
+    CHECK(hipHostMalloc(&host, n * len, 0) == hipSuccess && hipMalloc(&device, n * len) == hipSuccess);
+    for (void *src : {host, device}) {
+        memset(src, 1, n * len);
+        const int copies = g_fake.host_to_device, mallocs = g_fake.host_mallocs;
+        hb_db *db = nullptr;
+        CHECK(hb_db_upload(f.c, static_cast<const uint8_t *>(src), offs.data(), n, &db) == HB_OK);
+        CHECK(g_fake.host_to_device == copies + 3 && g_fake.host_mallocs == mallocs);
+        hb_db_free(db);
+    }
+    (void)hipHostFree(host);
+    (void)hipFree(device);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -348,6 +370,7 @@ const struct {
     {"pool_sizes", pool_sizes},
     {"freed_memory", freed_memory},
     {"pinned_buffers", pinned_buffers},
+    {"upload_sources", upload_sources},
 };
 
 }  // namespace

@@ -69,3 +69,7 @@ def test_freed_databases_are_free_memory(driver):
 
 def test_small_requests_leave_large_pinned_buffers(driver):
     run(driver, "pinned_buffers")
+
+
+def test_uploads_from_memory_the_runtime_knows(driver):
+    run(driver, "upload_sources")
