@@ -1586,12 +1586,12 @@ __global__ __launch_bounds__(kFinThreads) void fin_write_kernel(const uint32_t *
     for (int k = 0; k < kFinPer; ++k) {
         const uint32_t i = i0 + k;
         if (i < ns) {
-            hb_subject_stats o;
-            o.lookup_hits = st3[3 * (size_t)i];
-            o.extensions = st3[3 * (size_t)i + 1];
-            o.n_hsp = cnt[k];
-            o.first = cnt[k] ? (int64_t)first : -1;
-            out[i] = o;
+            // (as words: the structure's padding is 0, not what the buffer held)
+            static_assert(sizeof(hb_subject_stats) == 24 && offsetof(hb_subject_stats, first) == 16);
+            uint2 *o = reinterpret_cast<uint2 *>(out + i);
+            o[0] = make_uint2(st3[3 * (size_t)i], st3[3 * (size_t)i + 1]);
+            o[1] = make_uint2(cnt[k], 0u);
+            o[2] = cnt[k] ? make_uint2(first, 0u) : make_uint2(~0u, ~0u);
             cursor[i] = first;
         }
         first += cnt[k];
