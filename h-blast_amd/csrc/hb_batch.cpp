@@ -518,7 +518,9 @@ static int collect_host(hb_batch *b, uint32_t n)
 
 // Orders the n records of the last pass on the device, mapped to their
 // queries' contexts and offsets, and fetches them with the per-group counters.
-static int collect(hb_batch *b, uint32_t n)
+// The order takes 56 bytes a record beside the pass's 32: past `room` bytes (set
+// to what was taken) the host orders them.
+static int collect(hb_batch *b, uint32_t n, size_t *room)
 {
     hb_ctx *c = b->ctx;
     const size_t nq = b->queries.size(), ng = b->gs.desc.size(), nc = b->ctx_query.size();
@@ -541,7 +543,8 @@ static int collect(hb_batch *b, uint32_t n)
     for (size_t k = 0; k < nc; ++k)
         map[k] = make_int4(b->ctx_query[k], b->ctx_local[k], b->q_base[b->ctx_query[k]], 0);
     const size_t scr_b = n ? hb_sort_scratch(n) : 0, dev_b = up16(map_b) + up16(first_b) + rec_b + scr_b;
-    char *dev = n ? static_cast<char *>(hb_pool_get(c, dev_b)) : nullptr;
+    char *dev = n && dev_b <= *room ? static_cast<char *>(hb_pool_get(c, dev_b)) : nullptr;
+    *room = dev ? dev_b : 0;
     if (n && !dev) return collect_host(b, n);
     hipError_t e = hipMemcpyAsync(pin + o_tot, b->d_totals, tot_b, hipMemcpyDeviceToHost, b->st);
     hb_order_args a{};
@@ -662,8 +665,9 @@ bool hb_batch_ready(hb_batch *b)
 }
 
 // Waits for the launched pass, reruns it once with a larger buffer when
-// the records did not fit, and collects the results.
-int hb_batch_finish(hb_batch *b)
+// the records did not fit, and collects the results with at most *room bytes of
+// device memory more (set to what it took).
+int hb_batch_finish(hb_batch *b, size_t *room)
 {
     if (!b) return HB_ERR_ARG;
     if (!b->launched) return HB_ERR_STATE;
@@ -680,7 +684,7 @@ int hb_batch_finish(hb_batch *b)
         rc = run_pass(b, 0, b->db->n_tiles, false, &n);
         if (rc) return rc;
     }
-    return collect(b, n);
+    return collect(b, n, room);
 }
 
 bool hb_batch_rerun_needed(const hb_batch *b) { return b->reran; }
@@ -773,7 +777,8 @@ int hb_batch_run(hb_batch *b)
     uint32_t n = 0;
     rc = run_pass(b, 0, b->db->n_tiles, b->o.use_graph != 0, &n);
     if (rc) return rc;
-    return collect(b, n);
+    size_t room = (size_t)-1;
+    return collect(b, n, &room);
 }
 
 int hb_batch_results(hb_batch *b, int32_t query_id, hb_hsp *hsps, uint64_t cap, uint64_t *n_hsp)

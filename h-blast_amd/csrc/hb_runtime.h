@@ -184,13 +184,14 @@ static inline int32_t hb_diag_len(int32_t qlen, int32_t window, int32_t shift)
 // Asynchronous steps of a batch (hb_batch.cpp), used by the serving loop:
 // the batch runs on the given stream (nullptr: the context's); launch
 // returns at once, ready polls, finish collects (rerunning the pass if the
-// HSP buffer was too small).
+// HSP buffer was too small) with at most *room bytes of device memory for the
+// records' order, and sets it to what that took.
 struct hb_batch;
 int hb_batch_create_on(hb_ctx *ctx, hb_db *db, const hb_params *params, const hb_batch_opts *opts,
                        hipStream_t st, hb_batch **out);
 bool hb_batch_rerun_needed(const hb_batch *b);
 int hb_batch_launch(hb_batch *b);
 bool hb_batch_ready(hb_batch *b);
-int hb_batch_finish(hb_batch *b);
+int hb_batch_finish(hb_batch *b, size_t *room);
 size_t hb_batch_device_bytes(const hb_batch *b);
 int hb_batch_reserve(hb_batch *b, uint32_t cap);

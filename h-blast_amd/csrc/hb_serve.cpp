@@ -229,7 +229,18 @@ static void loop(hb_server *s)
                 ++i;
                 continue;
             }
-            const int rc = hb_batch_finish(f.b);
+            // the records' order within what the budget leaves (nothing is
+            // admitted meanwhile)
+            size_t order;
+            {
+                std::lock_guard<std::mutex> lk(s->mu);
+                order = (size_t)s->o.mem_budget - s->bytes_admitted;
+            }
+            const int rc = hb_batch_finish(f.b, &order);
+            if (rc == HB_OK) {
+                std::lock_guard<std::mutex> lk(s->mu);
+                s->st.peak_bytes = std::max<uint64_t>(s->st.peak_bytes, s->bytes_admitted + order);
+            }
             finish_requests(s, f, rc);
             hb_batch_free(f.b);
             s->inflight.erase(s->inflight.begin() + (long)i);

@@ -360,6 +360,42 @@ void upload_sources()
     (void)hipFree(device);
 }
 
+// A served batch orders its records within the budget: on the device when that
+// leaves room, on the host otherwise.
+void served_order()
+{
+    Fixture f;
+    hb_db *db = f.database(20000);
+    const uint32_t n = 20000;   // 1.1 MB for their order
+    found(n);
+    const std::vector<uint8_t> seq(100, 1);
+    const int32_t off = 0, len = 100, x = 16, cut = 41;
+    for (int64_t room : {1 << 14, 1 << 24}) {
+        hb_serve_opts o;
+        hb_serve_opts_default(&o);
+        o.hsp_per_cell = 20000 / (100.0 * 320000);
+        o.max_inflight = 1;
+        // the request's estimate (records, tables, entries) and `room`
+        o.mem_budget = (20000 + 256) * 32 + 32768 * 8 + 4096 + 4096 + 8192 + 64 * 4 * 100 + room;
+        hb_server *s = nullptr;
+        CHECK(hb_serve_start(f.c, db, nullptr, &o, &s) == HB_OK);
+        const int orders = g_fake.orders;
+        uint64_t t = 0, k = 0;
+        CHECK(hb_serve_submit(s, seq.data(), len, 1, &off, &len, &x, &cut, &t) == HB_OK);
+        CHECK(hb_serve_wait(s, t, -1) == HB_OK);
+        std::vector<hb_hsp> got(n);
+        CHECK(hb_serve_results(s, t, got.data(), n, &k) == HB_OK && k == n && got[n - 1].oid == n - 1);
+        hb_serve_stats st;
+        CHECK(hb_serve_stats_get(s, &st) == HB_OK);
+        CHECK(st.peak_bytes <= (uint64_t)o.mem_budget);
+        const bool device = room > (1 << 20);
+        CHECK((g_fake.orders != orders) == device);
+        CHECK((st.peak_bytes > (uint64_t)(o.mem_budget - room)) == device);
+        hb_serve_stop(s);
+    }
+    hb_db_free(db);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -371,6 +407,7 @@ const struct {
     {"freed_memory", freed_memory},
     {"pinned_buffers", pinned_buffers},
     {"upload_sources", upload_sources},
+    {"served_order", served_order},
 };
 
 }  // namespace

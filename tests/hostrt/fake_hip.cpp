@@ -303,6 +303,7 @@ hipError_t hb_launch_load_records(hb_load_args a, void *, hipStream_t st)
 hipError_t hb_launch_load_copy(const hb_load_args &, uint64_t, hipStream_t st) { return launched(st); }
 hipError_t hb_launch_order(hb_order_args a, void *, hipStream_t st)
 {
+    ++g_fake.orders;
     for (int32_t q = 0; q <= a.n_queries; ++q) a.q_first[q] = q ? a.n : 0;
     memcpy(a.out, a.in, a.n * sizeof(*a.out));
     const hipError_t e = launched(st);

@@ -28,6 +28,7 @@ struct FakeHip {
     std::atomic<int> fail_stream_create{0};
     std::atomic<int> fail_order{0};           // the next n hb_launch_order calls fail
     std::atomic<int> fail_finalize{0};        // ... hb_launch_finalize(_compact) after their work
+    std::atomic<int> orders{0};               // hb_launch_order calls
     std::atomic<int> host_to_device{0};       // synchronous host-to-device copies
     // the HSPs that a scan of one group finds (called by hb_launch_scan)
     std::function<void(const hb_scan_args &)> scan;

@@ -73,3 +73,7 @@ def test_small_requests_leave_large_pinned_buffers(driver):
 
 def test_uploads_from_memory_the_runtime_knows(driver):
     run(driver, "upload_sources")
+
+
+def test_served_batches_order_within_the_budget(driver):
+    run(driver, "served_order")
