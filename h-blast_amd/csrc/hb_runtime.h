@@ -70,6 +70,7 @@ size_t hb_pool_held(hb_ctx *c);
 
 struct hb_db {
     hb_ctx *ctx = nullptr;
+    int device = 0;
     uint32_t n = 0;
     uint64_t total = 0;
     uint8_t *d_res = nullptr;

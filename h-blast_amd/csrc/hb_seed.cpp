@@ -911,18 +911,21 @@ int hb_synchronize(hb_ctx *c)
 }
 
 // ------------------------------------------------------------------ database
+// (Also after the database's context was destroyed: its memory then goes back to
+// the device.)
 int hb_db_free(hb_db *db)
 {
     if (!db) return HB_ERR_ARG;
-    hipSetDevice(db->ctx->device);
+    hipSetDevice(db->device);
     hipDeviceSynchronize();   // work that reads it, on any stream
-    hb_ctx *c = db->ctx;
-    db_put(c, db->load_scratch);
-    db_put(c, db->d_res);
-    db_put(c, db->d_offs);
-    db_put(c, db->d_subj);
-    db_put(c, db->d_scan_alloc);
-    db_put(c, db->d_tiles);
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        const bool kept = std::find(g_ctxs.begin(), g_ctxs.end(), db->ctx) != g_ctxs.end();
+        for (void *p : {db->load_scratch, (void *)db->d_res, (void *)db->d_offs, (void *)db->d_subj,
+                        (void *)db->d_scan_alloc, (void *)db->d_tiles})
+            if (kept) db_put(db->ctx, p);
+            else hipFree(p);
+    }
     delete db;
     return HB_OK;
 }
@@ -1088,6 +1091,7 @@ int hb_db_upload(hb_ctx *c, const uint8_t *residues, const uint64_t *offsets, ui
     hb_db *db = new (std::nothrow) hb_db;
     if (!db) return HB_ERR_NOMEM;
     db->ctx = c;
+    db->device = c->device;
     db->n = n;
     const uint64_t first = n ? offsets[0] : 0;
     db->total = n ? offsets[n] - first : 0;
@@ -1139,6 +1143,7 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
     hb_db *db = new (std::nothrow) hb_db;
     if (!db) return HB_ERR_NOMEM;
     db->ctx = c;
+    db->device = c->device;
     db->n = (uint32_t)n_seqs;
     uint8_t *d_hdb = nullptr;
     uint64_t *d_gbase = nullptr;

@@ -396,6 +396,22 @@ void served_order()
     hb_db_free(db);
 }
 
+// A database outlives its context.
+void database_after_context()
+{
+    hb_db *db = nullptr;
+    {
+        Fixture f;
+        db = f.database(1000);
+    }
+    CHECK(g_fake.device_used > 0);
+    CHECK(hb_db_free(db) == HB_OK);
+    CHECK(g_fake.device_used == 0);
+    Fixture f;   // (a context that may stand at the same address)
+    hb_db_free(f.database(1000));
+    CHECK(hb_pool_held(f.c) == g_fake.device_used);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -408,6 +424,7 @@ const struct {
     {"pinned_buffers", pinned_buffers},
     {"upload_sources", upload_sources},
     {"served_order", served_order},
+    {"database_after_context", database_after_context},
 };
 
 }  // namespace

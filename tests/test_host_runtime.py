@@ -77,3 +77,7 @@ def test_uploads_from_memory_the_runtime_knows(driver):
 
 def test_served_batches_order_within_the_budget(driver):
     run(driver, "served_order")
+
+
+def test_database_outlives_its_context(driver):
+    run(driver, "database_after_context")
