@@ -5,7 +5,6 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include "hb_internal.h"
@@ -40,7 +39,7 @@ struct hb_ctx {
     std::mutex pool_mu;
     std::vector<hb_pool_buf> pool;
     size_t pool_bytes = 0, pool_db_bytes = 0;   // of all buffers, of databases'
-    std::unordered_map<void *, size_t> lent;    // sizes of the buffers handed out
+    std::vector<std::pair<void *, size_t>> lent;   // the buffers handed out and their sizes
     // pinned host staging for result copies (grown on demand, kept)
     std::mutex pinned_mu;
     void *pinned = nullptr;

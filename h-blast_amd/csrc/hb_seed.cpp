@@ -88,14 +88,14 @@ void *hb_pool_get(hb_ctx *c, size_t bytes)
             c->pool_bytes -= b.bytes;
             if (b.db) c->pool_db_bytes -= b.bytes;
             c->pool.erase(c->pool.begin() + (long)best);
-            c->lent.emplace(b.p, b.bytes);
+            c->lent.emplace_back(b.p, b.bytes);
             return b.p;
         }
     }
     void *p = device_alloc(c->device, bytes);
     if (!p) return nullptr;
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    c->lent.emplace(p, bytes);
+    c->lent.emplace_back(p, bytes);
     return p;
 }
 
@@ -118,9 +118,13 @@ void hb_pool_put(hb_ctx *c, void *p, bool db)
 {
     if (!p) return;
     std::lock_guard<std::mutex> lk(c->pool_mu);
-    const auto it = c->lent.find(p);
-    const size_t bytes = it == c->lent.end() ? 0 : it->second;
-    if (bytes) c->lent.erase(it);
+    size_t bytes = 0;
+    for (size_t i = c->lent.size(); i-- > 0 && !bytes;)   // (the last ones mostly)
+        if (c->lent[i].first == p) {
+            bytes = c->lent[i].second;
+            c->lent[i] = c->lent.back();
+            c->lent.pop_back();
+        }
     if (!bytes || (db && bytes > kDbKeep)) {
         hipFree(p);
         return;
