@@ -3,9 +3,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <numeric>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -497,21 +499,42 @@ static int collect_host(hb_batch *b, uint32_t n)
     }
     b->tot[0] = b->tot[1] = b->tot[2] = 0;
     for (size_t i = 0; i < tot.size(); ++i) b->tot[i % 3] += tot[i];
-    std::sort(b->many.begin(), b->many.end(), [&](const hb_hsp &x, const hb_hsp &y) {
-        const int32_t qx = b->ctx_query[x.context], qy = b->ctx_query[y.context];
-        return std::tie(qx, x.oid, x.s_off, x.q_off) < std::tie(qy, y.oid, y.s_off, y.q_off);
-    });
+    // by query (counting), then each query's records, queries dealt to threads
+    // (1.5 million records of 48 queries: 115 ms with their copies on 8 CPUs, where
+    // one sort of them all took 280)
     const size_t nq = b->queries.size();
     b->q_first.assign(nq + 1, 0);
     b->q_count.assign(nq, 0);
-    for (hb_hsp &h : b->many) {
-        const int32_t q = b->ctx_query[h.context];
-        h.context = b->ctx_local[h.context];
-        h.q_start -= b->q_base[q];
-        h.q_off -= b->q_base[q];
-        b->q_count[q]++;
-    }
+    for (const hb_hsp &h : b->many) b->q_count[b->ctx_query[h.context]]++;
     for (size_t q = 0; q < nq; ++q) b->q_first[q + 1] = b->q_first[q] + b->q_count[q];
+    std::vector<hb_hsp> sorted(n);
+    std::vector<uint64_t> at(b->q_first.begin(), b->q_first.end() - 1);
+    for (const hb_hsp &h : b->many) {
+        const int32_t q = b->ctx_query[h.context];
+        hb_hsp &o = sorted[at[q]++];
+        o = h;
+        o.context = b->ctx_local[h.context];
+        o.q_start -= b->q_base[q];
+        o.q_off -= b->q_base[q];
+    }
+    b->many.swap(sorted);
+    std::atomic<size_t> next{0};
+    auto order = [&] {
+        for (size_t q; (q = next++) < nq;)
+            std::sort(b->many.begin() + (long)b->q_first[q], b->many.begin() + (long)b->q_first[q + 1],
+                      [](const hb_hsp &x, const hb_hsp &y) {
+                          return std::tie(x.oid, x.s_off, x.q_off) < std::tie(y.oid, y.s_off, y.q_off);
+                      });
+    };
+    const size_t nt = n < 65536 ? 1
+                                : std::min<size_t>({16, nq, std::thread::hardware_concurrency()});
+    std::vector<std::thread> th;
+    try {
+        for (size_t t = 1; t < nt; ++t) th.emplace_back(order);
+    } catch (...) {   // the threads that there are do all of it
+    }
+    order();
+    for (auto &t : th) t.join();
     b->results = b->many.data();
     return HB_OK;
 }

@@ -412,6 +412,65 @@ void database_after_context()
     CHECK(hb_pool_held(f.c) == g_fake.device_used);
 }
 
+// The order on the host: by query, subject and offsets, with the query's own
+// contexts and offsets.
+void host_order()
+{
+    Fixture f;
+    hb_db *db = f.database(20000);
+    constexpr uint32_t kQueries = 48;
+    for (uint32_t n : {0u, 1u, 1000u, 65535u, 65536u, 1500000u}) {
+        std::vector<uint32_t> perm(n);
+        for (uint32_t i = 0; i < n; ++i) perm[i] = (uint32_t)((i * 2654435761ull + 12345) % n);
+        std::vector<hb_hsp> all(n);   // each value of perm may stand more than once: s_off tells
+        for (uint32_t i = 0; i < n; ++i) {
+            memset(&all[i], 0, sizeof(hb_hsp));
+            all[i].oid = perm[i] / 64 % 20000;
+            all[i].s_off = (int32_t)(perm[i] % 64);
+            all[i].q_off = (int32_t)i;   // (a unique one; made relative below)
+        }
+        g_fake.scan = [&](const hb_scan_args &a) {
+            // five queries of 100 residues and 40 between them to a group of 768
+            for (uint32_t i = 0; i < n && i < a.out_cap; ++i) {
+                a.out[i] = all[i];
+                a.out[i].context = (int32_t)(i % kQueries);
+            }
+            *a.out_count = n;
+        };
+        hipStream_t st = nullptr;
+        CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+        hb_batch *b = f.batch(db, kQueries, st);
+        CHECK(hb_batch_reserve(b, n + 1) == HB_OK && hb_batch_launch(b) == HB_OK);
+        const int orders = g_fake.orders;
+        size_t room = 0;
+        CHECK(hb_batch_finish(b, &room) == HB_OK && room == 0 && g_fake.orders == orders);
+        uint64_t sum = 0;
+        for (uint32_t q = 0; q < kQueries; ++q) {
+            uint64_t k = 0;
+            std::vector<hb_hsp> got(n);
+            CHECK(hb_batch_results(b, (int32_t)q, got.data(), n, &k) == HB_OK);
+            sum += k;
+            int32_t base = 0;   // the query's place in its group, the same for all its records
+            for (uint64_t i = 0; i < k; ++i) {
+                const hb_hsp &x = got[i];
+                CHECK(x.context == 0);
+                if (i == 0) base = -x.q_start;
+                const uint32_t from = (uint32_t)(x.q_off + base);
+                CHECK(x.q_start == -base && from < n && all[from].oid == x.oid &&
+                      all[from].s_off == x.s_off && base % 140 == 0);
+                if (i == 0) continue;
+                const hb_hsp &y = got[i - 1];
+                CHECK(y.oid < x.oid ||
+                      (y.oid == x.oid &&
+                       (y.s_off < x.s_off || (y.s_off == x.s_off && y.q_off < x.q_off))));
+            }
+        }
+        CHECK(sum == n);
+        hb_batch_free(b);
+    }
+    hb_db_free(db);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -425,6 +484,7 @@ const struct {
     {"upload_sources", upload_sources},
     {"served_order", served_order},
     {"database_after_context", database_after_context},
+    {"host_order", host_order},
 };
 
 }  // namespace

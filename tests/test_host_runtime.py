@@ -81,3 +81,7 @@ def test_served_batches_order_within_the_budget(driver):
 
 def test_database_outlives_its_context(driver):
     run(driver, "database_after_context")
+
+
+def test_order_on_the_host(driver):
+    run(driver, "host_order")
