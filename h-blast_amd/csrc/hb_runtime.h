@@ -155,9 +155,9 @@ static inline int32_t hb_state_limit(int place, uint64_t max_len)
 // memory.
 int hb_state_choose(const hb_ctx *c, int32_t D, size_t fixed, uint64_t max_len, int32_t window);
 // The scan keeps a concatenated query, its context tables and the score
-// matrix in LDS (with the diagonal state in global memory at the least), and
-// the lookup-table build keeps the query in LDS too: queries past about
-// 150,000 concatenated residues do not fit a workgroup's 160 KB.
+// matrix in LDS, with the diagonal state in global memory at the least:
+// queries past about 150,000 concatenated residues do not fit a workgroup's
+// 160 KB.
 bool hb_query_lds_ok(const hb_ctx *c, int32_t qlen, int32_t n_ctx);
 // Global-memory diagonal state of one launch is capped at this size: a
 // launch for a very long query then runs fewer workgroups.

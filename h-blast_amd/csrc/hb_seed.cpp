@@ -724,7 +724,7 @@ bool hb_query_lds_ok(const hb_ctx *c, int32_t qlen, int32_t n_ctx)
 {
     const size_t qpad = (size_t)((qlen + 15) & ~15);
     const size_t fixed = hb_scan_fixed_lds((int32_t)qpad, hb_ctx_pad(n_ctx));
-    return fixed + hb_scan_wave_lds(0, 256, 0) <= c->max_lds && 1024 + qpad <= c->max_lds;
+    return fixed + hb_scan_wave_lds(0, 256, 0) <= c->max_lds;
 }
 
 size_t hb_gstate_bytes_max(const hb_ctx *c, int32_t D)
@@ -1314,8 +1314,7 @@ int hb_query_prepare_masked(hb_ctx *c, const uint8_t *seq, int32_t len, int32_t 
     // The diagonal state (4 bytes per diagonal) stays in LDS when it fits;
     // longer queries (the reference accepts 32,768 residues,
     // H-BLAST/h_blast.cu:1293) keep it in global memory.  The query itself,
-    // its context tables and the matrix are always in LDS, and so is the
-    // lookup-table build's copy of the query.
+    // its context tables and the matrix are always in LDS.
     const int32_t D = (len + q->p.window + 63) & ~63;
     if (!hb_query_lds_ok(c, len, n_ctx)) {
         delete q;

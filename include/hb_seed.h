@@ -669,7 +669,7 @@ int hb_gapped_search(hb_ctx *ctx, hb_db *db, const uint8_t *seq, int32_t len, in
  * separated by `window` code-0 residues so that hits of different queries
  * never pair (each query's HSPs equal its HSPs searched alone); each group
  * has its own lookup table in one device arena, and workgroups pop (group,
- * tile chunk) items from one queue.  The launch sequence is captured in a
+ * tile chunk) items from the queues of each group.  The launch sequence is captured in a
  * hipGraph on the first run and replayed on later runs.  H-BLAST's closest
  * counterpart is NCBI's concatenation of a query batch into one query
  * (contexts) searched by H_BLAST_pre/H_BLAST_get_data
@@ -688,7 +688,9 @@ typedef struct hb_batch_opts {
     int32_t ring_bytes;            /* staging ring per wavefront (multiple of 64, >= 256;
                                       default: the largest that keeps the occupancy) */
     int32_t items_per_workgroup;   /* (group, tile chunk) work items per workgroup, which
-                                      sets the subjects per item (default 64) */
+                                      sets the subjects per item.  Default: a pass over the
+                                      whole database takes tiles that shrink towards its end
+                                      one by one, the autotuner's slices take 64 items */
 } hb_batch_opts;
 
 typedef struct hb_batch_info {
@@ -703,7 +705,7 @@ typedef struct hb_batch_info {
     uint64_t hsps;
     int32_t waves_per_workgroup;   /* chosen launch geometry (of the largest class) */
     int32_t ring_bytes;
-    int32_t items_per_workgroup;
+    int32_t items_per_workgroup;   /* given or chosen by the autotuner, else 64 */
     int32_t tune_candidates;       /* autotune candidates timed (0: none) */
 } hb_batch_info;
 
