@@ -29,9 +29,11 @@
 // column state's decrement (all compares of a row are between cells of that
 // row), and the bias makes 0, which lane moves fill in, lower than any live cell.
 //
-// Bound by vector instruction issue: 118 of them per row of four sides (30 a
-// side; hb_gapped.hip spends 53 and as many scalar ones on a row of one side),
-// which fill 3/4 of the kernel's time.  The 73,052 HSPs of a 1,000-residue query
+// Bound by vector instruction issue: 120 of them per row of four sides, set-up
+// included (30 a side; hb_gapped.hip spends 53 and as many scalar ones on a row
+// of one side).  They fill 88% of the issue slots on the 297,173 HSPs of a
+// 1,000-residue query against 2,000,000 subjects and 3/4 of them against 500,000,
+// where the end of the work list weighs more.  The 73,052 HSPs of a 1,000-residue query
 // against 500,000 subjects take 920 us here and 1,507 us there, the 5,191 of 350
 // residues against 50,000 long-tailed subjects 186 and 340 us (950 and 195 us with
 // two tests a row for the letters at hand and the last row instead of one).  One set of 6

@@ -411,7 +411,7 @@ int hb_balance_next_ratio(const hb_runtime_options *o, const hb_balance_in *in, 
  * metadata, the scan's copy of the residues, the HSP reservation, the
  * per-subject counters and the result layout, and the diagonal state if q
  * keeps it in global memory for subjects up to max_len.  residues = 0 takes
- * file_bytes as its bound.  budget < 0 takes the device's free memory.
+ * file_bytes as its bound.  budget < 0 takes the free memory of hb_mem_info.
  * *fits = 1 if *need <= the budget.  (The lookup table of q is already on
  * the device.) */
 int hb_check_memory(hb_ctx *ctx, const hb_query *q, uint64_t file_bytes, uint64_t residues,
@@ -744,7 +744,8 @@ typedef struct hb_serve_opts {
     int32_t max_batch_queries;   /* queries per batch (default 64) */
     int32_t max_inflight;        /* batches on the device at once (default 2) */
     int64_t max_batch_residues;  /* query residues per batch (default 16384) */
-    int64_t mem_budget;          /* device bytes for admitted batches; 0 = half the free memory */
+    int64_t mem_budget;          /* device bytes for admitted batches; 0 = half the free memory
+                                    (of hb_mem_info) */
     int32_t group_residues;      /* group size of the batched scans (default 768) */
     int32_t max_pending;         /* queued requests beyond which submit is refused (default 65536) */
     double hsp_per_cell;         /* expected HSPs per (query residue x subject residue), for
