@@ -58,6 +58,7 @@ constexpr uint32_t kPastLetter = 31;
 constexpr int32_t kPad = 160;               // such letters kept on either side of a subject
 static_assert(kPad >= 2 * kCols + 2 * kC + 8 && kC == 4, "letters of a window, a word a lane");
 static_assert(HB_GAP_PAIR_HSPS <= 256, "order");
+static_assert(kSaved <= HB_GAP_SAVED, "a subject that is left with them goes on in hb_gapped.hip");
 
 // Lane move within 16 lanes; lanes without a source get 0, or old.
 template <int CTRL>
@@ -210,7 +211,13 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                 const int32_t ra = half_get(abest, 16), rb = half_get(bbest, 16);
                 const bool right = half_get((int32_t)(M > 0 && N > 0), 16) != 0;
                 if (ovf || (score >= cut && n_saved >= kSaved)) {
-                    if (hl == 0) A.mid[1 + atomicAdd(A.mid, 1u)] = k;
+                    if (hl == 0) {   // hb_gapped.hip goes on with this HSP
+                        A.st3[3 * (size_t)k] = r;
+                        A.st3[3 * (size_t)k + 1] = ext - 1;
+                        A.st3[3 * (size_t)k + 2] = n_saved;
+                        A.mid[1 + atomicAdd(A.mid, 1u)] = k;
+                    }
+                    sync_lanes();   // (before the next pop of this half's first lane)
                     fresh = true;
                 } else if (score >= cut) {
                     const int32_t q0 = ql - la, s0 = so + 1 - lb;
@@ -263,6 +270,7 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                     const uint64_t o1 = A.offs[k + 1];
                     if (n > HB_GAP_PAIR_HSPS || o1 - o0 >= (uint64_t)kLongSubject) {
                         if (hl == 0) A.mid[1 + atomicAdd(A.mid, 1u)] = k;
+                        sync_lanes();
                         continue;
                     }
                     slen = (int32_t)(o1 - o0);
@@ -310,6 +318,7 @@ __global__ __launch_bounds__(kWaves * HB_WAVE) __attribute__((amdgpu_waves_per_e
                         A.st3[3 * (size_t)k + 1] = ext;
                         A.st3[3 * (size_t)k + 2] = n_saved;
                     }
+                    sync_lanes();
                     fresh = true;
                     continue;
                 }

@@ -270,7 +270,8 @@ struct hb_gap_args {
     const uint32_t *list;          // subjects with HSPs, most HSPs first
     const uint32_t *n_list;        // their number (device)
     hb_gapped_hsp *out;            // subject k's gapped HSPs at ust[k].first + i
-    uint32_t *st3;                 // per subject {0, extensions, saved}
+    uint32_t *st3;                 // per subject {0, extensions, saved}; of one left to the next
+                                   // pass {HSPs done, extensions and saved of those}
     uint32_t *wide;                // [0] count, then subjects for the wide pass
     // wide pass: subjects wide[1 .. n_wide], one per wavefront-iteration,
     // each wavefront with its own global scratch of scratch_words int32:
