@@ -953,7 +953,9 @@ static constexpr uint64_t kTileMax = 16384, kQueueTileMin = 256;
 // The database's lengths, longest first, as runs of equal ones.
 static std::vector<std::pair<uint64_t, uint32_t>> length_runs(const hb_db *db)
 {
-    constexpr uint64_t kCounted = 1 << 16;   // longer subjects are few: sorted
+    // (as many counters as there are lengths, so that a few short subjects do
+    // not cost 65,536 of them; subjects past those are few: sorted)
+    const uint64_t kCounted = std::min<uint64_t>(1 << 16, db->max_len + 1);
     std::vector<uint32_t> cnt(kCounted, 0);
     std::vector<uint64_t> longer;
     for (uint32_t i = 0; i < db->n; ++i) {
@@ -1006,7 +1008,7 @@ static uint32_t cut_tiles(const std::vector<std::pair<uint64_t, uint32_t>> &runs
     return (uint32_t)(tiles->size() - t0) - 1;
 }
 
-// Tiles of a database whose host offsets are set, and the device copies of
+// Tiles of a database whose host offsets and longest subject are set, and the device copies of
 // offsets and tiles; then, enqueued on the context's stream, the records in
 // processing order (length-descending: the longest subjects start first).
 // The scan reads each subject's oid, length and offset from one 16-byte
@@ -1019,7 +1021,6 @@ static int db_meta(hb_db *db)
     hb_ctx *c = db->ctx;
     const uint32_t n = db->n;
     const auto runs = length_runs(db);
-    db->max_len = runs.empty() ? 0 : runs.front().first;
     db->scan_bytes = 0;   // the scan stages subjects with 16-byte loads
     for (const auto &r : runs) db->scan_bytes += ((r.first + 15) & ~15ull) * r.second;
     const uint64_t waves = c->n_cu * 16ull;
@@ -1087,9 +1088,12 @@ int hb_db_upload(hb_ctx *c, const uint8_t *residues, const uint64_t *offsets, ui
     *out = nullptr;
     // subject lengths are int32 on the device and diagonal state keeps
     // position + offset below 2^31: cap a subject at 2^28 residues
-    for (uint32_t i = 0; i < n; ++i)
-        if (offsets[i + 1] < offsets[i] || offsets[i + 1] - offsets[i] > (1ull << 28))
-            return HB_ERR_ARG;
+    uint64_t longest = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const uint64_t len = offsets[i + 1] - offsets[i];
+        if (offsets[i + 1] < offsets[i] || len > (1ull << 28)) return HB_ERR_ARG;
+        longest = std::max(longest, len);
+    }
     std::lock_guard<std::mutex> lk(c->mu);
     HB_CHECK(hipSetDevice(c->device));
     hb_db *db = new (std::nothrow) hb_db;
@@ -1097,6 +1101,7 @@ int hb_db_upload(hb_ctx *c, const uint8_t *residues, const uint64_t *offsets, ui
     db->ctx = c;
     db->device = c->device;
     db->n = n;
+    db->max_len = longest;
     const uint64_t first = n ? offsets[0] : 0;
     db->total = n ? offsets[n] - first : 0;
     db->h_offs.resize((size_t)n + 1);
@@ -1203,7 +1208,10 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
         return fail(HB_ERR_DEVICE);
     db->h_offs.resize((size_t)n_seqs + 1);
     db->h_offs[0] = 0;
-    for (int32_t i = 0; i < n_seqs; ++i) db->h_offs[i + 1] = db->h_offs[i] + lens[i];
+    for (int32_t i = 0; i < n_seqs; ++i) {
+        db->h_offs[i + 1] = db->h_offs[i] + lens[i];
+        db->max_len = std::max<uint64_t>(db->max_len, lens[i]);
+    }
     db->total = db->h_offs[n_seqs];
     if (!db_get(c, &db->d_res, db->total + 64)) return fail(HB_ERR_NOMEM);
     int rc = db_meta(db);
