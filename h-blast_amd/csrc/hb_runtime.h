@@ -82,7 +82,8 @@ struct hb_db {
     uint32_t *d_tiles = nullptr;   // n_tiles + 1 boundaries (batched scans), then the
     uint32_t n_tiles = 0;          // n_qtiles + 1 of the plain scan's queue tiles
     uint32_t n_qtiles = 0;
-    void *load_scratch = nullptr;  // while it is loaded
+    void *load_scratch = nullptr, *load_pin = nullptr;   // while it is loaded
+    size_t load_pin_bytes = 0;
     std::vector<uint64_t> h_offs;
     uint64_t max_len = 0;   // longest subject
     float hdb_len_ms = 0.f, hdb_copy_ms = 0.f;   // hb_db_upload_hdb's kernels

@@ -196,9 +196,12 @@ void hb_pin_put(hb_ctx *c, void *p, size_t bytes)
 // (the copies then go through the DMA engine at 50 GB/s while the context's
 // stream makes the records).  Whole loads of 36, 108 and 216 MB: 2.16, 6.20 and
 // 12.8 ms before, 1.12, 2.86 and 5.47 ms now; chunks of 2 MB 7% slower, of 1 MB
-// 20%; four threads the same as two.  Memory that the runtime knows (page-locked,
-// managed, a device's) travels from where it is; below kMin the threads' start costs what they save (3.6 MB:
-// 366 us without, 352 us with the rest of it).
+// 20%; four threads the same as two.  Below kMin, where the threads' start costs
+// what they save, the caller's thread fills one buffer (the runtime page-locks
+// small memory for its copy, 50 to 190 us for 360 KB: the load 310 us with that,
+// 180 without).  Memory that the runtime knows (page-locked, managed, a device's)
+// travels from where it is, on that stream too (36 MB and the rest of the load
+// 820 us, 1,180 with a copy on the null stream behind the records).
 namespace {
 class Upload {
   public:
@@ -209,37 +212,18 @@ class Upload {
         dst_ = static_cast<char *>(dst);
         src_ = static_cast<const char *>(src);
         bytes_ = bytes;
-        if (bytes < kMin) return;
-        hipPointerAttribute_t at{};
-        if (hipPointerGetAttributes(&at, src) != hipSuccess) (void)hipGetLastError();
-        else if (at.type != hipMemoryTypeUnregistered) return;
-        if (!c->up_stream &&
-            hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) != hipSuccess) {
-            (void)hipGetLastError();
-            c->up_stream = nullptr;
-            return;
-        }
-        pin_bytes_ = kThreads * kSlots * kChunk;
-        pin_ = static_cast<char *>(hb_pin_get(c, &pin_bytes_));
-        if (!pin_) return;
-        try {
-            th_.reserve(kThreads);
-            for (size_t t = 0; t < kThreads; ++t) th_.emplace_back([this, t] { work(t); });
-        } catch (...) {   // the threads that there are do all of it
-        }
+        if (bytes && !start_own()) e_ = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
     }
     int finish()
     {
         if (!c_) return HB_OK;
-        hipError_t e = hipSuccess;
-        if (th_.empty()) {
-            if (bytes_) e = hipMemcpy(dst_, src_, bytes_, hipMemcpyHostToDevice);
-        } else {
-            for (auto &t : th_) t.join();
+        hipError_t e = e_;
+        for (auto &t : th_) t.join();
+        th_.clear();
+        if (own_) {
             e = hipStreamSynchronize(c_->up_stream);
             if (failed_) e = hipErrorUnknown;
         }
-        th_.clear();
         hb_pin_put(c_, pin_, pin_bytes_);
         pin_ = nullptr;
         c_ = nullptr;
@@ -251,6 +235,42 @@ class Upload {
   private:
     static constexpr size_t kThreads = 2, kSlots = 2, kChunk = (size_t)4 << 20;
     static constexpr size_t kMin = (size_t)4 << 20;
+    // Starts the copy on the stream of its own; false if there is nothing to start
+    // that for, or no way to.
+    bool start_own()
+    {
+        hipPointerAttribute_t at{};
+        bool known = false;
+        if (hipPointerGetAttributes(&at, src_) != hipSuccess) (void)hipGetLastError();
+        else known = at.type != hipMemoryTypeUnregistered;
+        if (!c_->up_stream &&
+            hipStreamCreateWithFlags(&c_->up_stream, hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
+            c_->up_stream = nullptr;
+            return false;
+        }
+        auto send = [&](const void *from) {
+            own_ = hipMemcpyAsync(dst_, from, bytes_, hipMemcpyHostToDevice, c_->up_stream) ==
+                   hipSuccess;
+            if (!own_) (void)hipGetLastError();
+            return own_;
+        };
+        if (known) return send(src_);
+        pin_bytes_ = bytes_ < kMin ? bytes_ : kThreads * kSlots * kChunk;
+        pin_ = static_cast<char *>(hb_pin_get(c_, &pin_bytes_));
+        if (!pin_) return false;
+        if (bytes_ < kMin) {
+            memcpy(pin_, src_, bytes_);
+            return send(pin_);
+        }
+        try {
+            th_.reserve(kThreads);
+            for (size_t t = 0; t < kThreads; ++t) th_.emplace_back([this, t] { work(t); });
+        } catch (...) {   // the threads that there are do all of it
+        }
+        own_ = !th_.empty();
+        return own_;
+    }
     // Start of chunk i: two of each size from an eighth of kChunk up, so that
     // the link need not wait for a full chunk to be filled.
     static size_t chunk_at(size_t i)
@@ -287,6 +307,8 @@ class Upload {
     std::vector<std::thread> th_;
     std::atomic<size_t> next_{0};
     std::atomic<bool> failed_{false};
+    bool own_ = false;            // the copy is on the stream of its own
+    hipError_t e_ = hipSuccess;   // ... else it is done, with this
 };
 }  // namespace
 
@@ -929,6 +951,8 @@ int hb_db_free(hb_db *db)
                         (void *)db->d_scan_alloc, (void *)db->d_tiles})
             if (kept) db_put(db->ctx, p);
             else hipFree(p);
+        if (kept) hb_pin_put(db->ctx, db->load_pin, db->load_pin_bytes);
+        else hipHostFree(db->load_pin);
     }
     delete db;
     return HB_OK;
@@ -1039,11 +1063,27 @@ static int db_meta(hb_db *db)
     a.n = n;
     a.max_len = db->max_len;
     a.subj = db->d_subj;
-    if (hipMemcpy(db->d_offs, db->h_offs.data(), ((size_t)n + 1) * sizeof(uint64_t),
-                  hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(db->d_tiles, tiles.data(), tiles.size() * sizeof(uint32_t),
-                  hipMemcpyHostToDevice) != hipSuccess ||
-        hb_launch_load_records(a, db->load_scratch, c->stream) != hipSuccess)
+    // Small ones go through a page-locked buffer and are not waited for (each copy
+    // of pageable memory is, 15 us).
+    constexpr size_t kStage = (size_t)1 << 20;
+    const size_t b_offs = ((size_t)n + 1) * sizeof(uint64_t);
+    const size_t b_tiles = tiles.size() * sizeof(uint32_t);
+    db->load_pin_bytes = b_offs + b_tiles;
+    if (b_offs + b_tiles <= kStage) db->load_pin = hb_pin_get(c, &db->load_pin_bytes);
+    bool ok;
+    if (char *pin = static_cast<char *>(db->load_pin)) {
+        memcpy(pin, db->h_offs.data(), b_offs);
+        memcpy(pin + b_offs, tiles.data(), b_tiles);
+        ok = hipMemcpyAsync(db->d_offs, pin, b_offs, hipMemcpyHostToDevice, c->stream) ==
+                 hipSuccess &&
+             hipMemcpyAsync(db->d_tiles, pin + b_offs, b_tiles, hipMemcpyHostToDevice,
+                            c->stream) == hipSuccess;
+    } else {
+        ok = hipMemcpy(db->d_offs, db->h_offs.data(), b_offs, hipMemcpyHostToDevice) ==
+                 hipSuccess &&
+             hipMemcpy(db->d_tiles, tiles.data(), b_tiles, hipMemcpyHostToDevice) == hipSuccess;
+    }
+    if (!ok || hb_launch_load_records(a, db->load_scratch, c->stream) != hipSuccess)
         return HB_ERR_DEVICE;
     return HB_OK;
 }
@@ -1078,6 +1118,8 @@ static int db_scan_copy(hb_db *db)
         return HB_ERR_DEVICE;
     db_put(c, db->load_scratch);
     db->load_scratch = nullptr;
+    hb_pin_put(c, db->load_pin, db->load_pin_bytes);
+    db->load_pin = nullptr;
     return flag ? HB_ERR_RESIDUE : HB_OK;
 }
 

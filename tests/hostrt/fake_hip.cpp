@@ -176,8 +176,12 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k)
     memcpy(d, s, n);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st)
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
 {
+    if (k == hipMemcpyHostToDevice && n > g_fake.async_bytes) {
+        g_fake.async_bytes = n;
+        g_fake.async_from = s;
+    }
     memcpy(d, s, n);
     enqueue(st);
     return hipSuccess;

@@ -30,6 +30,8 @@ struct FakeHip {
     std::atomic<int> fail_finalize{0};        // ... hb_launch_finalize(_compact) after their work
     std::atomic<int> orders{0};               // hb_launch_order calls
     std::atomic<int> host_to_device{0};       // synchronous host-to-device copies
+    std::atomic<const void *> async_from{nullptr};   // source of the largest asynchronous one
+    std::atomic<size_t> async_bytes{0};
     // the HSPs that a scan of one group finds (called by hb_launch_scan)
     std::function<void(const hb_scan_args &)> scan;
 };
