@@ -168,13 +168,17 @@ static void make_groups(hb_batch *b, int32_t target, std::vector<hb_concat> *gro
 
 static int32_t items_per_workgroup(const hb_batch *b) { return b->g_items > 0 ? b->g_items : 64; }
 
-// Sizes work items for a pass over n_tiles tiles: about 64 items per
-// workgroup for balance, few enough for the queue atomic.
+// Sizes work items for a pass over n_tiles tiles: about 64 items for every
+// wavefront of a workgroup for balance, few enough for the queue atomic.  (The
+// wavefronts pop their own items; with as many for the whole workgroup, from
+// when they shared them, 16 items took 48 queries against 100,000 subjects
+// 19.7 ms, 15.7 so.)
 static void size_items(hb_batch *b, uint32_t n_tiles)
 {
     for (Class &c : b->classes) {
         const uint32_t n_groups = (uint32_t)(c.g_end - c.g_begin);
-        const uint64_t want = (uint64_t)c.cfg.blocks * (uint64_t)items_per_workgroup(b);
+        const uint64_t want =
+            (uint64_t)c.cfg.blocks * (uint64_t)(c.cfg.waves * items_per_workgroup(b));
         const uint64_t per_group = std::max<uint64_t>(1, want / std::max<uint32_t>(n_groups, 1));
         c.tiles_per_item = (uint32_t)std::max<uint64_t>(1, (n_tiles + per_group - 1) / per_group);
     }

@@ -687,10 +687,11 @@ typedef struct hb_batch_opts {
     int32_t waves_per_workgroup;   /* 4, 2 or 1 (default: the most wavefronts per CU) */
     int32_t ring_bytes;            /* staging ring per wavefront (multiple of 64, >= 256;
                                       default: the largest that keeps the occupancy) */
-    int32_t items_per_workgroup;   /* (group, tile chunk) work items per workgroup, which
-                                      sets the subjects per item.  Default: a pass over the
-                                      whole database takes tiles that shrink towards its end
-                                      one by one, the autotuner's slices take 64 items */
+    int32_t items_per_workgroup;   /* (group, tile chunk) work items for each wavefront of a
+                                      workgroup, which sets the subjects per item.  Default: a
+                                      pass over the whole database takes tiles that shrink
+                                      towards its end one by one, the autotuner's slices take
+                                      64 items */
 } hb_batch_opts;
 
 typedef struct hb_batch_info {
