@@ -312,13 +312,16 @@ class Upload {
 };
 }  // namespace
 
-// Copies between host buffers, 1 MiB or more a thread: a search with 4.8 MB of
-// counters and a gapped stage with 8 MB took 1,159 and 1,520 us with one thread,
-// 1,090 and 1,468 with two, 1,089 and 1,437 with four, and the same with eight.
+// Copies between host buffers, on up to four threads of 1 MiB or more, and up to
+// eight of 4 MiB: a search with 4.8 MB of counters and a gapped stage with 8 MB
+// took 1,159 and 1,520 us with one thread, 1,090 and 1,468 with two, 1,089 and
+// 1,437 with four, and the same with eight; 48 MB of counters into new arrays took
+// 2.17 ms with four and 1.85 with eight.
 static void host_copy(void *dst, const void *src, size_t bytes)
 {
     constexpr size_t kPart = (size_t)1 << 20;
-    const size_t nt = std::min<size_t>(4, std::max<size_t>(1, bytes / kPart));
+    const size_t few = std::min<size_t>(4, std::max<size_t>(1, bytes / kPart));
+    const size_t nt = std::min<size_t>(8, std::max<size_t>(few, bytes / (4 * kPart)));
     const size_t per = (bytes + nt - 1) / nt;
     auto part = [&](size_t t) {
         const size_t b = t * per, e = std::min(bytes, b + per);
