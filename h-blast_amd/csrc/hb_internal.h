@@ -79,6 +79,7 @@ struct hb_scan_args {
     int32_t ctx_pad_max;         // multiple of 4
     int32_t diag_len_max;
     int32_t split;               // some group has shift > 0
+    int32_t many;                // plain, not split: the kernel of 20 wavefronts per CU
     uint32_t wave_lds;           // LDS bytes per wave
     uint32_t ring;               // staging ring bytes per wave (multiple of 16): subjects up
                                  // to this length are staged in LDS
@@ -155,6 +156,8 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
 // launching or capturing a launch with that LDS size).
 // Raises both scan kernels' dynamic LDS limit to max_lds (once per context).
 hipError_t hb_scan_allow_lds(size_t max_lds);
+// Workgroups of that kernel per CU.
+hipError_t hb_scan_short_occupancy(size_t lds_bytes, int *blocks_per_cu);
 hipError_t hb_scan_occupancy(bool multi, bool gstate, bool split, size_t lds_bytes,
                              int block_threads, int *blocks_per_cu);
 hipError_t hb_launch_copy(void *dst, const void *src, uint64_t bytes, hipStream_t st);

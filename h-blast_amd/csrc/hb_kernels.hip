@@ -1212,7 +1212,8 @@ __device__ __forceinline__ void scan_tile(WaveScan<GS, SPLIT> &w, const hb_scan_
 // Every scan kernel keeps a register budget for four wavefronts per SIMD
 // (128 VGPRs), the most a 1000-residue query's LDS leaves room for: at five
 // (96 VGPRs) the many-group kernel spills to scratch, and 20 wavefronts per
-// CU measured slower than 16 where the LDS would allow them.
+// CU measured slower than 16 where the LDS would allow them, up to 152 residues
+// (hb_scan_kernel_short) excepted.
 template <bool MULTI, bool GSTATE, bool SPLIT>
 __device__ __forceinline__ void scan_body(const hb_scan_args &a);
 
@@ -1220,6 +1221,14 @@ template <bool MULTI, bool SPLIT>
 __global__ __launch_bounds__(SPLIT && !MULTI ? HB_BLOCK_SPLIT : HB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void hb_scan_kernel(hb_scan_args a)
 {
     scan_body<MULTI, false, SPLIT>(a);
+}
+// Short queries' LDS lets five workgroups into a CU: 20 wavefronts in 96 VGPRs
+// (11 values that the loops do not change go to scratch) took 60 residues against
+// 2,000,000 subjects 3.39 ms where 16 in 109 take 3.85, 152 against 1,000,000 2.01
+// and 2.28.
+__global__ __launch_bounds__(HB_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void hb_scan_kernel_short(hb_scan_args a)
+{
+    scan_body<false, false, false>(a);
 }
 template <bool MULTI>
 __global__ __launch_bounds__(HB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void hb_scan_kernel_g(hb_scan_args a)
@@ -1798,6 +1807,7 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
                           size_t lds_bytes, hipStream_t st)
 {
     const bool g = a.gstate != nullptr, split = a.split != 0;
+    if (a.many && (multi || g || split)) return hipErrorInvalidValue;
     const int top = hb_block_max(multi, split, g);
     if (block_threads < HB_WAVE || block_threads > top || block_threads % HB_WAVE)
         return hipErrorInvalidValue;
@@ -1806,6 +1816,8 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
     if (g) {
         if (multi) hipLaunchKernelGGL(hb_scan_kernel_g<true>, grid, block, lds_bytes, st, a);
         else hipLaunchKernelGGL(hb_scan_kernel_g<false>, grid, block, lds_bytes, st, a);
+    } else if (a.many) {
+        hipLaunchKernelGGL(hb_scan_kernel_short, grid, block, lds_bytes, st, a);
     } else if (split) {
         if (multi) hipLaunchKernelGGL((hb_scan_kernel<true, true>), grid, block, lds_bytes, st, a);
         else hipLaunchKernelGGL((hb_scan_kernel<false, true>), grid, block, lds_bytes, st, a);
@@ -1818,8 +1830,9 @@ hipError_t hb_launch_scan(const hb_scan_args &a, bool multi, int n_blocks, int b
 
 hipError_t hb_scan_allow_lds(size_t max_lds)
 {
-    for (int k = 0; k < 6; ++k) {
-        const void *fn = scan_fn((k & 1) != 0, k >= 4, (k & 2) != 0);
+    for (int k = 0; k < 7; ++k) {
+        const void *fn = k == 6 ? reinterpret_cast<const void *>(hb_scan_kernel_short)
+                                : scan_fn((k & 1) != 0, k >= 4, (k & 2) != 0);
         hipFuncAttributes fa;
         hipError_t e = hipFuncGetAttributes(&fa, fn);
         if (e != hipSuccess) return e;
@@ -1829,6 +1842,12 @@ hipError_t hb_scan_allow_lds(size_t max_lds)
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+hipError_t hb_scan_short_occupancy(size_t lds_bytes, int *blocks_per_cu)
+{
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        blocks_per_cu, reinterpret_cast<const void *>(hb_scan_kernel_short), HB_BLOCK, lds_bytes);
 }
 
 hipError_t hb_scan_occupancy(bool multi, bool gstate, bool split, size_t lds_bytes,

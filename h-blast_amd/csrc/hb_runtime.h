@@ -33,6 +33,7 @@ struct hb_ctx {
     hipStream_t stream = nullptr;
     int n_cu = 0;
     size_t max_lds = 0;
+    bool short_scan = false;   // five workgroups of the short queries' scan fit a CU
     std::mutex mu;
     // Device buffers of finished scans, reused by later scans so that a
     // per-query loop does not pay hipMalloc/hipFree per call.
@@ -134,6 +135,7 @@ struct hb_launch_cfg {
     size_t lds = 0;
     int blocks = 0;
     int32_t ring = 1024;   // staging ring bytes per wave
+    bool many = false;     // hb_scan_args::many
 };
 // Where a launch keeps its per-diagonal two-hit state: 32-bit words in LDS,
 // or 32-bit words in a global-memory region per wavefront (markers in LDS).

@@ -758,6 +758,10 @@ size_t hb_gstate_bytes_max(const hb_ctx *c, int32_t D)
     return std::min(full, std::max(HB_GSTATE_MAX_BYTES, 4 * HB_GSTATE_WORD * (size_t)D));
 }
 
+// Dynamic LDS of a workgroup of which five fit a CU: 25 steps of 1,280 bytes,
+// less the kernel's own variables.
+static constexpr size_t kShortLds = 25 * 1280 - 16;
+
 struct hb_query {
     hb_ctx *ctx = nullptr;
     hb_resolved_params p;
@@ -868,12 +872,15 @@ int hb_create(int device, hb_ctx **out)
     // one dynamic-LDS limit for every launch of the scan kernels, so that
     // launches of different sizes on different streams never disagree; the
     // no-alloc scan's scratch address of this device
+    int five = 0;
     if (hb_scan_allow_lds(c->max_lds) != hipSuccess ||
+        hb_scan_short_occupancy(kShortLds, &five) != hipSuccess ||
         scratch_address(device, &c->scratch_dev) != HB_OK) {
         hipStreamDestroy(c->stream);
         delete c;
         return HB_ERR_DEVICE;
     }
+    c->short_scan = five >= 5;
     std::lock_guard<std::mutex> lk(g_ctx_mu);
     g_ctxs.push_back(c);
     *out = c;
@@ -1487,6 +1494,7 @@ static int plain_scan_args(const hb_db *db, const hb_query *q, int place,
     a->ctx_pad_max = q->gs.ctx_pad_max;
     a->diag_len_max = q->gs.diag_len_max;
     a->split = q->gs.split;
+    a->many = cfg.many;
     a->wave_lds = (uint32_t)hb_scan_wave_lds(q->gs.diag_len_max, cfg.ring, hb_state_bytes(place));
     a->ring = (uint32_t)cfg.ring;
     a->state_limit = hb_state_limit(place, db->max_len);
@@ -1501,6 +1509,30 @@ static int plain_scan_args(const hb_db *db, const hb_query *q, int place,
     return HB_OK;
 }
 
+// Configuration of a plain scan.  A query of up to 152 residues leaves five
+// workgroups the LDS they need with the largest ring (their share of 160 KB in
+// steps of 1,280 bytes; the runtime's count knows no steps, and at 160 residues
+// the fifth would start when the others are done): 20 wavefronts per CU, where
+// each of them gets kShortShare residues (us with 16 and with 20: 60 residues
+// against 20,000 subjects 83 and 87, 50,000 127 and 120, 200,000 414 and 370).
+// (Not in a scan that must allocate nothing: that kernel has scratch.)
+static constexpr uint64_t kShortShare = 4096;
+static int plain_config(const hb_db *db, const hb_query *q, int place, bool noalloc,
+                        hb_launch_cfg *cfg)
+{
+    hb_ctx *c = db->ctx;
+    const uint32_t items = db->n_qtiles << q->gs.desc[0].shift;
+    int rc = hb_scan_config(c, false, q->gs.split != 0, q->gs.qlen_pad_max, q->gs.ctx_pad_max,
+                            q->gs.diag_len_max, items, cfg, place);
+    if (rc) return rc;
+    cfg->many = !noalloc && c->short_scan && place == HB_PLACE_LDS && !q->gs.split &&
+                cfg->waves * HB_WAVE == HB_BLOCK && cfg->ring == HB_RING_MAX &&
+                cfg->lds <= kShortLds && db->total >= c->n_cu * 16ull * kShortShare;
+    if (cfg->many)
+        cfg->blocks = (int)std::min<uint64_t>(5ull * c->n_cu, (items + cfg->waves - 1) / cfg->waves);
+    return HB_OK;
+}
+
 static int launch_scan(hb_scan *s)
 {
     hb_ctx *c = s->ctx;
@@ -1510,8 +1542,7 @@ static int launch_scan(hb_scan *s)
     const int place = state_place(q, db);
     if (place < 0) return HB_ERR_UNSUPPORTED;   // LDS state asked for, subjects too long
     s->place = place;
-    int rc = hb_scan_config(c, false, q->gs.split != 0, q->gs.qlen_pad_max, q->gs.ctx_pad_max,
-                            q->gs.diag_len_max, db->n_qtiles << q->gs.desc[0].shift, &cfg, place);
+    int rc = plain_config(db, q, place, false, &cfg);
     if (rc) return rc;
     if (place == HB_PLACE_GLOBAL && !s->d_gstate) {
         s->d_gstate = static_cast<uint32_t *>(hb_pool_get(
@@ -1702,8 +1733,7 @@ int hb_scan_noalloc(hb_ctx *c, hb_db *db, hb_query *q, hb_hsp *d_hsps, uint32_t 
     const int place = state_place(q, db);
     if (place < 0) return HB_ERR_UNSUPPORTED;
     hb_launch_cfg cfg;
-    int rc = hb_scan_config(c, false, q->gs.split != 0, q->gs.qlen_pad_max, q->gs.ctx_pad_max,
-                            q->gs.diag_len_max, db->n_qtiles << q->gs.desc[0].shift, &cfg, place);
+    int rc = plain_config(db, q, place, true, &cfg);
     if (rc) return rc;
     hb_scan_args a;
     rc = plain_scan_args(db, q, place, cfg, &a);

@@ -261,6 +261,11 @@ hipError_t hb_scan_occupancy(bool, bool, bool, size_t lds, int, int *per_cu)
     *per_cu = (int)((160 << 10) / lds);
     return hipSuccess;
 }
+hipError_t hb_scan_short_occupancy(size_t, int *per_cu)
+{
+    *per_cu = 5;
+    return hipSuccess;
+}
 hipError_t hb_launch_copy(void *d, const void *s, uint64_t n, hipStream_t st)
 {
     memcpy(d, s, n);
