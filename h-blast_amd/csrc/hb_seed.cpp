@@ -992,8 +992,9 @@ static std::vector<std::pair<uint64_t, uint32_t>> length_runs(const hb_db *db)
     const uint64_t kCounted = std::min<uint64_t>(1 << 16, db->max_len + 1);
     std::vector<uint32_t> cnt(kCounted, 0);
     std::vector<uint64_t> longer;
+    const uint64_t *offs = db->h_offs.data();
     for (uint32_t i = 0; i < db->n; ++i) {
-        const uint64_t len = db->h_offs[i + 1] - db->h_offs[i];
+        const uint64_t len = offs[i + 1] - offs[i];
         if (len < kCounted) ++cnt[len];
         else longer.push_back(len);
     }
@@ -1259,12 +1260,18 @@ int hb_db_upload_hdb(hb_ctx *c, const uint8_t *hdb, uint64_t bytes, int32_t bloc
         hipStreamSynchronize(c->stream) != hipSuccess)
         return fail(HB_ERR_DEVICE);
     db->h_offs.resize((size_t)n_seqs + 1);
-    db->h_offs[0] = 0;
+    // (sum and longest in locals: through the object each sequence's wait for the
+    // stores of the one before)
+    uint64_t at = 0;
+    uint32_t longest = 0;
     for (int32_t i = 0; i < n_seqs; ++i) {
-        db->h_offs[i + 1] = db->h_offs[i] + lens[i];
-        db->max_len = std::max<uint64_t>(db->max_len, lens[i]);
+        db->h_offs[i] = at;
+        at += lens[i];
+        longest = std::max(longest, lens[i]);
     }
-    db->total = db->h_offs[n_seqs];
+    db->h_offs[n_seqs] = at;
+    db->max_len = longest;
+    db->total = at;
     if (!db_get(c, &db->d_res, db->total + 64)) return fail(HB_ERR_NOMEM);
     int rc = db_meta(db);
     if (rc != HB_OK) return fail(rc);
